@@ -49,6 +49,26 @@ struct KbPoly {
   float dc[kPolyCoefs][kMaxTaps];
 };
 
+// The polynomials as the matrix-core kernels read them: the plain values, and
+// copies times the powers of two the operands enter the FP16 split with.
+struct WinPoly {
+  KbPoly p;
+  float fac[kPolyCoefs][kMaxTaps];  // c * kFacScale
+  float op[kPolyCoefs][kMaxTaps];   // c * kOpScale
+  float dop[kPolyCoefs][kMaxTaps];  // dc * kOpScaleD
+};
+// Operands enter the FP16 split multiplied by 2^12 (exact), so that the low
+// halves of operands down to 2^-14 of the largest stay FP16-normal (11
+// significant bits): values in [0, 1] become [0, 4096] (FP16 max 65504).
+// Products carry 2^24, removed with the output scale.  Kernel derivatives
+// (|phi'| < 64 for w <= 8) use 2^8.  The x and y weights of spreading enter
+// their split multiplied by 2^6 each, so that their product carries 2^12.
+constexpr float kOpScale = 4096.0f;
+constexpr float kOpScaleD = 256.0f;
+constexpr float kFacScale = 64.0f;
+constexpr float kProdUnscale = 1.0f / (4096.0f * 4096.0f);
+constexpr float kProdUnscaleD = 1.0f / (4096.0f * 256.0f);
+
 // Geometry of the oversampled grid and the spreading tiles.
 struct Geom {
   int m[3];          // oversampled sizes (1D: m[1] = m[2] = 1)
@@ -73,6 +93,23 @@ __host__ __device__ __forceinline__ int cell_div(int cell, const Geom &g, int a)
 constexpr uint32_t kWorkUnit = 16;
 constexpr uint32_t kSubWork = 48;
 
+// Window classes of the matrix-core kernels.  A tile's points are listed by
+// the class of their y offset: class k holds `cw` consecutive offsets, so all
+// taps of its points lie in the 16 rows that start at the class's first
+// offset.  `ncls` classes per tile.
+constexpr int kMaxCls = 16;
+constexpr int kClassSub = 4096;  // points of a tile listed by class at once
+
+// The class list of a binning (sort.hip, class_sort_kernel).
+struct ClassBuffers {
+  int ncls = 0;      // 0: no class list
+  int cw = 1;
+  int bits = 0;      // bits of a (class, x offset) key
+  uint32_t *perm;    // list order -> sorted position: a subproblem's points by class and x offset
+  uint16_t *start;   // per subproblem: first entry of each class in its part of the list
+  uint32_t *vmax;    // bits of the largest |re|, |im| of the values
+};
+
 struct SortBuffers {
   uint32_t *keys[2];
   uint32_t *idx[2];
@@ -86,6 +123,8 @@ struct SortBuffers {
   int passes;
   int max_sub;
   int sub_work;        // fixed cost of a subproblem in kWorkUnit units
+  bool along_x;        // pencils of the list run along x (else y)
+  ClassBuffers cls;
 };
 
 // One batched FFT pass over lines of a 3D (or 1D) array.
@@ -145,6 +184,11 @@ struct PointArgs {
   const uint32_t *perm;      // sorted order -> original point index
   const int4 *subs;
   const uint32_t *nsub;      // device: [0] subproblems, [1] their total work (subs[i].w units)
+  // the class list of the matrix-core kernels (ClassBuffers)
+  const uint32_t *cperm;
+  const uint16_t *cstart;
+  const uint32_t *vmax;
+  int ncls, cw;
 };
 
 // Compact per-point records in sorted order for the MFMA kernels, 32 bytes
@@ -184,8 +228,9 @@ struct BinProblem {
   ZRec out;                 // records (REC) ...
   uint32_t *keys_out, *idx_out;  // ... or sorted keys and the permutation
   const float2 *values;     // record values (Type-1 strengths, gradient u) or null
-  int dim, nbins, bits, max_sub, sub_work, nchunks;
-  uint32_t chunk0, scan0;
+  int dim, nbins, bits, max_sub, sub_work, nchunks, along_x;
+  ClassBuffers cls;
+  uint32_t chunk0, scan0, piece0;
   int fused;                // one problem: the scatter launch also writes the list
 };
 
@@ -199,7 +244,7 @@ struct SpreadProblem {
   Geom g;
 };
 
-constexpr int kBatchChunk = 16;  // descriptors per table-fill launch (kernarg size)
+constexpr int kBatchChunk = 12;  // descriptors per table-fill launch (kernarg size)
 struct BatchChunk {
   int first;
   int count;
@@ -220,7 +265,8 @@ hipError_t sort_points_batched(BinProblem *host_probs, int nprob, BinProblem *de
 // Whether a tile count takes the one-pass binning, and the entries of
 // SortBuffers::cnt the binning of num_points points needs.
 bool sort_one_pass(int nbins);
-size_t sort_count_entries(int64_t num_points, int nbins);
+size_t radix_count_entries(int64_t num_points);              // digit passes
+size_t one_pass_count_entries(int64_t num_points, int nbins);  // 0: not one pass
 
 hipError_t launch_fft_pass(const FftPass &p, hipStream_t s);
 
@@ -231,28 +277,45 @@ hipError_t launch_fft_pass(const FftPass &p, hipStream_t s);
 int point_rec_floats(int w);
 hipError_t launch_point_prep(int w, const PointArgs &pa, const float2 *values, const Geom &g,
                              const KbPoly &poly, float *rec, uint8_t *xo, hipStream_t s);
-hipError_t launch_spread3d(int w, int method, const PointArgs &pa, const float *rec,
-                           const uint8_t *xo, ZRec zr, float2 *grid, const Geom &g,
-                           const KbPoly &poly, const KbPoly *dpoly, int num_blocks, hipStream_t s);
-hipError_t launch_spread3d_batched(int w, int method, const SpreadProblem *host_probs, int nprob,
+// 3D kernels on the vector ALUs.
+hipError_t launch_spread3d(int w, const PointArgs &pa, const float *rec, const uint8_t *xo,
+                           float2 *grid, const Geom &g, const KbPoly &poly, int num_blocks,
+                           hipStream_t s);
+hipError_t launch_spread3d_batched(int w, const SpreadProblem *host_probs, int nprob,
                                    SpreadProblem *dev_table, uint32_t *dev_prefix,
-                                   const KbPoly &poly, const KbPoly *dpoly, int num_blocks,
-                                   hipStream_t s);
-// MFMA interpolation needs 2 nbins floats of scratch (bin and tile maxima).
-// Tile maxima of the grid for the MFMA interpolation (no-op for the vector
-// ALU method); launch_interp3d reads them from the same scratch.
-// bin_max_done: the bin maxima (first half of the scratch) were written by the
-// last FFT pass (FftPass::bmax), so only the tile maxima are computed.
-hipError_t launch_tile_max3d(int w, int method, const float2 *grid, float *scratch, const Geom &g,
-                             hipStream_t s, bool bin_max_done = false);
-// cus: the device's CU count (the windowed kernel weights the shares of the
-// older and younger workgroup of a CU when the grid holds two per CU).
-hipError_t launch_interp3d(int w, int method, const PointArgs &pa, ZRec zr, const float2 *grid,
-                           float *scratch, float2 *out, const Geom &g, const KbPoly &poly,
-                           const KbPoly *dpoly, int num_blocks, int cus, hipStream_t s);
-hipError_t launch_grad3d(int w, int method, const PointArgs &pa, ZRec zr, const float2 *grid,
-                         const float2 *u, float *gx, float *gy, float *gz, const Geom &g,
-                         const KbPoly &poly, const KbPoly *dpoly, int num_blocks, hipStream_t s);
+                                   const KbPoly &poly, int num_blocks, hipStream_t s);
+hipError_t launch_interp3d(int w, const PointArgs &pa, const float2 *grid, float2 *out,
+                           const Geom &g, const KbPoly &poly, int num_blocks, hipStream_t s);
+hipError_t launch_grad3d(int w, const PointArgs &pa, const float2 *grid, const float2 *u, float *gx,
+                         float *gy, float *gz, const Geom &g, const KbPoly &poly, int num_blocks,
+                         hipStream_t s);
+// Matrix-core kernels on 16-row windows (window.hip), on the class list of
+// the binning (PointArgs::cperm, cstart) and its records.
+int win_bin_x(int w);          // tile interior along x
+// workgroups per CU of the launches
+int win_spread_groups(int w, int64_t num_points, int cus);
+hipError_t launch_win_spread(int w, const PointArgs &pa, ZRec zr, float2 *grid, const Geom &g,
+                             const WinPoly *dpoly, int num_blocks, hipStream_t s);
+// On 32 x 32 blocks (block_spread.hip), on a tile list along x.
+int block_bin_x(int w);
+hipError_t launch_block_spread(int w, const PointArgs &pa, ZRec zr, float2 *grid, const Geom &g,
+                               const WinPoly *dpoly, int num_blocks, hipStream_t s);
+hipError_t launch_win_spread_batched(int w, const SpreadProblem *host_probs, int nprob,
+                                     SpreadProblem *dev_table, uint32_t *dev_prefix,
+                                     const WinPoly *dpoly, int num_blocks, hipStream_t s);
+int win_interp_groups(int w, int64_t num_points, int cus);
+int win_grad_groups(int w, int64_t num_points, int cus);
+// Tile maxima from the bin maxima the last FFT pass wrote (FftPass::bmax):
+// the scales of the interpolation and gradient windows of class geometry
+// (ncls, cw).
+hipError_t launch_win_tile_max(int w, const float *bmax, float *tmax, const Geom &g, int ncls,
+                               int cw, hipStream_t s);
+hipError_t launch_win_interp(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
+                             const float *tmax, float2 *out, const Geom &g, const WinPoly *dpoly,
+                             int num_blocks, hipStream_t s);
+hipError_t launch_win_grad(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
+                           const float *tmax, float *gx, float *gy, float *gz, const Geom &g,
+                           const WinPoly *dpoly, int num_blocks, hipStream_t s);
 
 // Direct FP64 sums (direct.hip): type 1 writes every mode, type 2 every point.
 hipError_t launch_direct(int type, const PointArgs &pa, int dim, const int64_t n[3],
@@ -281,11 +344,12 @@ inline int bin1d(int w) { return kTile1d - 2 * w + 1; }
 // LDS bytes of the 3D spread/interp kernels for a geometry.
 size_t spread_lds_bytes(int w, int method, const Geom &g);
 int spread_bin_x(int w, int method);        // spreading tile interior along x
-int interp_blocks_per_cu(int w, int method);  // workgroups per CU of 3D interpolation
-// The MFMA gradient kernel keeps two x cells per wave; at w = 8 (32-cell
-// tiles, 16 waves) it would not fit the registers, so w = 8 uses LDS tiles.
-inline bool grad_uses_mfma(int w, int method) { return method == kSpreadMfma && w < 8; }
-int spread_block_threads(int w, int method);
+// Window classes of a matrix-core tile of bin_y rows: the points whose y
+// offsets fill `cw` <= 17 - 2w consecutive values share one 16-row window.
+inline int class_count(int w, int bin_y) { return (bin_y + 16 - 2 * w) / (17 - 2 * w); }
+inline int class_width(int w, int bin_y) { return (bin_y + class_count(w, bin_y) - 1) / class_count(w, bin_y); }
+// Plans whose backward calls share one binning (the two fused entry points).
+inline bool fused_backward_ok(int w, int method) { return method == kSpreadMfma && w < 8; }
 size_t interp_lds_bytes(int w, const Geom &g, bool grad);
 
 // ---- device helpers ----------------------------------------------------------

@@ -212,7 +212,7 @@ struct anufft_plan {
   int blue_n[3] = {0, 0, 0};        // Bluestein length per axis (0: direct mixed radix)
   float2 *d_chirp[3] = {nullptr, nullptr, nullptr};
   float2 *d_bhat[3] = {nullptr, nullptr, nullptr};
-  KbPoly *d_poly = nullptr;         // device copy of poly (read by the MFMA kernels)
+  WinPoly *d_poly = nullptr;        // device polynomials of the matrix-core kernels
   KbPoly poly{};
   double poly_err = 0;
   // Binning geometries: spreading (register columns) and interpolation /
@@ -222,7 +222,19 @@ struct anufft_plan {
     int nbins = 1;
     int passes = 1;
     int max_sub = 1024;
+    // 3D matrix-core tiles: y-offset classes per tile, offsets per class
+    int ncls = 0, cw = 1;
+    bool along_x = false;  // pencils of the tile list
+    // points per entry of the tile list: max_sub, for a class list at most
+    // the points it lists at once (and not so few that the entries outgrow
+    // the workspace kept for them)
+    int list_sub() const { return ncls > 0 ? std::max(32, std::min(max_sub, kClassSub)) : max_sub; }
+    // entries at most: empty tiles have none
+    int64_t list_len(int64_t M) const {
+      return std::min<int64_t>(nbins, M) + (M + list_sub() - 1) / list_sub();
+    }
   } bs, bi, bg;
+  Binning bf;  // blocks of the FP64 host Type-1 (3D, matrix cores)
   int lds_max = 163840; // gfx950 LDS per workgroup
   int kernel_method = kSpreadMfma;
   hipStream_t host_stream = nullptr;
@@ -251,7 +263,7 @@ struct DeviceGuard {
   }
 };
 
-Layout layout(const anufft_plan *p, int64_t M) {
+Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
   Layout l;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -267,17 +279,23 @@ Layout layout(const anufft_plan *p, int64_t M) {
     l.keys1 = take(4 * Mp);
     l.idx0 = take(4 * Mp);
     l.idx1 = take(4 * Mp);
-    const int nb = std::max(p->bs.nbins, std::max(p->bi.nbins, p->bg.nbins));
-    size_t cnt_n = 0;
-    for (const anufft_plan::Binning *b : {&p->bs, &p->bi, &p->bg})
-      cnt_n = std::max(cnt_n, sort_count_entries(M, b->nbins));
+    const anufft_plan::Binning *const all[] = {&p->bs, &p->bi, &p->bg, &p->bf};
+    const int kinds = blocks ? 4 : 3;
+    int nb = 1;
+    size_t cnt_n = radix_count_entries(M), one_n = 0;
+    for (int i = 0; i < kinds; ++i) {
+      const anufft_plan::Binning *b = all[i];
+      nb = std::max(nb, b->nbins);
+      one_n = std::max(one_n, one_pass_count_entries(M, b->nbins));
+    }
+    const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
+    if (!classes) cnt_n = std::max(cnt_n, one_n);
     l.cnt = take(4 * cnt_n);
     l.scan = take(4 * (size_t)std::max(kRadix, nb));  // digit (or tile) totals
     l.bin_start = take(4 * (size_t)(nb + 1));
-    l.sub_ofs = take(4 * (size_t)(nb + 2));
+    l.sub_ofs = take(4 * (size_t)(nb + 3));  // (nb unused,) list totals, value maximum
     int64_t nsub = 1;
-    for (const anufft_plan::Binning *b : {&p->bs, &p->bi, &p->bg})
-      nsub = std::max<int64_t>(nsub, b->nbins + (M + b->max_sub - 1) / b->max_sub + 1);
+    for (int i = 0; i < kinds; ++i) nsub = std::max<int64_t>(nsub, all[i]->list_len(M) + 1);
     l.subs = take(16 * (size_t)nsub);
     if (p->dim == 1) {
       l.zrec = take(32 * Mp);   // point records of the 1D binning
@@ -286,14 +304,18 @@ Layout layout(const anufft_plan *p, int64_t M) {
       l.total = off;
       return l;
     }
-    if (p->kernel_method == kSpreadMfma) {
+    if (classes) {
       l.zrec = take(32 * Mp);   // ZRec: 32-byte record per point
-      l.zrec2 = take(32 * Mp);  // the other record buffer of the binning passes
+      // the other record buffer of the digit passes, or the chunk counts of
+      // the one-pass binning; once the records are in place, the class starts
+      // of the subproblems (2 bytes each, at most 16 a point).  The class list
+      // itself takes the place of the permutation, which the records replace.
+      l.zrec2 = take(std::max(32 * Mp, 4 * one_n));
       l.tmax = take(2 * sizeof(float) * (size_t)(p->bi.nbins + 1));  // bin and tile maxima
-    }
-    else
+    } else {
       l.rec = take(sizeof(float) * (size_t)point_rec_floats(p->w) * Mp);
-    l.xo = take(Mp);
+      l.xo = take(Mp);
+    }
     l.grid = take(8 * (size_t)p->cells());
     l.fftbuf = take(8 * (size_t)(p->m[0] * p->m[1] * p->n[2]));
   }
@@ -405,8 +427,16 @@ anufft_status build_tables(anufft_plan *p) {
 
   DeviceGuard guard(p->device);
   {
-    hipError_t e = hipMalloc(&p->d_poly, sizeof(KbPoly));
-    if (e == hipSuccess) e = hipMemcpy(p->d_poly, &p->poly, sizeof(KbPoly), hipMemcpyHostToDevice);
+    WinPoly wp;
+    wp.p = p->poly;
+    for (int d = 0; d < kPolyCoefs; ++d)
+      for (int i = 0; i < kMaxTaps; ++i) {
+        wp.fac[d][i] = p->poly.c[d][i] * kFacScale;
+        wp.op[d][i] = p->poly.c[d][i] * kOpScale;
+        wp.dop[d][i] = p->poly.dc[d][i] * kOpScaleD;
+      }
+    hipError_t e = hipMalloc(&p->d_poly, sizeof(WinPoly));
+    if (e == hipSuccess) e = hipMemcpy(p->d_poly, &wp, sizeof(WinPoly), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "device kernel polynomials");
   }
   hipError_t es = hipStreamCreateWithFlags(&p->host_stream, hipStreamNonBlocking);
@@ -520,13 +550,23 @@ void choose_bins(anufft_plan *p) {
   // with the cells shared evenly (128 cells: 8 tiles of 16 rather than 7 of
   // 18 and one of 2), so that no tile pays the fixed cost of a tile for a
   // sliver of the points
-  auto even = [&](int a) {
-    const int m = (int)p->m[a], nt = (m + cyz - 1) / cyz;
-    return p->kernel_method == kSpreadMfma ? (m + nt - 1) / nt : cyz;
+  const bool mfma = p->kernel_method == kSpreadMfma;
+  auto even = [&](int a, int c) {
+    const int m = (int)p->m[a], nt = (m + c - 1) / c;
+    return mfma ? (m + nt - 1) / nt : cyz;
   };
-  const int bsp[3] = {spread_bin_x(p->w, p->kernel_method), even(1), even(2)};
+  const int bsp[3] = {spread_bin_x(p->w, p->kernel_method), even(1, p->w == 7 ? 15 : cyz), even(2, cyz)};
+  // (y at w = 7: five whole classes of three offsets rather than six)
   set_geom(p->bs, p, bsp);
   p->bs.max_sub = p->opts.max_subproblem > 0 ? p->opts.max_subproblem : 4096;
+  if (p->kernel_method == kSpreadMfma) {
+    p->bs.cw = class_width(p->w, p->bs.g.bin[1]);
+    p->bs.ncls = (p->bs.g.bin[1] + p->bs.cw - 1) / p->bs.cw;
+    const int bf[3] = {block_bin_x(p->w), even(1, cyz), even(2, cyz)};
+    set_geom(p->bf, p, bf);
+    p->bf.max_sub = p->bs.max_sub;
+    p->bf.along_x = true;
+  }
 
   // LDS-tile geometry (gradient; interpolation on the vector-ALU path)
   const int cand[] = {32, 24, 16, 12, 10, 8, 6, 4, 3, 2, 1};
@@ -559,6 +599,8 @@ void choose_bins(anufft_plan *p) {
   if (p->kernel_method == kSpreadMfma) {
     set_geom(p->bi, p, bsp);  // MFMA interpolation uses the spreading tiles
     p->bi.max_sub = p->bs.max_sub;
+    p->bi.ncls = p->bs.ncls;
+    p->bi.cw = p->bs.cw;
   } else {
     p->bi = p->bg;
   }
@@ -745,8 +787,50 @@ struct Exec {
       if (e != hipSuccess) return e;
     }
     return timed(ANUFFT_STAGE_SPREAD, [&] {
-      return launch_spread3d(p->w, p->kernel_method, pa, rec(), xo(), zrec(pa.num_points), grid,
-                             p->bs.g, p->poly, p->d_poly, blocks(p->bs, pa.num_points, 2), s);
+      if (p->kernel_method == kSpreadMfma)
+        return launch_win_spread(p->w, pa, zrec(pa.num_points), grid, p->bs.g, p->d_poly,
+                                 blocks(p->bs, pa.num_points, win_spread_groups(p->w, pa.num_points, p->cus)), s);
+      return launch_spread3d(p->w, pa, rec(), xo(), grid, p->bs.g, p->poly,
+                             blocks(p->bs, pa.num_points, 2), s);
+    });
+  }
+  hipError_t spread_blocks(const PointArgs &pa, float2 *grid) const {
+    return timed(ANUFFT_STAGE_SPREAD, [&] {
+      return launch_block_spread(p->w, pa, zrec(pa.num_points), grid, p->bf.g, p->d_poly,
+                                 blocks(p->bf, pa.num_points, 2), s);
+    });
+  }
+  // Bin maxima, then tile maxima, of the fine grid (matrix-core kernels).
+  float *bmax() const { return (float *)(ws + lay.tmax); }
+  float *tmax() const { return bmax() + p->bi.nbins; }
+  // The fine grid of `modes` (this workspace), with the tile maxima the
+  // matrix-core interpolation and gradient scale by.
+  hipError_t fine_grid(const float2 *modes, bool compat) const {
+    const bool mf = p->kernel_method == kSpreadMfma;
+    hipError_t e = timed(ANUFFT_STAGE_FFT, [&] { return modes_to_grid(modes, compat, mf); });
+    if (e != hipSuccess || !mf) return e;
+    return timed(ANUFFT_STAGE_TILE_MAX, [&] {
+      return launch_win_tile_max(p->w, bmax(), tmax(), p->bi.g, p->bi.ncls, p->bi.cw, s);
+    });
+  }
+  // Type-2 interpolation and coordinate gradient of binned points from the
+  // fine grid in `from`'s workspace.
+  hipError_t interp3(const PointArgs &pa, const Exec &from, float2 *out) const {
+    return timed(ANUFFT_STAGE_INTERP, [&] {
+      if (p->kernel_method == kSpreadMfma)
+        return launch_win_interp(p->w, pa, zrec(pa.num_points), from.grid(), from.tmax(), out, p->bi.g,
+                                 p->d_poly, blocks(p->bi, pa.num_points, win_interp_groups(p->w, pa.num_points, p->cus)), s);
+      return launch_interp3d(p->w, pa, from.grid(), out, p->bi.g, p->poly,
+                             blocks(p->bi, pa.num_points, 4), s);
+    });
+  }
+  hipError_t grad3(const PointArgs &pa, const Exec &from, const float2 *u, float *const g[3]) const {
+    return timed(ANUFFT_STAGE_GRAD, [&] {
+      if (p->kernel_method == kSpreadMfma)
+        return launch_win_grad(p->w, pa, zrec(pa.num_points), from.grid(), from.tmax(), g[0], g[1], g[2],
+                               p->bi.g, p->d_poly, blocks(p->bi, pa.num_points, win_grad_groups(p->w, pa.num_points, p->cus)), s);
+      return launch_grad3d(p->w, pa, from.grid(), u, g[0], g[1], g[2], p->bg.g, p->poly,
+                           blocks(p->bg, pa.num_points, 4), s);
     });
   }
   float2 *fftbuf() const { return (float2 *)(ws + lay.fftbuf); }
@@ -756,7 +840,8 @@ struct Exec {
     sb.keys[1] = (uint32_t *)(ws + lay.keys1);
     sb.idx[0] = (uint32_t *)(ws + lay.idx0);
     sb.idx[1] = (uint32_t *)(ws + lay.idx1);
-    sb.cnt = (uint32_t *)(ws + lay.cnt);
+    const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
+    sb.cnt = (uint32_t *)(ws + (classes && sort_one_pass(b.nbins) ? lay.zrec2 : lay.cnt));
     sb.scan_tmp = (uint32_t *)(ws + lay.scan);
     sb.bin_start = (uint32_t *)(ws + lay.bin_start);
     sb.sub_ofs = (uint32_t *)(ws + lay.sub_ofs);
@@ -764,8 +849,21 @@ struct Exec {
     sb.nbins = b.nbins;
     sb.nchunks = lay.nchunks;
     sb.passes = b.passes;
-    sb.max_sub = b.max_sub;
+    sb.max_sub = b.list_sub();
+    sb.along_x = b.along_x;
     sb.sub_work = p->opts.sub_work > 0 ? p->opts.sub_work : (int)kSubWork;
+    if (b.ncls > 0) {
+      // the fixed cost of a subproblem is that of its classes, each an eighth
+      // of the setting (a partly filled round, the rows the window steps)
+      sb.sub_work = std::max(1, sb.sub_work * b.ncls / 8);
+      ClassBuffers &c = sb.cls;
+      c.ncls = b.ncls;
+      c.cw = b.cw;
+      while ((1 << c.bits) < b.ncls * b.g.bin[0]) ++c.bits;
+      c.perm = sb.idx[0];
+      c.start = (uint16_t *)(ws + lay.zrec2);
+      c.vmax = sb.sub_ofs + b.nbins + 2;
+    }
     return sb;
   }
   PointArgs point_args(const anufft_plan::Binning &b, int64_t M, const float *const c[3],
@@ -780,14 +878,19 @@ struct Exec {
     pa.perm = sb.idx[b.passes & 1];
     pa.subs = sb.subs;
     pa.nsub = sb.sub_ofs + b.nbins;
+    pa.cperm = sb.cls.perm;
+    pa.cstart = sb.cls.start;
+    pa.vmax = sb.cls.vmax;
+    pa.ncls = b.ncls;
+    pa.cw = b.cw;
     return pa;
   }
   // Workgroups of a 3D point kernel: per_cu per CU (the plan's blocks_per_cu
   // when set), at most one per subproblem.
   int blocks(const anufft_plan::Binning &b, int64_t M, int per_cu) const {
     if (p->opts.blocks_per_cu > 0) per_cu = p->opts.blocks_per_cu;
-    int64_t up = (int64_t)b.nbins + (M + b.max_sub - 1) / b.max_sub;
-    int64_t n = std::min<int64_t>(up, (int64_t)per_cu * p->cus);
+    int64_t up = b.list_len(M) * std::max(1, b.ncls);
+    int64_t n = std::min<int64_t>(std::min(up, M), (int64_t)per_cu * p->cus);
     return (int)std::max<int64_t>(n, 1);
   }
 
@@ -857,7 +960,7 @@ struct Exec {
 };
 
 // Smallest subproblem (points) of the fused batched spreading.
-constexpr int kBatchMinSub = 4096;
+constexpr int kBatchMinSub = kClassSub;
 
 // Point counts: the subproblem list and the per-point records carry point
 // positions as signed 32-bit integers, so at most 2^31 - 1 points per call.
@@ -1083,27 +1186,28 @@ anufft_status anufft_workspace_size(const anufft_plan *p, int64_t max_points, si
   return ANUFFT_OK;
 }
 
-anufft_status anufft_execute_type1(const anufft_plan *p, int64_t M, const float *const coords[3],
-                                   int64_t stride, const float *values, float *out, void *ws,
-                                   size_t ws_bytes, void *stream) {
-  Layout lay;
-  anufft_status st = check_exec(p, M, coords, stride, values, out, ws, ws_bytes, lay);
-  if (st != ANUFFT_OK) return st;
+// Type-1 of checked arguments; blocks: spread on the blocks of bf, in a
+// workspace laid out for them.
+static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *const coords[3],
+                               int64_t stride, const float *values, float *out, void *ws,
+                               const Layout &lay, hipStream_t stream, bool blocks) {
   DeviceGuard guard(p->device);
-  Exec ex{p, (hipStream_t)stream, (char *)ws, lay};
+  Exec ex{p, stream, (char *)ws, lay};
+  const anufft_plan::Binning &bs = blocks ? p->bf : p->bs;
   hipError_t e = hipSuccess;
   if (M > 0) {
-    PointArgs pa = ex.point_args(p->bs, M, coords, stride);
+    PointArgs pa = ex.point_args(bs, M, coords, stride);
     const bool records = p->dim == 1 || p->kernel_method == kSpreadMfma;
     // zeroing the grid (second stream) is independent of the binning
     e = ex.fork_join(
         [&](const Exec &ea) {
           return ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
         },
-        [&] { return ex.bin(p->bs, pa, (const float2 *)values, records); });
+        [&] { return ex.bin(bs, pa, (const float2 *)values, records); });
     if (e != hipSuccess) return hip_fail(e, "fill / binning");
     if (p->dim == 3) {
-      e = ex.spread3(pa, (const float2 *)values, ex.grid());
+      e = blocks ? ex.spread_blocks(pa, ex.grid())
+                 : ex.spread3(pa, (const float2 *)values, ex.grid());
     } else {
       e = ex.timed(ANUFFT_STAGE_SPREAD, [&] {
         return launch_spread1d(p->w, pa, ex.zrec(M), ex.grid(), p->bs.g, p->poly,
@@ -1118,6 +1222,15 @@ anufft_status anufft_execute_type1(const anufft_plan *p, int64_t M, const float 
   e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.grid_to_modes((float2 *)out); });
   if (e != hipSuccess) return hip_fail(e, "fft");
   return ANUFFT_OK;
+}
+
+anufft_status anufft_execute_type1(const anufft_plan *p, int64_t M, const float *const coords[3],
+                                   int64_t stride, const float *values, float *out, void *ws,
+                                   size_t ws_bytes, void *stream) {
+  Layout lay;
+  anufft_status st = check_exec(p, M, coords, stride, values, out, ws, ws_bytes, lay);
+  if (st != ANUFFT_OK) return st;
+  return run_type1(p, M, coords, stride, values, out, ws, lay, (hipStream_t)stream, false);
 }
 
 anufft_status anufft_scratch_capacity(size_t *bytes) {
@@ -1164,24 +1277,11 @@ anufft_status anufft_execute_type2(const anufft_plan *p, int64_t M, const float 
     // the FFT goes to the plan's second stream, joined before interpolation
     e = ex.fork_join(
         [&](const Exec &ea) {
-          hipError_t r = ea.timed(ANUFFT_STAGE_FFT, [&] {
-            return ea.modes_to_grid((const float2 *)modes,
-                                    p->opts.compat_reference_type2_3d_scaling != 0, true);
-          });
-          if (r != hipSuccess) return r;
-          return ea.timed(ANUFFT_STAGE_TILE_MAX, [&] {
-            return launch_tile_max3d(p->w, p->kernel_method, ea.grid(),
-                                     (float *)(ea.ws + lay.tmax), p->bi.g, ea.s, true);
-          });
+          return ea.fine_grid((const float2 *)modes, p->opts.compat_reference_type2_3d_scaling != 0);
         },
         [&] { return ex.bin(p->bi, pa, nullptr, p->kernel_method == kSpreadMfma); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
-    e = ex.timed(ANUFFT_STAGE_INTERP, [&] {
-      return launch_interp3d(p->w, p->kernel_method, pa, ex.zrec(M), ex.grid(),
-                             (float *)(ex.ws + lay.tmax), (float2 *)out, p->bi.g, p->poly, p->d_poly,
-                             ex.blocks(p->bi, M, interp_blocks_per_cu(p->w, p->kernel_method)),
-                             p->cus, ex.s);
-    });
+    e = ex.interp3(pa, ex, (float2 *)out);
   } else {
     PointArgs pa = ex.point_args(p->bi, M, coords, stride);
     e = ex.fork_join(
@@ -1214,21 +1314,14 @@ anufft_status anufft_execute_grad_points(const anufft_plan *p, int64_t M,
   hipError_t e;
   // the derivative always uses the unnormalized (direct-sum) scaling
   if (p->dim == 3) {
-    const bool gm = grad_uses_mfma(p->w, p->kernel_method);
+    const bool gm = p->kernel_method == kSpreadMfma;
     const anufft_plan::Binning &b = gm ? p->bi : p->bg;
     PointArgs pa = ex.point_args(b, M, coords, stride);
     // FFT passes (second stream) concurrent with the binning
-    e = ex.fork_join(
-        [&](const Exec &ea) {
-          return ea.timed(ANUFFT_STAGE_FFT, [&] { return ea.modes_to_grid((const float2 *)modes_h, false); });
-        },
-        [&] { return ex.bin(b, pa, (const float2 *)u, gm); });
+    e = ex.fork_join([&](const Exec &ea) { return ea.fine_grid((const float2 *)modes_h, false); },
+                     [&] { return ex.bin(b, pa, (const float2 *)u, gm); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
-    e = ex.timed(ANUFFT_STAGE_GRAD, [&] {
-      return launch_grad3d(p->w, p->kernel_method, pa, ex.zrec(M), ex.grid(), (const float2 *)u,
-                           grad[0], grad[1], grad[2], b.g, p->poly, p->d_poly,
-                           ex.blocks(b, M, gm ? 1 : 4), ex.s);
-    });
+    e = ex.grad3(pa, ex, (const float2 *)u, grad);
   } else {
     // records carry u (value fields): the gradient reads it in sorted order
     PointArgs pa = ex.point_args(p->bg, M, coords, stride);
@@ -1257,7 +1350,7 @@ anufft_status anufft_execute_type2_backward(const anufft_plan *p, int64_t M,
   if (st != ANUFFT_OK) return st;
   if (!grad_modes) return fail(ANUFFT_INVALID_ARG, "grad_modes is NULL");
   if (M > 0 && (!grad_x || !grad_x[0])) return fail(ANUFFT_INVALID_ARG, "grad_x[0] is NULL");
-  if (p->dim != 3 || !grad_uses_mfma(p->w, p->kernel_method))
+  if (p->dim != 3 || !fused_backward_ok(p->w, p->kernel_method))
     return fail(ANUFFT_UNSUPPORTED, "the fused Type-2 backward needs a 3D plan on the MFMA kernels (w <= 7)");
   if (ws_bytes < 2 * lay.total)
     return fail(ANUFFT_CAPACITY_EXCEEDED, "workspace of %zu bytes is smaller than the %zu required",
@@ -1275,7 +1368,7 @@ anufft_status anufft_execute_type2_backward(const anufft_plan *p, int64_t M,
       [&](const Exec &ea) {
         Exec eb = eh;
         eb.s = ea.s;
-        hipError_t r = eb.timed(ANUFFT_STAGE_FFT, [&] { return eb.modes_to_grid((const float2 *)modes, false); });
+        hipError_t r = eb.fine_grid((const float2 *)modes, false);
         if (r == hipSuccess)
           r = ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
         return r;
@@ -1286,11 +1379,7 @@ anufft_status anufft_execute_type2_backward(const anufft_plan *p, int64_t M,
   if (e != hipSuccess) return hip_fail(e, "spread");
   e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.grid_to_modes((float2 *)grad_modes); });
   if (e != hipSuccess) return hip_fail(e, "fft");
-  e = ex.timed(ANUFFT_STAGE_GRAD, [&] {
-    return launch_grad3d(p->w, p->kernel_method, pa, ex.zrec(M), eh.grid(), (const float2 *)g,
-                         grad_x[0], grad_x[1], grad_x[2], p->bi.g, p->poly, p->d_poly,
-                         ex.blocks(p->bi, M, 1), ex.s);
-  });
+  e = ex.grad3(pa, eh, (const float2 *)g, grad_x);
   if (e != hipSuccess) return hip_fail(e, "grad");
   return ANUFFT_OK;
 }
@@ -1305,7 +1394,7 @@ anufft_status anufft_execute_type1_backward(const anufft_plan *p, int64_t M,
   if (st != ANUFFT_OK) return st;
   if (M > 0 && !grad_values) return fail(ANUFFT_INVALID_ARG, "grad_values is NULL");
   if (M > 0 && (!grad_x || !grad_x[0])) return fail(ANUFFT_INVALID_ARG, "grad_x[0] is NULL");
-  if (p->dim != 3 || !grad_uses_mfma(p->w, p->kernel_method))
+  if (p->dim != 3 || !fused_backward_ok(p->w, p->kernel_method))
     return fail(ANUFFT_UNSUPPORTED, "the fused Type-1 backward needs a 3D plan on the MFMA kernels (w <= 7)");
   if (M == 0) return ANUFFT_OK;
   DeviceGuard guard(p->device);
@@ -1315,28 +1404,12 @@ anufft_status anufft_execute_type1_backward(const anufft_plan *p, int64_t M,
   // the values c (ignored by the interpolation, u of the gradient)
   PointArgs pa = ex.point_args(p->bi, M, coords, stride);
   hipError_t e = ex.fork_join(
-      [&](const Exec &ea) {
-        hipError_t r = ea.timed(ANUFFT_STAGE_FFT, [&] { return ea.modes_to_grid((const float2 *)G, false, true); });
-        if (r != hipSuccess) return r;
-        return ea.timed(ANUFFT_STAGE_TILE_MAX, [&] {
-          return launch_tile_max3d(p->w, p->kernel_method, ea.grid(), (float *)(ea.ws + lay.tmax),
-                                   p->bi.g, ea.s, true);
-        });
-      },
+      [&](const Exec &ea) { return ea.fine_grid((const float2 *)G, false); },
       [&] { return ex.bin(p->bi, pa, (const float2 *)values, true); });
   if (e != hipSuccess) return hip_fail(e, "fft / binning");
-  e = ex.timed(ANUFFT_STAGE_INTERP, [&] {
-    return launch_interp3d(p->w, p->kernel_method, pa, ex.zrec(M), ex.grid(),
-                           (float *)(ex.ws + lay.tmax), (float2 *)grad_values, p->bi.g, p->poly,
-                           p->d_poly, ex.blocks(p->bi, M, interp_blocks_per_cu(p->w, p->kernel_method)),
-                           p->cus, ex.s);
-  });
+  e = ex.interp3(pa, ex, (float2 *)grad_values);
   if (e != hipSuccess) return hip_fail(e, "interp");
-  e = ex.timed(ANUFFT_STAGE_GRAD, [&] {
-    return launch_grad3d(p->w, p->kernel_method, pa, ex.zrec(M), ex.grid(), (const float2 *)values,
-                         grad_x[0], grad_x[1], grad_x[2], p->bi.g, p->poly, p->d_poly,
-                         ex.blocks(p->bi, M, 1), ex.s);
-  });
+  e = ex.grad3(pa, ex, (const float2 *)values, grad_x);
   if (e != hipSuccess) return hip_fail(e, "grad");
   return ANUFFT_OK;
 }
@@ -1430,6 +1503,7 @@ anufft_status anufft_debug_sort(const anufft_plan *p, int64_t M, const float *co
   Exec ex{p, (hipStream_t)stream, (char *)ws, lay};
   PointArgs pa = ex.point_args(p->bs, M, coords, stride);
   SortBuffers sb = ex.sort_buffers(p->bs);
+  sb.cls = ClassBuffers{};  // the permutation only
   hipError_t e = sort_points(pa, p->bs.g, p->dim, sb, ex.s);
   if (e != hipSuccess) return hip_fail(e, "binning");
   if (M > 0 && (e = hipMemcpyAsync(perm, pa.perm, 4 * (size_t)M, hipMemcpyDeviceToDevice, ex.s)) != hipSuccess)
@@ -1528,7 +1602,7 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
   std::vector<SpreadProblem> probs(nprob);
   ex.reserve(nprob);
   size_t off = 0;
-  int64_t sub_upper = 0;
+  int64_t sub_upper = 0, points = 0;
   for (int i = 0; i < nprob; ++i) {
     Layout lay = layout(plans[i], num_points[i]);
     ex.push_back(Exec{plans[i], s, (char *)ws + off, lay});
@@ -1540,7 +1614,8 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
     probs[i].zr = ex[i].zrec(num_points[i]);
     probs[i].grid = ex[i].grid();
     probs[i].g = plans[i]->bs.g;
-    sub_upper += plans[i]->bs.nbins + (num_points[i] + plans[i]->bs.max_sub - 1) / plans[i]->bs.max_sub;
+    points += num_points[i];
+    sub_upper += plans[i]->bs.list_len(num_points[i]) * std::max(1, plans[i]->bs.ncls);
   }
   SpreadProblem *table = (SpreadProblem *)((char *)ws + off);
   off += align_up(sizeof(SpreadProblem) * (size_t)nprob);
@@ -1557,12 +1632,15 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
   // one persistent launch splits the problems' combined work prefix, so
   // every problem weighs its subproblems alike, with the automatic weight
   // (the plans' own settings are tuned for single calls)
-  const int sub_work = (int)kSubWork;
+  auto sub_work = [&](int i) {
+    const int ncls = plans[i]->bs.ncls;
+    return ncls > 0 ? std::max(1, (int)kSubWork * ncls / 8) : (int)kSubWork;
+  };
   auto sort_range = [&](int parity, hipStream_t st) {
     for (int i = parity; i < nprob; i += 2) {
       const RecordOut ro{probs[i].zr, ex[i].zrec(num_points[i], true), (const float2 *)values[i]};
       SortBuffers sb = ex[i].sort_buffers(plans[i]->bs);
-      sb.sub_work = sub_work;
+      sb.sub_work = sub_work(i);
       // the persistent launch balances work across all problems itself:
       // smaller subproblems only add fixed costs there
       sb.max_sub = std::max(sb.max_sub, kBatchMinSub);
@@ -1593,7 +1671,8 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
       b.dim = 3;
       b.nbins = sb.nbins;
       b.max_sub = std::max(sb.max_sub, kBatchMinSub);
-      b.sub_work = sub_work;
+      b.sub_work = sub_work(i);
+      b.cls = sb.cls;
     }
   }
   e = e0.timed(ANUFFT_STAGE_BIN, [&] {
@@ -1622,10 +1701,12 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
     });
     if (e != hipSuccess) return hip_fail(e, "spread records");
   }
-  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(sub_upper, 2 * (int64_t)p0->cus));
+  const int per_cu = mf ? win_spread_groups(p0->w, points, p0->cus) : 2;
+  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(sub_upper, per_cu * (int64_t)p0->cus));
   e = e0.timed(ANUFFT_STAGE_SPREAD, [&] {
-    return launch_spread3d_batched(p0->w, p0->kernel_method, probs.data(), nprob, table, prefix,
-                                   p0->poly, p0->d_poly, nblk, s);
+    if (mf)
+      return launch_win_spread_batched(p0->w, probs.data(), nprob, table, prefix, p0->d_poly, nblk, s);
+    return launch_spread3d_batched(p0->w, probs.data(), nprob, table, prefix, p0->poly, nblk, s);
   });
   if (e != hipSuccess) return hip_fail(e, "spread");
   // the problems' FFT passes, odd problems on the second stream
@@ -1756,7 +1837,11 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   std::vector<float> hc((size_t)std::max<int64_t>(M, 1) * p->dim);
   for (int a = 0; a < p->dim; ++a)
     for (int64_t j = 0; j < M; ++j) hc[(size_t)a * M + j] = (float)coords[a][j * stride];
-  size_t wsb = layout(p, M).total;
+  // FP64 results keep one summation order (block_spread.hip)
+  const bool blocks = type == 1 && storage == ANUFFT_STORAGE_C128 && p->dim == 3 &&
+                      p->kernel_method == kSpreadMfma;
+  const Layout lay = layout(p, M, blocks);
+  const size_t wsb = lay.total;
   char *buf = nullptr;
   size_t b_in = align_up(8 * (size_t)std::max<int64_t>(nin, 1));
   size_t b_out = align_up(8 * (size_t)std::max<int64_t>(nout, 1));
@@ -1771,7 +1856,8 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
     if ((e = hipMemcpyAsync(d_in, hin.data(), 8 * (size_t)nin, hipMemcpyHostToDevice, s)) != hipSuccess) break;
     if ((e = hipMemcpyAsync(d_c, hc.data(), 4 * hc.size(), hipMemcpyHostToDevice, s)) != hipSuccess) break;
     const float *dc[3] = {d_c, p->dim == 3 ? d_c + M : d_c, p->dim == 3 ? d_c + 2 * M : d_c};
-    st = type == 1 ? anufft_execute_type1(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, wsb, s)
+    st = blocks    ? run_type1(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, lay, s, true)
+         : type == 1 ? anufft_execute_type1(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, wsb, s)
                    : anufft_execute_type2(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, wsb, s);
     if (st != ANUFFT_OK) break;
     if ((e = hipMemcpyAsync(hout.data(), d_out, 8 * (size_t)nout, hipMemcpyDeviceToHost, s)) != hipSuccess) break;

@@ -14,7 +14,7 @@
 //   bounds : bin_start[b] = lower_bound(sorted keys, b)
 //   subproblems (one block): scan of per-tile subproblem counts, list
 //   subs   : subproblems of at most max_sub points per tile, tiles in pencil
-//            order (x fastest)
+//            order (along y, or along x)
 #include <algorithm>
 
 #include "internal.h"
@@ -43,8 +43,9 @@ __device__ __forceinline__ uint32_t tile_key(const PointArgs &pa, const Geom &g,
 // keys + digit-0 histogram of each chunk, written digit-major.
 __global__ __launch_bounds__(kSortThreads) void keys_kernel(PointArgs pa, Geom g, int dim,
                                                             uint32_t *keys, uint32_t *cnt,
-                                                            int nchunks) {
+                                                            int nchunks, uint32_t *vmax) {
   __shared__ uint32_t hist[kRadix];
+  if (vmax && blockIdx.x == 0 && threadIdx.x == 0) *vmax = 0u;
   for (int d = threadIdx.x; d < kRadix; d += kSortThreads) hist[d] = 0;
   __syncthreads();
   int64_t base = (int64_t)blockIdx.x * kSortChunk;
@@ -158,7 +159,10 @@ struct RecMove {
   PointArgs pa;
   Geom g;
   int first;
+  uint32_t *vmax;        // first pass with values: their largest component, or null
 };
+
+__device__ __forceinline__ void value_max(float mx, uint32_t *vmax);
 
 template <bool REC>
 __global__ __launch_bounds__(kSortThreads) void scatter_kernel(
@@ -180,6 +184,7 @@ __global__ __launch_bounds__(kSortThreads) void scatter_kernel(
   __syncthreads();
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int64_t base = (int64_t)blockIdx.x * kSortChunk;
+  float mx = 0.f;
   for (int step = 0; step < kSortItems; ++step) {
     int64_t j = base + (int64_t)step * kSortThreads + tid;
     bool valid = j < n;
@@ -198,6 +203,7 @@ __global__ __launch_bounds__(kSortThreads) void scatter_kernel(
         const float2 c = rm.values ? rm.values[j] : make_float2(0.f, 0.f);
         ra = make_float4(z[0], z[1], z[2], __int_as_float(off));
         rb = make_float4(c.x, c.y, __uint_as_float(key), __uint_as_float(idx));
+        mx = fmaxf(mx, fmaxf(fabsf(c.x), fabsf(c.y)));
       } else {
         ra = rm.in.r[2 * j];
         rb = rm.in.r[2 * j + 1];
@@ -237,6 +243,7 @@ __global__ __launch_bounds__(kSortThreads) void scatter_kernel(
     }
     __syncthreads();
   }
+  if (REC && rm.vmax) value_max(mx, rm.vmax);
 }
 
 // bin_start[b] = first sorted position with key >= b, b in [0, nbins].
@@ -252,12 +259,17 @@ __global__ void bounds_kernel(KeySrc keys, int64_t n, uint32_t *bin_start, int n
   bin_start[b] = (uint32_t)lo;
 }
 
-// The subproblem list runs over the tiles in pencil order -- x fastest,
-// then z, then y -- so that consecutive entries are neighbouring tiles
-// along x; q is the position of a tile in that order.
-__device__ __forceinline__ int pencil_bin(int q, int3 nb) {
-  const int bx = q % nb.x, pz = q / nb.x;
-  return (bx * nb.y + pz / nb.z) * nb.z + pz % nb.z;
+// The subproblem list runs over the tiles in pencil order -- y fastest, then
+// z, then x, so that consecutive entries are neighbouring tiles along y, or
+// (along_x) x, z, y; q is the position of a tile in that order.
+__device__ __forceinline__ int pencil_bin(int q, int3 nb, bool along_x) {
+  if (along_x) {
+    const int bx = q % nb.x, pz = q / nb.x;
+    return (bx * nb.y + pz / nb.z) * nb.z + pz % nb.z;
+  }
+  const int by = q % nb.y, t = q / nb.y;
+  const int bx = t / nb.z;
+  return (bx * nb.y + by) * nb.z + (t - bx * nb.z);
 }
 
 // 64-bit exclusive scan over a block of NT threads (see block_scan_waves).
@@ -312,7 +324,7 @@ struct SubLds {
 template <int NT>
 __device__ __forceinline__ void subproblems_body(SubLds<NT> &L, uint32_t *bin_start,
                                                  const uint32_t *tot, int from_tot, int nbins,
-                                                 int3 nb, int max_sub, int sub_work,
+                                                 int3 nb, bool along_x, int max_sub, int sub_work,
                                                  uint32_t *nsub, int4 *subs) {
   constexpr int kSubRound = SubLds<NT>::kRound;
   uint32_t *sh = L.sh;
@@ -354,7 +366,7 @@ __device__ __forceinline__ void subproblems_body(SubLds<NT> &L, uint32_t *bin_st
       b[i] = 0;
       start[i] = c[i] = k[i] = wk[i] = 0u;
       if (q0 + i < nbins) {
-        b[i] = pencil_bin(q0 + i, nb);
+        b[i] = pencil_bin(q0 + i, nb, along_x);
         start[i] = bin_start[b[i]];
         c[i] = bin_start[b[i] + 1] - start[i];
         k[i] = (c[i] + ms - 1) / ms;
@@ -402,12 +414,12 @@ __device__ __forceinline__ void subproblems_body(SubLds<NT> &L, uint32_t *bin_st
 
 __global__ __launch_bounds__(kSubThreads) void subproblems_kernel(uint32_t *bin_start,
                                                                   const uint32_t *tot, int from_tot,
-                                                                  int nbins, int3 nb, int max_sub,
-                                                                  int sub_work, uint32_t *nsub,
+                                                                  int nbins, int3 nb, bool along_x,
+                                                                  int max_sub, int sub_work, uint32_t *nsub,
                                                                   int4 *subs) {
   __shared__ SubLds<kSubThreads> L;
-  subproblems_body<kSubThreads>(L, bin_start, tot, from_tot, nbins, nb, max_sub, sub_work, nsub,
-                                subs);
+  subproblems_body<kSubThreads>(L, bin_start, tot, from_tot, nbins, nb, along_x, max_sub, sub_work,
+                                nsub, subs);
 }
 
 // ---- one-pass binning (tile count <= kOneMaxBins) ---------------------------
@@ -427,6 +439,16 @@ __global__ __launch_bounds__(kSubThreads) void subproblems_kernel(uint32_t *bin_
 //                   chunk's offset + its wave's offset + its rank.
 // Ties keep input order, so the result equals the LSD passes' (and
 // numpy.argsort(keys, kind="stable")).
+
+// Largest |component| of the values, as bits (non-negative floats order like
+// their bit patterns): one atomic per wave that raises it.
+__device__ __forceinline__ void value_max(float mx, uint32_t *vmax) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  const uint32_t b = __float_as_uint(mx);
+  if ((threadIdx.x & 63) == 0 && b > __hip_atomic_load(vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(vmax, b);
+}
 
 // Peers of this lane (lanes of the wave with the same key among `valid`
 // lanes), from one ballot per key bit.
@@ -550,6 +572,7 @@ __global__ __launch_bounds__(kScanDigits * kChunkScanSegs) void chunk_scan_kerne
   const BinProblem &pr = bin_problem<BATCH, true>(one, table, nprob, blk);
   uint32_t *cnt = pr.cnt;
   const int nchunks = pr.nchunks, nbins = pr.nbins;
+  if (blk == 0 && threadIdx.x == 0 && pr.cls.ncls > 0) *pr.cls.vmax = 0u;
   const int dl = threadIdx.x & (kScanDigits - 1), sg = threadIdx.x / kScanDigits;
   const int d = (int)blk * kScanDigits + dl;
   const int per = (nchunks + kChunkScanSegs - 1) / kChunkScanSegs;
@@ -587,7 +610,7 @@ __global__ __launch_bounds__(kSubThreads) void subproblems_batched_kernel(const 
                               : make_int3(1, 1, 1);
   __shared__ SubLds<kSubThreads> L;
   subproblems_body<kSubThreads>(L, pr.bin_start, pr.pa.num_points > 0 ? pr.tot : nullptr, 1,
-                                pr.nbins, nb, pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
+                                pr.nbins, nb, pr.along_x, pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
 }
 
 // Fused list (one problem, one.fused): block 0 writes bin_start and the
@@ -615,7 +638,8 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
     const int3 nb = one.dim == 3 ? make_int3(one.g.nbin[0], one.g.nbin[1], one.g.nbin[2])
                                  : make_int3(1, 1, 1);
     subproblems_body<kOneThreads>(*(SubLds<kOneThreads> *)scatter_lds, one.bin_start, one.tot, 1,
-                                  one.nbins, nb, one.max_sub, one.sub_work, one.nsub, one.subs);
+                                  one.nbins, nb, one.along_x, one.max_sub, one.sub_work,
+                                  one.nsub, one.subs);
     return;
   }
   uint32_t chunk;
@@ -638,6 +662,13 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
     const bool valid = j < pa.num_points;
     load_point(pa, dim, j, valid, c[s]);
     val[s] = (REC && pr.values) ? pr.values[valid ? j : 0] : make_float2(0.f, 0.f);
+  }
+  if (REC && pr.values && pr.cls.ncls > 0) {
+    float mx = 0.f;
+#pragma unroll
+    for (int s = 0; s < kOneSteps; ++s)
+      if (j0 + 64 * s < pa.num_points) mx = fmaxf(mx, fmaxf(fabsf(val[s].x), fabsf(val[s].y)));
+    value_max(mx, pr.cls.vmax);
   }
   // fused: this thread's run of tile totals (clamped indices, no branch)
   const int per = (nbins + kOneThreads - 1) / kOneThreads;
@@ -716,7 +747,125 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
   }
 }
 
-constexpr int kBinTableChunk = 12;  // descriptors per table-fill launch (kernarg size)
+// ---- class list of the matrix-core kernels ----------------------------------
+// Their 16-row windows take the points of one y-offset class of a tile, and a
+// window slides along y from class to class.  The tile binning stays coarse
+// (its per-chunk counts grow with the tile count, and classes as tiles of
+// their own would be 3 to 16 times as many), and the classes are listed inside
+// each subproblem of the tile list: one block per subproblem (at most
+// kClassSub points) ranks every point among those of its class and x offset
+// (stable) and writes the sorted positions in that order (perm) and the
+// classes' starts.  The x order lets the kernels leave out the x cells no
+// point of a group reaches.
+constexpr int kClsThreads = 256;
+constexpr int kClsWaves = kClsThreads / 64;
+constexpr int kClsSteps = kClassSub / kClsThreads;
+constexpr int kClsKeys = 256;  // (class, x offset) pairs at most
+
+// The problem of this block: the one passed by value (no table), or the last
+// table entry whose first block is at most blockIdx.x.
+__device__ __forceinline__ const BinProblem &piece_problem(const BinProblem &one,
+                                                            const BinProblem *table, int nprob,
+                                                            uint32_t &local) {
+  local = blockIdx.x;
+  if (!table) return one;
+  int lo = 0, hi = nprob - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (table[mid].piece0 <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  local = blockIdx.x - table[lo].piece0;
+  return table[lo];
+}
+
+__global__ __launch_bounds__(kClsThreads) void class_sort_kernel(BinProblem one,
+                                                                 const BinProblem *table,
+                                                                 int nprob) {
+  __shared__ uint32_t cnt[kClsWaves][kClsKeys];  // per wave: points of each key, then their places
+  __shared__ uint32_t sh[kClsWaves];
+  uint32_t piece;
+  const BinProblem &pr = piece_problem(one, table, nprob, piece);
+  if (piece >= pr.nsub[0]) return;
+  const ClassBuffers &cb = pr.cls;
+  const int ncls = cb.ncls, binx = pr.g.bin[0], nkeys = ncls * binx, bits = cb.bits;
+  const int4 sub = pr.subs[piece];
+  const int n = sub.z;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  // each wave ranks one contiguous run of `steps` x 64 points
+  const int steps = (n + kClsThreads - 1) / kClsThreads;
+  const float *ofs = (const float *)pr.out.r + 8 * (int64_t)sub.y + 3;  // point p's offsets: ofs[8 p]
+  const int p0 = wave * steps * 64 + lane;
+  const float inv_cw = 1.0f / (float)cb.cw;
+  int o[kClsSteps];
+#pragma unroll
+  for (int s = 0; s < kClsSteps; ++s) {
+    const int p = p0 + 64 * s;
+    o[s] = s < steps && p < n ? __float_as_int(ofs[8 * (int64_t)p]) : -1;
+  }
+#pragma unroll
+  for (int w = 0; w < kClsWaves; ++w) cnt[w][threadIdx.x] = 0u;
+  __syncthreads();
+  uint32_t *row = cnt[wave];
+  uint32_t rk[kClsSteps];
+#pragma unroll
+  for (int s = 0; s < kClsSteps; ++s) {
+    if (s >= steps) break;
+    const bool valid = o[s] >= 0;
+    // class (o1 - 1) / cw of the y offset o1 >= 1 (cell_div's rounding argument)
+    const int c = (int)(((float)((o[s] >> 8) & 255) - 0.5f) * inv_cw);
+    const uint32_t k = valid ? (uint32_t)(c * binx + (o[s] & 255)) : 0u;
+    const uint64_t peers = key_peers(k, valid, bits);
+    const uint64_t below = peers & lt;
+    uint32_t b0 = 0;
+    if (valid && below == 0ull) {  // the first lane of each key claims the step's places
+      b0 = row[k];
+      row[k] = b0 + (uint32_t)__popcll(peers);
+    }
+    const int leader = valid ? __ffsll((unsigned long long)peers) - 1 : lane;
+    rk[s] = __shfl(b0, leader) + (uint32_t)__popcll(below);
+    o[s] = valid ? (int)k : -1;
+  }
+  __syncthreads();
+  {
+    // first place of each key, then of each wave's points of it
+    const int k = threadIdx.x;
+    uint32_t c[kClsWaves], tot = 0, all;
+#pragma unroll
+    for (int w = 0; w < kClsWaves; ++w) {
+      c[w] = cnt[w][k];
+      tot += c[w];
+    }
+    uint32_t at = block_scan_waves<kClsThreads>(tot, sh, all);
+    if (k < nkeys && k % binx == 0) cb.start[(int64_t)piece * ncls + k / binx] = (uint16_t)at;
+#pragma unroll
+    for (int w = 0; w < kClsWaves; ++w) {
+      cnt[w][k] = at;
+      at += c[w];
+    }
+  }
+  __syncthreads();
+  uint32_t *perm = cb.perm + (int64_t)sub.y;
+#pragma unroll
+  for (int s = 0; s < kClsSteps; ++s) {
+    if (s >= steps) break;
+    if (o[s] >= 0) perm[row[o[s]] + rk[s]] = (uint32_t)sub.y + (uint32_t)(p0 + 64 * s);
+  }
+}
+
+// Subproblems of a list at most.
+int class_pieces(int64_t n, int nbins, int max_sub) {
+  return (int)(std::min<int64_t>(nbins, n) + (n + max_sub - 1) / max_sub);
+}
+// The class list of one problem.
+void launch_class_sort(const BinProblem &pr, int64_t n, int nbins, int max_sub, hipStream_t s) {
+  hipLaunchKernelGGL(class_sort_kernel, dim3(class_pieces(n, nbins, max_sub)), dim3(kClsThreads), 0, s, pr,
+                     (const BinProblem *)nullptr, 1);
+}
+
+// descriptors per table-fill launch (kernarg size)
+constexpr int kBinTableChunk = 8;
 struct BinTableChunk {
   int first, count;
   BinProblem probs[kBinTableChunk];
@@ -745,11 +894,13 @@ hipError_t set_scatter_lds(bool rec, bool batch, size_t lds) {
 
 bool sort_one_pass(int nbins) { return nbins <= kOneMaxBins; }
 
-size_t sort_count_entries(int64_t num_points, int nbins) {
+size_t radix_count_entries(int64_t num_points) {
   const int64_t M = std::max<int64_t>(num_points, 1);
-  const int64_t old_n = (int64_t)kRadix * ((M + kSortChunk - 1) / kSortChunk);
-  const int64_t one_n = sort_one_pass(nbins) ? (int64_t)nbins * ((M + kOneChunk - 1) / kOneChunk) : 0;
-  return (size_t)std::max(old_n, one_n);
+  return (size_t)(kRadix * ((M + kSortChunk - 1) / kSortChunk));
+}
+size_t one_pass_count_entries(int64_t num_points, int nbins) {
+  const int64_t M = std::max<int64_t>(num_points, 1);
+  return sort_one_pass(nbins) ? (size_t)nbins * (size_t)((M + kOneChunk - 1) / kOneChunk) : 0;
 }
 
 // One-pass binning: see the comment above chunk_count_kernel.
@@ -778,6 +929,8 @@ static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int d
   pr.bits = key_bits(nbins);
   pr.max_sub = sb.max_sub;
   pr.sub_work = sb.sub_work;
+  pr.along_x = sb.along_x;
+  if (rec) pr.cls = sb.cls;
   pr.nchunks = (int)((n + kOneChunk - 1) / kOneChunk);
   const int nch = pr.nchunks;
   // with the tile starts in LDS beside the count rows, the scatter launch
@@ -794,7 +947,7 @@ static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int d
     const int3 nb = dim == 3 ? make_int3(g.nbin[0], g.nbin[1], g.nbin[2]) : make_int3(1, 1, 1);
     hipLaunchKernelGGL(subproblems_kernel, dim3(1), dim3(kSubThreads), 0, s, sb.bin_start,
                        n > 0 ? (const uint32_t *)sb.scan_tmp : (const uint32_t *)nullptr, 1,
-                       sb.nbins, nb, sb.max_sub, sb.sub_work, sb.sub_ofs + sb.nbins, sb.subs);
+                       sb.nbins, nb, sb.along_x, sb.max_sub, sb.sub_work, sb.sub_ofs + sb.nbins, sb.subs);
   }
   if (n > 0) {
     size_t lds = sizeof(uint16_t) * (size_t)kOneWaves * nbins;
@@ -808,13 +961,14 @@ static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int d
     else
       hipLaunchKernelGGL((chunk_scatter_kernel<false, false>), dim3(blocks), dim3(kOneThreads),
                          lds, s, pr, (const BinProblem *)nullptr, 1);
+    if (pr.cls.ncls > 0) launch_class_sort(pr, n, nbins, sb.max_sub, s);
   }
   return hipGetLastError();
 }
 
 hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, hipStream_t s) {
   if (nprob <= 0) return hipSuccess;
-  uint32_t chunks = 0, scans = 0;
+  uint32_t chunks = 0, scans = 0, pieces = 0;
   int max_bins = 1;
   bool rec = probs[0].out.r != nullptr;
   for (int i = 0; i < nprob; ++i) {
@@ -824,6 +978,9 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
     pr.nchunks = (int)((pr.pa.num_points + kOneChunk - 1) / kOneChunk);
     pr.chunk0 = chunks;
     pr.scan0 = scans;
+    pr.piece0 = pieces;
+    if (pr.cls.ncls > 0)
+      pieces += (uint32_t)class_pieces(pr.pa.num_points, pr.nbins, pr.max_sub);
     chunks += (uint32_t)pr.nchunks;
     if (pr.pa.num_points > 0) scans += (uint32_t)((pr.nbins + kScanDigits - 1) / kScanDigits);
     max_bins = std::max(max_bins, pr.nbins);
@@ -856,6 +1013,9 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
       hipLaunchKernelGGL((chunk_scatter_kernel<false, true>), dim3(chunks), dim3(kOneThreads), lds,
                          s, none, (const BinProblem *)table, nprob);
   }
+  if (pieces > 0)
+    hipLaunchKernelGGL(class_sort_kernel, dim3(pieces), dim3(kClsThreads), 0, s, none,
+                       (const BinProblem *)table, nprob);
   return hipGetLastError();
 }
 
@@ -867,7 +1027,7 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
   auto dst = [&](int q) { return ((sb.passes - 1 - q) & 1) == 0 ? rec->out : rec->tmp; };
   if (n > 0) {
     hipLaunchKernelGGL(keys_kernel, dim3(sb.nchunks), dim3(kSortThreads), 0, s, pa, g, dim,
-                       sb.keys[0], sb.cnt, sb.nchunks);
+                       sb.keys[0], sb.cnt, sb.nchunks, sb.cls.ncls > 0 ? sb.cls.vmax : nullptr);
     for (int p = 0; p < sb.passes; ++p) {
       if (p > 0) {
         const KeySrc ks{sb.keys[p & 1], rec ? dst(p - 1).r : nullptr};
@@ -884,6 +1044,7 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
         rm.pa = pa;
         rm.g = g;
         rm.first = p == 0;
+        rm.vmax = p == 0 && rec->values && sb.cls.ncls > 0 ? sb.cls.vmax : nullptr;
         hipLaunchKernelGGL(scatter_kernel<true>, dim3(sb.nchunks), dim3(kSortThreads), 0, s,
                            sb.keys[0], (const uint32_t *)nullptr, (uint32_t *)nullptr,
                            (uint32_t *)nullptr, n, p * kRadixBits, sb.cnt, sb.scan_tmp,
@@ -902,8 +1063,17 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
   hipLaunchKernelGGL(bounds_kernel, dim3((nb1 + 255) / 256), dim3(256), 0, s, sorted, n,
                      sb.bin_start, sb.nbins);
   hipLaunchKernelGGL(subproblems_kernel, dim3(1), dim3(kSubThreads), 0, s, sb.bin_start,
-                     (const uint32_t *)nullptr, 0, sb.nbins, nb, sb.max_sub, sb.sub_work,
+                     (const uint32_t *)nullptr, 0, sb.nbins, nb, sb.along_x, sb.max_sub, sb.sub_work,
                      sb.sub_ofs + sb.nbins, sb.subs);
+  if (n > 0 && rec && sb.cls.ncls > 0) {
+    BinProblem pr{};
+    pr.g = g;
+    pr.out = rec->out;
+    pr.nsub = sb.sub_ofs + sb.nbins;
+    pr.subs = sb.subs;
+    pr.cls = sb.cls;
+    launch_class_sort(pr, n, sb.nbins, sb.max_sub, s);
+  }
   return hipGetLastError();
 }
 
