@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libapollo_nufft_hip.so")
 ARCH = os.environ.get("APOLLO_NUFFT_ARCH", "gfx950")
 
 SOURCES = ["plan.cpp", "autotune.cpp", "sort.hip", "fft.hip", "spread.hip", "window.hip", "block_spread.hip",
-           "direct.hip"]
+           "points1d.hip", "direct.hip"]
 
 # -packed-fp32-ops: the compiler must not form packed FP32 instructions.
 COMMON = [

@@ -22,7 +22,6 @@
 namespace anufft {
 namespace {
 
-constexpr int kFftThreads = 256;
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -109,12 +108,12 @@ __device__ __forceinline__ void small_dft<5>(float2 *v, const float2 *tw, int L)
 // Stockham radix-R stage (decimation in time, autosorting):
 //   j in [0, L/R), k = j mod Ns, v_r = src[j + r L/R] * W_{Ns R}^{k r},
 //   dst[(j - k) R + k + u Ns] = DFT_R(v)_u.
-template <int R>
+template <int R, int NT>
 __device__ __forceinline__ void stage(const float2 *src, float2 *dst, int L, int Ns,
                                       const float2 *tw, int lines, uint32_t mag_nbf,
                                       uint32_t mag_ns, int twstep) {
   const int nbf = L / R;
-  for (int it = threadIdx.x; it < lines * nbf; it += kFftThreads) {
+  for (int it = threadIdx.x; it < lines * nbf; it += NT) {
     const int li = fdiv(it, nbf, mag_nbf);
     const int j = it - li * nbf;
     const int k = j - fdiv(j, Ns, mag_ns) * Ns;
@@ -136,11 +135,12 @@ __device__ __forceinline__ void stage(const float2 *src, float2 *dst, int L, int
 // Any radix (primes above 5): one thread per output element.  With
 // W_R = W_L^(L/R), the twiddle of input r is W_L^(r (k twstep + u L/R)), so
 // its exponent advances by a fixed step modulo L.
+template <int NT>
 __device__ void stage_generic(const float2 *src, float2 *dst, int L, int Ns, int R,
                               const float2 *tw, int lines) {
   const int nbf = L / R;
   const int twstep = L / (Ns * R);
-  for (int it = threadIdx.x; it < lines * L; it += kFftThreads) {
+  for (int it = threadIdx.x; it < lines * L; it += NT) {
     int li = it / L;
     int o = it - li * L;
     int k = o % Ns;
@@ -167,6 +167,7 @@ __device__ __forceinline__ int kept_pos(int i, int nk, int L) {
 
 // All Stockham stages of one length-Lf transform of nl lines, ping-ponging
 // between *src and *dst (the result ends in *src).
+template <int NT>
 __device__ __forceinline__ void run_stages(const FftPass &p, int Lf, const float2 *tw, int nl,
                                            float2 *&src, float2 *&dst) {
   int Ns = 1;
@@ -176,12 +177,12 @@ __device__ __forceinline__ void run_stages(const FftPass &p, int Lf, const float
     const uint32_t mb = p.mag_nbf[f], ms = p.mag_ns[f];
     const int ts = p.twstep[f];
     switch (R) {
-    case 2: stage<2>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
-    case 3: stage<3>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
-    case 4: stage<4>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
-    case 5: stage<5>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
-    case 8: stage<8>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
-    default: stage_generic(src, dst, Lf, Ns, R, tw, nl); break;
+    case 2: stage<2, NT>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
+    case 3: stage<3, NT>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
+    case 4: stage<4, NT>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
+    case 5: stage<5, NT>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
+    case 8: stage<8, NT>(src, dst, Lf, Ns, tw, nl, mb, ms, ts); break;
+    default: stage_generic<NT>(src, dst, Lf, Ns, R, tw, nl); break;
     }
     float2 *t = src;
     src = dst;
@@ -210,18 +211,18 @@ __device__ __forceinline__ int2 line_index(int idx, bool contig, int n, uint32_t
 
 // Input lines into LDS: deconvolution (DEC), conjugation for the inverse,
 // the Bluestein chirp, kept modes at their FFT positions.
-template <bool DEC>
+template <bool DEC, int NT>
 __device__ __forceinline__ void load_lines(const FftPass &p, const int64_t *lbase, int nl,
                                            uint32_t mag_nl, int Lf, bool blue, float2 *buf0) {
   const bool contig = p.in_si == 1;
   const int n = nl * p.nin;
-  for (int base = threadIdx.x; base < n; base += kFftThreads * kLoadBatch) {
+  for (int base = threadIdx.x; base < n; base += NT * kLoadBatch) {
     float2 v[kLoadBatch];
     double f[kLoadBatch];
     int2 e[kLoadBatch];  // (line, index)
 #pragma unroll
     for (int r = 0; r < kLoadBatch; ++r) {
-      const int idx = base + r * kFftThreads;
+      const int idx = base + r * NT;
       e[r] = line_index(idx < n ? idx : 0, contig, p.nin, p.mag_nin, nl, mag_nl);
       v[r] = p.in[lbase[e[r].x] + (int64_t)e[r].y * p.in_si];
       f[r] = DEC ? p.dec_in[e[r].y] : 1.0;
@@ -237,31 +238,31 @@ __device__ __forceinline__ void load_lines(const FftPass &p, const int64_t *lbas
       if (p.inverse) x.y = -x.y;
       const int pos = kept_pos(e[r].y, p.nin, p.L);
       if (blue) x = cmul(x, p.chirp[pos]);
-      if (base + r * kFftThreads < n) buf0[e[r].x * Lf + pos] = x;
+      if (base + r * NT < n) buf0[e[r].x * Lf + pos] = x;
     }
   }
 }
 
 // LDS lines to the output: kept modes, Bluestein chirp, conjugation for the
 // inverse, scale and deconvolution (DEC), and the bin maxima (bm != null).
-template <bool DEC>
+template <bool DEC, int NT>
 __device__ __forceinline__ void store_lines(const FftPass &p, const int64_t *lbase, int nl,
                                             uint32_t mag_nl, int Lf, bool blue, const float2 *src,
                                             uint32_t *bm, int nbz) {
   const bool contig = p.out_si == 1;
   const int n = nl * p.nout;
-  for (int base = threadIdx.x; base < n; base += kFftThreads * kLoadBatch) {
+  for (int base = threadIdx.x; base < n; base += NT * kLoadBatch) {
     double f[kLoadBatch];
     int2 e[kLoadBatch];  // (line, output index)
 #pragma unroll
     for (int r = 0; r < kLoadBatch; ++r) {
-      const int idx = base + r * kFftThreads;
+      const int idx = base + r * NT;
       e[r] = line_index(idx < n ? idx : 0, contig, p.nout, p.mag_nout, nl, mag_nl);
       f[r] = DEC ? p.dec_out[e[r].y] : 1.0;
     }
 #pragma unroll
     for (int r = 0; r < kLoadBatch; ++r) {
-      if (base + r * kFftThreads >= n) continue;
+      if (base + r * NT >= n) continue;
       const int li = e[r].x, o = e[r].y;
       const int pos = kept_pos(o, p.nout, p.L);
       float2 v = src[li * Lf + pos];
@@ -278,7 +279,8 @@ __device__ __forceinline__ void store_lines(const FftPass &p, const int64_t *lba
   }
 }
 
-__global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(FftPass p) {
+template <int NT>
+__global__ __launch_bounds__(NT) void fft_pass_kernel(FftPass p) {
   extern __shared__ float2 sh[];
   const int L = p.L, lb = p.lb;
   const bool blue = p.blue_n > 0;
@@ -287,18 +289,18 @@ __global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(FftPass p) {
   float2 *buf1 = sh + (size_t)lb * Lf;
   float2 *tw = sh + 2 * (size_t)lb * Lf;  // twiddle table of length Lf
   int64_t *lbase = (int64_t *)(tw + Lf);  // [lb] input, [lb] output line offsets
-  // the first 2 x kFftThreads twiddles: loaded now, stored to LDS after the
+  // the first 2 NT twiddles: loaded now, stored to LDS after the
   // input lines (their latency overlaps the line set-up and loads)
   const float2 tw0 = p.tw[min((int)threadIdx.x, Lf - 1)];
-  const float2 tw1 = p.tw[min((int)threadIdx.x + kFftThreads, Lf - 1)];
+  const float2 tw1 = p.tw[min((int)threadIdx.x + NT, Lf - 1)];
   if (p.zero)
-    for (int i = blockIdx.x * kFftThreads + threadIdx.x; i < p.zero_n; i += gridDim.x * kFftThreads)
+    for (int i = blockIdx.x * NT + threadIdx.x; i < p.zero_n; i += gridDim.x * NT)
       p.zero[i] = 0.f;
   const int64_t l0 = (int64_t)blockIdx.x * lb;
   const int nl = (int)((p.nlines - l0) < lb ? (p.nlines - l0) : lb);
   const uint32_t mag_nl = nl == lb ? p.mag_lb : p.mag_last;  // nl < lb only in the last block
   // element offsets of the block's lines, one 64-bit division per line
-  for (int li = threadIdx.x; li < nl; li += kFftThreads) {
+  for (int li = threadIdx.x; li < nl; li += NT) {
     const int64_t l = l0 + li;
     const int64_t a = p.use_mag_nb ? (int64_t)fdiv((int)l, (int)p.nb, p.mag_nb) : l / p.nb;
     const int64_t b = l - a * p.nb;
@@ -309,18 +311,18 @@ __global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(FftPass p) {
 
   if (blue) {
     // a_n = x_n chirp_n on [0, L), zero on [L, Lf): clear everything first
-    for (int idx = threadIdx.x; idx < nl * Lf; idx += kFftThreads) buf0[idx] = make_float2(0.f, 0.f);
+    for (int idx = threadIdx.x; idx < nl * Lf; idx += NT) buf0[idx] = make_float2(0.f, 0.f);
     __syncthreads();
   }
   // ---- load (with deconvolution, conjugation for the inverse, zero pad) ----
-  if (p.dec_in) load_lines<true>(p, lbase, nl, mag_nl, Lf, blue, buf0);
-  else load_lines<false>(p, lbase, nl, mag_nl, Lf, blue, buf0);
+  if (p.dec_in) load_lines<true, NT>(p, lbase, nl, mag_nl, Lf, blue, buf0);
+  else load_lines<false, NT>(p, lbase, nl, mag_nl, Lf, blue, buf0);
   if ((int)threadIdx.x < Lf) tw[threadIdx.x] = tw0;
-  if ((int)threadIdx.x + kFftThreads < Lf) tw[threadIdx.x + kFftThreads] = tw1;
-  for (int i = threadIdx.x + 2 * kFftThreads; i < Lf; i += kFftThreads) tw[i] = p.tw[i];
+  if ((int)threadIdx.x + NT < Lf) tw[threadIdx.x + NT] = tw1;
+  for (int i = threadIdx.x + 2 * NT; i < Lf; i += NT) tw[i] = p.tw[i];
   if (!blue && p.nin < L) {
     const int gap = L - p.nin, g0 = p.nin / 2 + 1;
-    for (int idx = threadIdx.x; idx < nl * gap; idx += kFftThreads) {
+    for (int idx = threadIdx.x; idx < nl * gap; idx += NT) {
       int li = idx / gap;
       buf0[li * L + g0 + (idx - li * gap)] = make_float2(0.f, 0.f);
     }
@@ -328,15 +330,15 @@ __global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(FftPass p) {
 
   // ---- Stockham stages in LDS ----
   float2 *src = buf0, *dst = buf1;
-  run_stages(p, Lf, tw, nl, src, dst);
+  run_stages<NT>(p, Lf, tw, nl, src, dst);
   if (blue) {
     // C = FFT(a) FFT(b) / Lf; the inverse FFT of C is conj(FFT(conj(C)))
     __syncthreads();
-    for (int idx = threadIdx.x; idx < nl * Lf; idx += kFftThreads) {
+    for (int idx = threadIdx.x; idx < nl * Lf; idx += NT) {
       const float2 c = cmul(src[idx], p.bhat[idx & (Lf - 1)]);  // Lf: a power of two
       src[idx] = make_float2(c.x, -c.y);
     }
-    run_stages(p, Lf, tw, nl, src, dst);
+    run_stages<NT>(p, Lf, tw, nl, src, dst);
   }
   __syncthreads();
 
@@ -347,15 +349,15 @@ __global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(FftPass p) {
   uint32_t *bm = (uint32_t *)dst;
   const int nbz = p.bmax ? p.bm_nbin[2] : 0;
   if (p.bmax) {
-    for (int i = threadIdx.x; i < nl * nbz; i += kFftThreads) bm[i] = 0u;
+    for (int i = threadIdx.x; i < nl * nbz; i += NT) bm[i] = 0u;
     __syncthreads();
   }
   uint32_t *bmx = p.bmax ? bm : nullptr;
-  if (p.dec_out) store_lines<true>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
-  else store_lines<false>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
+  if (p.dec_out) store_lines<true, NT>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
+  else store_lines<false, NT>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
   if (p.bmax) {
     __syncthreads();
-    for (int i = threadIdx.x; i < nl * nbz; i += kFftThreads) {
+    for (int i = threadIdx.x; i < nl * nbz; i += NT) {
       const int li = i / nbz, zb = i - li * nbz;
       const int64_t l = l0 + li, x = l / p.nb, y = l - x * p.nb;
       const int64_t bin = ((x / p.bm_bin[0]) * p.bm_nbin[1] + y / p.bm_bin[1]) * p.bm_nbin[2] + zb;
@@ -408,12 +410,19 @@ hipError_t launch_fft_pass(const FftPass &pass, hipStream_t s) {
   int64_t blocks = (p.nlines + p.lb - 1) / p.lb;
   const int Lf = p.blue_n > 0 ? p.blue_n : p.L;
   size_t lds = (2 * (size_t)p.lb + 1) * Lf * sizeof(float2) + 2 * (size_t)p.lb * sizeof(int64_t);
+  // 256 threads for the usual 1024 points of a block, 1024 from 2048 points
+  // on: a single long line is a chain of stages and loads on one CU (one
+  // line of 4096 points, Bluestein: 62 us at 256 threads in a stage by itself, 32 at 1024).
+  const bool wide = (int64_t)p.lb * Lf >= 2048;
+  const void *fn = wide ? (const void *)fft_pass_kernel<1024> : (const void *)fft_pass_kernel<256>;
   if (lds > 65536) {
-    hipError_t e = hipFuncSetAttribute((const void *)fft_pass_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(fft_pass_kernel, dim3((unsigned)blocks), dim3(kFftThreads), lds, s, p);
+  if (wide)
+    hipLaunchKernelGGL(fft_pass_kernel<1024>, dim3((unsigned)blocks), dim3(1024), lds, s, p);
+  else
+    hipLaunchKernelGGL(fft_pass_kernel<256>, dim3((unsigned)blocks), dim3(256), lds, s, p);
   return hipGetLastError();
 }
 

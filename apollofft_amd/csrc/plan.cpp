@@ -298,8 +298,6 @@ Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
     for (int i = 0; i < kinds; ++i) nsub = std::max<int64_t>(nsub, all[i]->list_len(M) + 1);
     l.subs = take(16 * (size_t)nsub);
     if (p->dim == 1) {
-      l.zrec = take(32 * Mp);   // point records of the 1D binning
-      l.zrec2 = take(32 * Mp);
       l.grid = take(8 * (size_t)p->m[0]);
       l.total = off;
       return l;
@@ -535,8 +533,8 @@ void set_geom(anufft_plan::Binning &b, const anufft_plan *p, const int bin[3]) {
 
 void choose_bins(anufft_plan *p) {
   if (p->dim == 1) {
-    // tiles of one wave (64 cells with their taps); subproblems of at most
-    // 1024 points (one workgroup walks a subproblem 64 points at a time)
+    // tiles of 64 cells with their taps, for the binning of anufft_debug_sort
+    // (the 1D kernels take the points in input order)
     const int b[3] = {bin1d(p->w), 1, 1};
     set_geom(p->bs, p, b);
     p->bs.max_sub = p->opts.max_subproblem > 0 ? p->opts.max_subproblem : 1024;
@@ -792,6 +790,11 @@ struct Exec {
                                  blocks(p->bs, pa.num_points, win_spread_groups(p->w, pa.num_points, p->cus)), s);
       return launch_spread3d(p->w, pa, rec(), xo(), grid, p->bs.g, p->poly,
                              blocks(p->bs, pa.num_points, 2), s);
+    });
+  }
+  hipError_t spread1(const PointArgs &pa, const float2 *values, float2 *grid) const {
+    return timed(ANUFFT_STAGE_SPREAD, [&] {
+      return launch_spread1d(p->w, pa, values, grid, p->bs.g, p->poly, p->cus, s);
     });
   }
   hipError_t spread_blocks(const PointArgs &pa, float2 *grid) const {
@@ -1195,9 +1198,14 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
   Exec ex{p, stream, (char *)ws, lay};
   const anufft_plan::Binning &bs = blocks ? p->bf : p->bs;
   hipError_t e = hipSuccess;
-  if (M > 0) {
+  if (M > 0 && p->dim == 1) {
+    e = ex.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ex.grid(), p->cells(), ex.s); });
+    if (e != hipSuccess) return hip_fail(e, "fill");
+    e = ex.spread1(ex.point_args(bs, M, coords, stride), (const float2 *)values, ex.grid());
+    if (e != hipSuccess) return hip_fail(e, "spread");
+  } else if (M > 0) {
     PointArgs pa = ex.point_args(bs, M, coords, stride);
-    const bool records = p->dim == 1 || p->kernel_method == kSpreadMfma;
+    const bool records = p->kernel_method == kSpreadMfma;
     // zeroing the grid (second stream) is independent of the binning
     e = ex.fork_join(
         [&](const Exec &ea) {
@@ -1205,15 +1213,7 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
         },
         [&] { return ex.bin(bs, pa, (const float2 *)values, records); });
     if (e != hipSuccess) return hip_fail(e, "fill / binning");
-    if (p->dim == 3) {
-      e = blocks ? ex.spread_blocks(pa, ex.grid())
-                 : ex.spread3(pa, (const float2 *)values, ex.grid());
-    } else {
-      e = ex.timed(ANUFFT_STAGE_SPREAD, [&] {
-        return launch_spread1d(p->w, pa, ex.zrec(M), ex.grid(), p->bs.g, p->poly,
-                               ex.blocks(p->bs, M, 8), ex.s);
-      });
-    }
+    e = blocks ? ex.spread_blocks(pa, ex.grid()) : ex.spread3(pa, (const float2 *)values, ex.grid());
     if (e != hipSuccess) return hip_fail(e, "spread");
   } else {
     e = ex.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ex.grid(), p->cells(), ex.s); });
@@ -1283,16 +1283,11 @@ anufft_status anufft_execute_type2(const anufft_plan *p, int64_t M, const float 
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
     e = ex.interp3(pa, ex, (float2 *)out);
   } else {
-    PointArgs pa = ex.point_args(p->bi, M, coords, stride);
-    e = ex.fork_join(
-        [&](const Exec &ea) {
-          return ea.timed(ANUFFT_STAGE_FFT, [&] { return ea.modes_to_grid((const float2 *)modes, false); });
-        },
-        [&] { return ex.bin(p->bi, pa, nullptr, true); });
-    if (e != hipSuccess) return hip_fail(e, "fft / binning");
+    e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.modes_to_grid((const float2 *)modes, false); });
+    if (e != hipSuccess) return hip_fail(e, "fft");
     e = ex.timed(ANUFFT_STAGE_INTERP, [&] {
-      return launch_interp1d(p->w, pa, ex.zrec(M), ex.grid(), (float2 *)out, nullptr, p->bi.g,
-                             p->poly, ex.blocks(p->bi, M, 8), ex.s);
+      return launch_interp1d(p->w, ex.point_args(p->bi, M, coords, stride), ex.grid(), nullptr,
+                             (float2 *)out, nullptr, p->bi.g, p->poly, p->cus, ex.s);
     });
   }
   if (e != hipSuccess) return hip_fail(e, "interp");
@@ -1323,17 +1318,11 @@ anufft_status anufft_execute_grad_points(const anufft_plan *p, int64_t M,
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
     e = ex.grad3(pa, ex, (const float2 *)u, grad);
   } else {
-    // records carry u (value fields): the gradient reads it in sorted order
-    PointArgs pa = ex.point_args(p->bg, M, coords, stride);
-    e = ex.fork_join(
-        [&](const Exec &ea) {
-          return ea.timed(ANUFFT_STAGE_FFT, [&] { return ea.modes_to_grid((const float2 *)modes_h, false); });
-        },
-        [&] { return ex.bin(p->bg, pa, (const float2 *)u, true); });
-    if (e != hipSuccess) return hip_fail(e, "fft / binning");
+    e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.modes_to_grid((const float2 *)modes_h, false); });
+    if (e != hipSuccess) return hip_fail(e, "fft");
     e = ex.timed(ANUFFT_STAGE_GRAD, [&] {
-      return launch_interp1d(p->w, pa, ex.zrec(M), ex.grid(), nullptr, grad[0], p->bg.g, p->poly,
-                             ex.blocks(p->bg, M, 8), ex.s);
+      return launch_interp1d(p->w, ex.point_args(p->bg, M, coords, stride), ex.grid(),
+                             (const float2 *)u, nullptr, grad[0], p->bg.g, p->poly, p->cus, ex.s);
     });
   }
   if (e != hipSuccess) return hip_fail(e, "grad");
@@ -1525,13 +1514,13 @@ anufft_status anufft_debug_spread(const anufft_plan *p, int64_t M, const float *
   if (e != hipSuccess) return hip_fail(e, "fill");
   if (M == 0) return ANUFFT_OK;
   PointArgs pa = ex.point_args(p->bs, M, coords, stride);
-  e = ex.bin(p->bs, pa, (const float2 *)values, p->dim == 1 || p->kernel_method == kSpreadMfma);
-  if (e != hipSuccess) return hip_fail(e, "binning");
-  if (p->dim == 3)
+  if (p->dim == 3) {
+    e = ex.bin(p->bs, pa, (const float2 *)values, p->kernel_method == kSpreadMfma);
+    if (e != hipSuccess) return hip_fail(e, "binning");
     e = ex.spread3(pa, (const float2 *)values, (float2 *)grid);
-  else
-    e = launch_spread1d(p->w, pa, ex.zrec(M), (float2 *)grid, p->bs.g, p->poly,
-                        ex.blocks(p->bs, M, 8), ex.s);
+  } else {
+    e = ex.spread1(pa, (const float2 *)values, (float2 *)grid);
+  }
   if (e != hipSuccess) return hip_fail(e, "spread");
   return ANUFFT_OK;
 }
