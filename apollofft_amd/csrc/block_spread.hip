@@ -130,14 +130,14 @@ template <int NW>
 __device__ __forceinline__ int block_strength_exp(const ZRec &zr, int4 sub, float *red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int NT = 64 * NW, B = 4;  // B values per thread loaded before any is used
-  const float2 *vals = (const float2 *)zr.r + 4 * (int64_t)sub.y + 2;  // point p's value: vals[4 p]
+  const float2 *vals = zr.v + sub.y;
   float mx = 0.f;
   for (int p0 = threadIdx.x; p0 < sub.z; p0 += NT * B) {
     float2 c[B];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       const int p = p0 + u * NT;
-      c[u] = vals[4 * (int64_t)(p < sub.z ? p : 0)];
+      c[u] = vals[p < sub.z ? p : 0];
     }
 #pragma unroll
     for (int u = 0; u < B; ++u)
@@ -192,8 +192,8 @@ __device__ __forceinline__ void block_accumulate(f32x16 (&acc)[BSpread<W>::XW][2
 #pragma unroll
       for (int zz = 0; zz < 32; ++zz) WZ[p * kMWZ + zz] = 0.f;
       const bool ok = p < npts;
-      const float4 z = ok ? zr.r[2 * (int64_t)(start + p)] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float4 c = ok ? zr.r[2 * (int64_t)(start + p) + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 z = ok ? zr.r[start + p] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float2 c = ok ? zr.v[start + p] : make_float2(0.f, 0.f);
       ZS[p] = z.x;
       ZS[kMNP + p] = z.y;
       ZS[2 * kMNP + p] = z.z;

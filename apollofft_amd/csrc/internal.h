@@ -32,6 +32,7 @@ constexpr int kOneWaves = 8;
 constexpr int kOneThreads = 64 * kOneWaves;
 constexpr int kOneSteps = 8;
 constexpr int kOneChunk = kOneThreads * kOneSteps;
+constexpr int kTileMaxBins = 16384;  // tile binning: 64 KiB of LDS counts
 constexpr int kOneMaxBins = 9216;   // kOneWaves rows of 16-bit counts: 144 KiB of LDS
 constexpr int kSpreadBinX = 4;      // spreading tile x-extent (a lane holds bin_x + 2w - 1 cells)
 constexpr int kSpreadCols = 32;     // spreading tile (y,z) columns per axis, bin + 2w <= 32
@@ -104,7 +105,6 @@ constexpr int kClassSub = 4096;  // points of a tile listed by class at once
 struct ClassBuffers {
   int ncls = 0;      // 0: no class list
   int cw = 1;
-  int bits = 0;      // bits of a (class, x offset) key
   uint32_t *perm;    // list order -> sorted position: a subproblem's points by class and x offset
   uint16_t *start;   // per subproblem: first entry of each class in its part of the list
   uint32_t *vmax;    // bits of the largest |re|, |im| of the values
@@ -114,7 +114,7 @@ struct SortBuffers {
   uint32_t *keys[2];
   uint32_t *idx[2];
   uint32_t *cnt;       // per-chunk digit (one-pass: tile) counts, then offsets
-  uint32_t *scan_tmp;  // digit (one-pass: tile) totals
+  uint32_t *scan_tmp;  // digit (one-pass: tile) totals; [nbins] ClassBuffers::vmax
   uint32_t *bin_start; // nbins + 1
   uint32_t *sub_ofs;   // nbins + 2; [nbins] = number of subproblems, [nbins + 1] = total work
   int4 *subs;          // (bin, start, count, work before it)
@@ -191,32 +191,33 @@ struct PointArgs {
   int ncls, cw;
 };
 
-// Compact per-point records in sorted order for the MFMA kernels, 32 bytes
-// per point as two float4: r[2s] = (z0, z1, z2, off), r[2s+1] = (c.x, c.y,
-// key, idx).  z[a] = 1 - 2 (t - cell) of axis a (the argument of the tap
-// polynomials, FP64-folded and rounded once, exactly as kb_taps computes
-// it); off = x register cell | y column << 8 | z column << 16 of the first
-// taps in the point's tile; c = value (Type-1, else 0); key = tile; idx =
-// input index of the point.  off, key and idx are stored as their bits.
+// Compact per-point records in sorted order for the MFMA kernels: r[s] =
+// (z0, z1, z2, off), z[a] = 1 - 2 (t - cell) of axis a (the argument of the
+// tap polynomials, FP64-folded and rounded once, exactly as kb_taps computes
+// it), off = x register cell | y column << 8 | z column << 16 of the first
+// taps in the point's tile, stored as its bits; v[s] the point's value and
+// i[s] its input index, null where a call needs none.
 struct ZRec {
   float4 *r;
+  float2 *v;
+  uint32_t *i;
 };
 
-// Compact records built by the binning itself: the first digit pass reads
-// the coordinates and values in input order and scatters each point's record
-// (with its key and index) to its place; later passes move the records, and
-// the last one writes them to `out` (tmp is the other buffer of the
-// ping-pong).  The sorted keys and the permutation then live only in the
-// records: PointArgs::perm is not written.
+// Compact records built by the binning itself.  Of the digit passes, the
+// first reads the coordinates and values in input order, later ones move
+// 32-byte records (r[2 s] as above, r[2 s + 1] = (value, key, index)) between
+// tmp and the space of `out`, and the last writes out.  PointArgs::perm is
+// not written.
 struct RecordOut {
   ZRec out;
   ZRec tmp;
   const float2 *values;  // point values (Type-1) or null
 };
 
-// One problem of the one-pass binning (sort.hip).  A single binning passes
-// it by value; the batched binning reads a device table of them, chunk0 /
-// scan0 being the problem's first chunk / scan block in the shared launches.
+// One problem of the one-pass and tile binnings (sort.hip).  A single binning
+// passes it by value; the batched one reads a device table of them, chunk0, scan0
+// and piece0 being its first chunk, scan block and subproblem in the shared
+// launches.
 struct BinProblem {
   PointArgs pa;             // coordinates and point count
   Geom g;
@@ -227,11 +228,12 @@ struct BinProblem {
   int4 *subs;
   ZRec out;                 // records (REC) ...
   uint32_t *keys_out, *idx_out;  // ... or sorted keys and the permutation
-  const float2 *values;     // record values (Type-1 strengths, gradient u) or null
+  const float2 *values;     // record values (out.v: Type-1 strengths, gradient u) or null
   int dim, nbins, bits, max_sub, sub_work, nchunks, along_x;
   ClassBuffers cls;
+  int chunk;                // tile binning: points of a chunk
   uint32_t chunk0, scan0, piece0;
-  int fused;                // one problem: the scatter launch also writes the list
+  int fused;                // one pass: the scatter launch also writes the list
 };
 
 // One problem of a batched spreading launch.
@@ -256,17 +258,19 @@ hipError_t launch_fill(float2 *p, int64_t n, hipStream_t s);
 
 hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBuffers &sb,
                        hipStream_t s, const RecordOut *rec = nullptr);
-// Binning of nprob problems in shared launches (count, scan, subproblem
-// lists, scatter: four launches for all), records written to each problem's
-// out; every problem must take the one-pass binning.  host_probs' chunk0,
-// scan0, bits and nchunks are filled here; dev_table holds nprob entries.
+// Tile binning (records and class list) of nprob problems in shared
+// launches; every problem must take the tile binning.
+// host_probs' chunk fields are filled here; dev_table holds
+// nprob entries.
 hipError_t sort_points_batched(BinProblem *host_probs, int nprob, BinProblem *dev_table,
                                hipStream_t s);
 // Whether a tile count takes the one-pass binning, and the entries of
 // SortBuffers::cnt the binning of num_points points needs.
 bool sort_one_pass(int nbins);
+bool tile_binning(int nbins);  // records with a class list: without digit passes
 size_t radix_count_entries(int64_t num_points);              // digit passes
 size_t one_pass_count_entries(int64_t num_points, int nbins);  // 0: not one pass
+size_t tile_count_entries(int64_t num_points, int nbins);      // 0: not the tile binning
 
 hipError_t launch_fft_pass(const FftPass &p, hipStream_t s);
 

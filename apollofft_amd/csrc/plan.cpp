@@ -287,13 +287,14 @@ Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
       const anufft_plan::Binning *b = all[i];
       nb = std::max(nb, b->nbins);
       one_n = std::max(one_n, one_pass_count_entries(M, b->nbins));
+      if (b->ncls > 0) one_n = std::max(one_n, tile_count_entries(M, b->nbins));
     }
-    const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
-    if (!classes) cnt_n = std::max(cnt_n, one_n);
+    if (p->dim != 3 || p->kernel_method != kSpreadMfma) cnt_n = std::max(cnt_n, one_n);
     l.cnt = take(4 * cnt_n);
-    l.scan = take(4 * (size_t)std::max(kRadix, nb));  // digit (or tile) totals
+    const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
+    l.scan = take(4 * (size_t)(std::max(kRadix, nb) + 1));  // digit (or tile) totals, value maximum
     l.bin_start = take(4 * (size_t)(nb + 1));
-    l.sub_ofs = take(4 * (size_t)(nb + 3));  // (nb unused,) list totals, value maximum
+    l.sub_ofs = take(4 * (size_t)(nb + 2));  // (nb unused,) list totals
     int64_t nsub = 1;
     for (int i = 0; i < kinds; ++i) nsub = std::max<int64_t>(nsub, all[i]->list_len(M) + 1);
     l.subs = take(16 * (size_t)nsub);
@@ -757,19 +758,28 @@ struct Exec {
   float2 *grid() const { return (float2 *)(ws + lay.grid); }
   float *rec() const { return (float *)(ws + lay.rec); }
   uint8_t *xo() const { return (uint8_t *)(ws + lay.xo); }
-  ZRec zrec(int64_t, bool second = false) const {
-    ZRec z{};
-    z.r = (float4 *)(ws + (second ? lay.zrec2 : lay.zrec));
-    return z;
+  // Records of M points (32 bytes each kept for them and for the digit passes').
+  ZRec zrec(int64_t M) const {
+    char *r = ws + lay.zrec;
+    return ZRec{(float4 *)r, (float2 *)(r + 16 * M), (uint32_t *)(r + 24 * M)};
+  }
+  // What a binning's records hold besides the positions.
+  enum Fields { kValues = 1, kIndices = 2 };
+  RecordOut record_out(int64_t M, const float2 *values, int fields) const {
+    RecordOut ro{zrec(M), ZRec{(float4 *)(ws + lay.zrec2), nullptr, nullptr}, values};
+    if (!(fields & kValues)) ro.out.v = nullptr;
+    if (!(fields & kIndices)) ro.out.i = nullptr;
+    return ro;
   }
   // Binning; with records (MFMA kernels) the sort passes also build the
   // compact per-point records in sorted order.
   hipError_t bin(const anufft_plan::Binning &b, const PointArgs &pa, const float2 *values,
-                 bool records) const {
+                 int fields) const {
     return timed(ANUFFT_STAGE_BIN, [&] {
-      if (!records) return sort_points(pa, b.g, p->dim, sort_buffers(b), s);
-      const RecordOut ro{zrec(pa.num_points), zrec(pa.num_points, true), values};
-      return sort_points(pa, b.g, p->dim, sort_buffers(b), s, &ro);
+      const SortBuffers sb = sort_buffers(b);
+      if (p->kernel_method != kSpreadMfma) return sort_points(pa, b.g, p->dim, sb, s);
+      const RecordOut ro = record_out(pa.num_points, values, fields);
+      return sort_points(pa, b.g, p->dim, sb, s, &ro);
     });
   }
   // Full weight records of sorted points for the vector-ALU spreading kernel.
@@ -843,8 +853,10 @@ struct Exec {
     sb.keys[1] = (uint32_t *)(ws + lay.keys1);
     sb.idx[0] = (uint32_t *)(ws + lay.idx0);
     sb.idx[1] = (uint32_t *)(ws + lay.idx1);
+    // in the second record buffer where no digit pass with records needs it
     const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
-    sb.cnt = (uint32_t *)(ws + (classes && sort_one_pass(b.nbins) ? lay.zrec2 : lay.cnt));
+    const bool direct = sort_one_pass(b.nbins) || (b.ncls > 0 && tile_binning(b.nbins));
+    sb.cnt = (uint32_t *)(ws + (classes && direct ? lay.zrec2 : lay.cnt));
     sb.scan_tmp = (uint32_t *)(ws + lay.scan);
     sb.bin_start = (uint32_t *)(ws + lay.bin_start);
     sb.sub_ofs = (uint32_t *)(ws + lay.sub_ofs);
@@ -862,10 +874,9 @@ struct Exec {
       ClassBuffers &c = sb.cls;
       c.ncls = b.ncls;
       c.cw = b.cw;
-      while ((1 << c.bits) < b.ncls * b.g.bin[0]) ++c.bits;
       c.perm = sb.idx[0];
       c.start = (uint16_t *)(ws + lay.zrec2);
-      c.vmax = sb.sub_ofs + b.nbins + 2;
+      c.vmax = sb.scan_tmp + b.nbins;
     }
     return sb;
   }
@@ -1205,13 +1216,20 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
     if (e != hipSuccess) return hip_fail(e, "spread");
   } else if (M > 0) {
     PointArgs pa = ex.point_args(bs, M, coords, stride);
-    const bool records = p->kernel_method == kSpreadMfma;
-    // zeroing the grid (second stream) is independent of the binning
-    e = ex.fork_join(
-        [&](const Exec &ea) {
-          return ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
-        },
-        [&] { return ex.bin(bs, pa, (const float2 *)values, records); });
+    auto fill = [&](const Exec &ea) {
+      return ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
+    };
+    auto bin = [&] { return ex.bin(bs, pa, (const float2 *)values, Exec::kValues); };
+    // The grid is zeroed before the binning: beside it, on the second stream,
+    // the 2 us (64^3 cells) to 19 us (254^3) cost more in the fork and join,
+    // about 25 us.  Not so right after the copies of a host call, where the
+    // fork costs nothing (the call: 403 us with it, 458 without).
+    if (blocks) {
+      e = ex.fork_join(fill, bin);
+    } else {
+      e = fill(ex);
+      if (e == hipSuccess) e = bin();
+    }
     if (e != hipSuccess) return hip_fail(e, "fill / binning");
     e = blocks ? ex.spread_blocks(pa, ex.grid()) : ex.spread3(pa, (const float2 *)values, ex.grid());
     if (e != hipSuccess) return hip_fail(e, "spread");
@@ -1279,7 +1297,7 @@ anufft_status anufft_execute_type2(const anufft_plan *p, int64_t M, const float 
         [&](const Exec &ea) {
           return ea.fine_grid((const float2 *)modes, p->opts.compat_reference_type2_3d_scaling != 0);
         },
-        [&] { return ex.bin(p->bi, pa, nullptr, p->kernel_method == kSpreadMfma); });
+        [&] { return ex.bin(p->bi, pa, nullptr, Exec::kIndices); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
     e = ex.interp3(pa, ex, (float2 *)out);
   } else {
@@ -1314,7 +1332,7 @@ anufft_status anufft_execute_grad_points(const anufft_plan *p, int64_t M,
     PointArgs pa = ex.point_args(b, M, coords, stride);
     // FFT passes (second stream) concurrent with the binning
     e = ex.fork_join([&](const Exec &ea) { return ea.fine_grid((const float2 *)modes_h, false); },
-                     [&] { return ex.bin(b, pa, (const float2 *)u, gm); });
+                     [&] { return ex.bin(b, pa, (const float2 *)u, Exec::kValues | Exec::kIndices); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
     e = ex.grad3(pa, ex, (const float2 *)u, grad);
   } else {
@@ -1362,7 +1380,7 @@ anufft_status anufft_execute_type2_backward(const anufft_plan *p, int64_t M,
           r = ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
         return r;
       },
-      [&] { return ex.bin(p->bs, pa, (const float2 *)g, true); });
+      [&] { return ex.bin(p->bs, pa, (const float2 *)g, Exec::kValues | Exec::kIndices); });
   if (e != hipSuccess) return hip_fail(e, "fft / fill / binning");
   e = ex.spread3(pa, (const float2 *)g, ex.grid());
   if (e != hipSuccess) return hip_fail(e, "spread");
@@ -1394,7 +1412,7 @@ anufft_status anufft_execute_type1_backward(const anufft_plan *p, int64_t M,
   PointArgs pa = ex.point_args(p->bi, M, coords, stride);
   hipError_t e = ex.fork_join(
       [&](const Exec &ea) { return ea.fine_grid((const float2 *)G, false); },
-      [&] { return ex.bin(p->bi, pa, (const float2 *)values, true); });
+      [&] { return ex.bin(p->bi, pa, (const float2 *)values, Exec::kValues | Exec::kIndices); });
   if (e != hipSuccess) return hip_fail(e, "fft / binning");
   e = ex.interp3(pa, ex, (float2 *)grad_values);
   if (e != hipSuccess) return hip_fail(e, "interp");
@@ -1515,7 +1533,7 @@ anufft_status anufft_debug_spread(const anufft_plan *p, int64_t M, const float *
   if (M == 0) return ANUFFT_OK;
   PointArgs pa = ex.point_args(p->bs, M, coords, stride);
   if (p->dim == 3) {
-    e = ex.bin(p->bs, pa, (const float2 *)values, p->kernel_method == kSpreadMfma);
+    e = ex.bin(p->bs, pa, (const float2 *)values, Exec::kValues);
     if (e != hipSuccess) return hip_fail(e, "binning");
     e = ex.spread3(pa, (const float2 *)values, (float2 *)grid);
   } else {
@@ -1627,7 +1645,7 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
   };
   auto sort_range = [&](int parity, hipStream_t st) {
     for (int i = parity; i < nprob; i += 2) {
-      const RecordOut ro{probs[i].zr, ex[i].zrec(num_points[i], true), (const float2 *)values[i]};
+      const RecordOut ro = ex[i].record_out(num_points[i], (const float2 *)values[i], Exec::kValues);
       SortBuffers sb = ex[i].sort_buffers(plans[i]->bs);
       sb.sub_work = sub_work(i);
       // the persistent launch balances work across all problems itself:
@@ -1639,9 +1657,9 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
     return hipSuccess;
   };
   // all problems with one-pass tile counts and records: one fused binning
-  // (four launches for all problems) beside the grids' zeroing
+  // (its launches shared by all problems) beside the grids' zeroing
   bool one_launch = mf;
-  for (int i = 0; i < nprob && one_launch; ++i) one_launch = sort_one_pass(plans[i]->bs.nbins);
+  for (int i = 0; i < nprob && one_launch; ++i) one_launch = tile_binning(plans[i]->bs.nbins);
   std::vector<BinProblem> bprobs;
   if (one_launch) {
     bprobs.resize(nprob);
@@ -1652,10 +1670,9 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
       b.g = plans[i]->bs.g;
       b.cnt = sb.cnt;
       b.tot = sb.scan_tmp;
-      b.bin_start = sb.bin_start;
       b.nsub = sb.sub_ofs + sb.nbins;
       b.subs = sb.subs;
-      b.out = probs[i].zr;
+      b.out = ex[i].record_out(num_points[i], nullptr, Exec::kValues).out;
       b.values = (const float2 *)values[i];
       b.dim = 3;
       b.nbins = sb.nbins;

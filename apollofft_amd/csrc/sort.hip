@@ -158,7 +158,7 @@ struct RecMove {
   const float2 *values;  // value field present (Type-1) or null
   PointArgs pa;
   Geom g;
-  int first;
+  int first, last;
   uint32_t *vmax;        // first pass with values: their largest component, or null
 };
 
@@ -224,7 +224,12 @@ __global__ __launch_bounds__(kSortThreads) void scatter_kernel(
     if (valid) {
       uint32_t pos = running[d] + rank;
       for (int w = 0; w < wave; ++w) pos += wcount[w][d];
-      if (REC) {
+      if (REC && rm.last) {
+        rm.out.r[pos] = ra;
+        if (rm.out.v) rm.out.v[pos] = make_float2(rb.x, rb.y);
+        if (rm.out.i) rm.out.i[pos] = __float_as_uint(rb.w);
+        keys_out[pos] = key;
+      } else if (REC) {
         rm.out.r[2 * (int64_t)pos] = ra;
         rm.out.r[2 * (int64_t)pos + 1] = rb;
       } else {
@@ -311,9 +316,8 @@ __device__ __forceinline__ uint64_t block_scan_waves64(uint64_t v, uint64_t *sh,
 // first writes bin_start[b] = sum of tot[d] over d < b, b in [0, nbins];
 // tot == NULL with no points means all tiles are empty.
 constexpr int kSubThreads = 1024;
-constexpr int kSubPer = 4;
 // LDS of the list for a block of NT threads (rounds of NT * kSubPer tiles).
-template <int NT>
+template <int NT, int kSubPer = 4>
 struct SubLds {
   static constexpr int kRound = NT * kSubPer;
   uint32_t sh[NT / 64];
@@ -321,12 +325,12 @@ struct SubLds {
   uint32_t first[kRound];  // first entry of each tile of the round
   int4 tinfo[kRound];      // tile: bin, first point, count, work before it
 };
-template <int NT>
-__device__ __forceinline__ void subproblems_body(SubLds<NT> &L, uint32_t *bin_start,
+template <int NT, int kSubPer = 4>
+__device__ __forceinline__ void subproblems_body(SubLds<NT, kSubPer> &L, uint32_t *bin_start,
                                                  const uint32_t *tot, int from_tot, int nbins,
                                                  int3 nb, bool along_x, int max_sub, int sub_work,
                                                  uint32_t *nsub, int4 *subs) {
-  constexpr int kSubRound = SubLds<NT>::kRound;
+  constexpr int kSubRound = SubLds<NT, kSubPer>::kRound;
   uint32_t *sh = L.sh;
   uint64_t *sh64 = L.sh64;
   uint32_t *first = L.first;
@@ -507,33 +511,9 @@ __device__ __forceinline__ uint32_t fold_point(const float (&c)[3], const Geom &
 // LDS (the sums do not depend on the order of the atomic adds).
 constexpr int kCountThreads = 1024;
 constexpr int kCountPer = kOneChunk / kCountThreads;
-// The problem of this block: the one passed by value, or (BATCH) the last
-// table entry whose first block (chunk0 or scan0) is at most blockIdx.x.
-template <bool BATCH, bool SCAN>
-__device__ __forceinline__ const BinProblem &bin_problem(const BinProblem &one,
-                                                          const BinProblem *table, int nprob,
-                                                          uint32_t &local) {
-  if (!BATCH) {
-    local = blockIdx.x;
-    return one;
-  }
-  int lo = 0, hi = nprob - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if ((SCAN ? table[mid].scan0 : table[mid].chunk0) <= blockIdx.x) lo = mid;
-    else hi = mid - 1;
-  }
-  local = blockIdx.x - (SCAN ? table[lo].scan0 : table[lo].chunk0);
-  return table[lo];
-}
-
-template <bool BATCH>
-__global__ __launch_bounds__(kCountThreads) void chunk_count_kernel(BinProblem one,
-                                                                    const BinProblem *table,
-                                                                    int nprob) {
+__global__ __launch_bounds__(kCountThreads) void chunk_count_kernel(BinProblem pr) {
   extern __shared__ uint32_t hist[];  // nbins
-  uint32_t chunk;
-  const BinProblem &pr = bin_problem<BATCH, false>(one, table, nprob, chunk);
+  const uint32_t chunk = blockIdx.x;
   const int nbins = pr.nbins, dim = pr.dim;
   const PointArgs &pa = pr.pa;
   for (int d = threadIdx.x; d < nbins; d += kCountThreads) hist[d] = 0;
@@ -564,15 +544,10 @@ __global__ __launch_bounds__(kCountThreads) void chunk_count_kernel(BinProblem o
 // so each thread has one short run of loads in flight.
 constexpr int kScanDigits = 16;
 constexpr int kChunkScanSegs = 64;
-template <bool BATCH>
-__global__ __launch_bounds__(kScanDigits * kChunkScanSegs) void chunk_scan_kernel(
-    BinProblem one, const BinProblem *table, int nprob) {
+__device__ __forceinline__ void chunk_scan(const BinProblem &pr, uint32_t blk) {
   __shared__ uint32_t seg[kChunkScanSegs][kScanDigits];
-  uint32_t blk;
-  const BinProblem &pr = bin_problem<BATCH, true>(one, table, nprob, blk);
   uint32_t *cnt = pr.cnt;
   const int nchunks = pr.nchunks, nbins = pr.nbins;
-  if (blk == 0 && threadIdx.x == 0 && pr.cls.ncls > 0) *pr.cls.vmax = 0u;
   const int dl = threadIdx.x & (kScanDigits - 1), sg = threadIdx.x / kScanDigits;
   const int d = (int)blk * kScanDigits + dl;
   const int per = (nchunks + kChunkScanSegs - 1) / kChunkScanSegs;
@@ -602,18 +577,11 @@ __global__ __launch_bounds__(kScanDigits * kChunkScanSegs) void chunk_scan_kerne
     if (sg == 0) pr.tot[d] = total;
   }
 }
-
-// Subproblem lists of a batch: one block per problem.
-__global__ __launch_bounds__(kSubThreads) void subproblems_batched_kernel(const BinProblem *table) {
-  const BinProblem &pr = table[blockIdx.x];
-  const int3 nb = pr.dim == 3 ? make_int3(pr.g.nbin[0], pr.g.nbin[1], pr.g.nbin[2])
-                              : make_int3(1, 1, 1);
-  __shared__ SubLds<kSubThreads> L;
-  subproblems_body<kSubThreads>(L, pr.bin_start, pr.pa.num_points > 0 ? pr.tot : nullptr, 1,
-                                pr.nbins, nb, pr.along_x, pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
+__global__ __launch_bounds__(kScanDigits * kChunkScanSegs) void chunk_scan_kernel(BinProblem pr) {
+  chunk_scan(pr, blockIdx.x);
 }
 
-// Fused list (one problem, one.fused): block 0 writes bin_start and the
+// Fused list (pr.fused): block 0 writes bin_start and the
 // subproblem list from the tile totals, beside the scatter; every other
 // block scans the totals into LDS for the tile starts of its own points.
 // Otherwise bin_start comes from the list launch before this one.
@@ -626,25 +594,20 @@ constexpr int kFusedMaxBins = 8176;
 static_assert(kFusedMaxBins <= kFusedTotPer * kOneThreads, "fused scan covers the tiles");
 static_assert(20 * kFusedMaxBins + 4 * kOneWaves <= 160 * 1024, "fused scatter LDS");
 static_assert(sizeof(SubLds<kOneThreads>) + 4 * kOneWaves <= 160 * 1024, "list LDS");
-template <bool REC, bool BATCH>
-__global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem one,
-                                                                    const BinProblem *table,
-                                                                    int nprob) {
+template <bool REC>
+__global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem pr) {
   extern __shared__ uint4 scatter_lds[];
   __shared__ uint32_t wsum[kOneWaves];
   uint16_t *rows = (uint16_t *)scatter_lds;
-  const bool fused = !BATCH && one.fused;
+  const bool fused = pr.fused;
   if (fused && blockIdx.x == 0) {
-    const int3 nb = one.dim == 3 ? make_int3(one.g.nbin[0], one.g.nbin[1], one.g.nbin[2])
-                                 : make_int3(1, 1, 1);
-    subproblems_body<kOneThreads>(*(SubLds<kOneThreads> *)scatter_lds, one.bin_start, one.tot, 1,
-                                  one.nbins, nb, one.along_x, one.max_sub, one.sub_work,
-                                  one.nsub, one.subs);
+    const int3 nb = pr.dim == 3 ? make_int3(pr.g.nbin[0], pr.g.nbin[1], pr.g.nbin[2])
+                                : make_int3(1, 1, 1);
+    subproblems_body<kOneThreads>(*(SubLds<kOneThreads> *)scatter_lds, pr.bin_start, pr.tot, 1,
+                                  pr.nbins, nb, pr.along_x, pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
     return;
   }
-  uint32_t chunk;
-  const BinProblem &pr = bin_problem<BATCH, false>(one, table, nprob, chunk);
-  if (fused) chunk -= 1;
+  const uint32_t chunk = blockIdx.x - (fused ? 1u : 0u);
   const int nbins = pr.nbins, dim = pr.dim, bits = pr.bits;
   const PointArgs &pa = pr.pa;
   for (int i = threadIdx.x; i < kOneWaves / 2 * nbins; i += kOneThreads) ((uint32_t *)rows)[i] = 0u;
@@ -662,13 +625,6 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
     const bool valid = j < pa.num_points;
     load_point(pa, dim, j, valid, c[s]);
     val[s] = (REC && pr.values) ? pr.values[valid ? j : 0] : make_float2(0.f, 0.f);
-  }
-  if (REC && pr.values && pr.cls.ncls > 0) {
-    float mx = 0.f;
-#pragma unroll
-    for (int s = 0; s < kOneSteps; ++s)
-      if (j0 + 64 * s < pa.num_points) mx = fmaxf(mx, fmaxf(fabsf(val[s].x), fabsf(val[s].y)));
-    value_max(mx, pr.cls.vmax);
   }
   // fused: this thread's run of tile totals (clamped indices, no branch)
   const int per = (nbins + kOneThreads - 1) / kOneThreads;
@@ -736,14 +692,179 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
     const int64_t j = j0 + 64 * s;
     if (j >= pa.num_points) continue;
     if (REC) {
-      pr.out.r[2 * (int64_t)pos[s]] =
-          make_float4(zr[s][0], zr[s][1], zr[s][2], __int_as_float(off[s]));
-      pr.out.r[2 * (int64_t)pos[s] + 1] =
-          make_float4(val[s].x, val[s].y, __uint_as_float(key[s]), __uint_as_float((uint32_t)j));
+      pr.out.r[pos[s]] = make_float4(zr[s][0], zr[s][1], zr[s][2], __int_as_float(off[s]));
+      if (pr.out.v) pr.out.v[pos[s]] = val[s];
+      if (pr.out.i) pr.out.i[pos[s]] = (uint32_t)j;
     } else {
       pr.keys_out[pos[s]] = key[s];
       pr.idx_out[pos[s]] = (uint32_t)j;
     }
+  }
+}
+
+// ---- tile binning (records with a class list) -------------------------------
+// The matrix-core kernels order a tile's points by class and x offset
+// themselves (class_sort_kernel), so their records need no stable order
+// inside a tile: a point takes its place from an LDS counter of its tile
+// instead of a rank by ballots, and a chunk can be as long as keeps every CU
+// busy with two (the counts of (chunk, tile) pairs stay small).
+//   tile_count    : per-chunk tile histogram, cnt[chunk][tile]
+//   tile_scan     : per-tile exclusive scan over the chunks (in place) and the
+//                   tile totals; left out for a single chunk
+//   tile_scatter  : every block scans the totals in LDS for the tile starts;
+//                   the first writes the subproblem list, the others add their
+//                   chunk's offsets and stream their points to their places
+// The scatter is bound by its writes of 20 to 28 bytes a point to scattered
+// places.  Measured, count, scan, scatter and class list together against the
+// stable one-pass binning: 2e6 points, 1368 tiles, 92 and 75 us; 16e6
+// clustered, 6176 tiles, 850 and 480 (with places in input order, no scatter,
+// 55 and 316).  (Places from global counters, 490 chunks meeting on each: 26 us
+// more at 2e6, 125 at 16e6.)
+constexpr int kTileThreads = 1024;
+
+// The problem of this block: the one passed by value, or (BATCH) the last
+// table entry whose first block is at most blockIdx.x; first block of entry
+// i: chunk0 (COUNT), scan0 (SCAN), or chunk0 + i (SCATTER: a list block each).
+enum TileStep { kTileCount, kTileScan, kTileScatter };
+template <bool BATCH, TileStep STEP>
+__device__ __forceinline__ const BinProblem &tile_problem(const BinProblem &one,
+                                                           const BinProblem *table, int nprob,
+                                                           uint32_t &local) {
+  local = blockIdx.x;
+  if (!BATCH) return one;
+  auto first = [&](int i) {
+    return STEP == kTileScan ? table[i].scan0 : table[i].chunk0 + (STEP == kTileScatter ? i : 0);
+  };
+  int lo = 0, hi = nprob - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (first(mid) <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  local = blockIdx.x - first(lo);
+  return table[lo];
+}
+
+template <bool BATCH>
+__global__ __launch_bounds__(kTileThreads) void tile_count_kernel(BinProblem one,
+                                                                  const BinProblem *table,
+                                                                  int nprob) {
+  extern __shared__ uint32_t hist[];  // nbins
+  uint32_t chunk;
+  const BinProblem &pr = tile_problem<BATCH, kTileCount>(one, table, nprob, chunk);
+  const int nbins = pr.nbins;
+  const PointArgs &pa = pr.pa;
+  if (chunk == 0 && threadIdx.x == 0) *pr.cls.vmax = 0u;
+  for (int d = threadIdx.x; d < nbins; d += kTileThreads) hist[d] = 0;
+  const int64_t end = min(pa.num_points, (int64_t)(chunk + 1) * pr.chunk);
+  int64_t j = (int64_t)chunk * pr.chunk + threadIdx.x;
+  float c[3], cn[3];
+  load_point(pa, 3, j, j < end, c);
+  __syncthreads();
+  for (; j < end; j += kTileThreads) {
+    load_point(pa, 3, j + kTileThreads, j + kTileThreads < end, cn);
+    float z[3];
+    int off;
+    atomicAdd(&hist[fold_point<false>(c, pr.g, 3, z, off)], 1u);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[a] = cn[a];
+  }
+  __syncthreads();
+  uint32_t *row = pr.cnt + (int64_t)chunk * nbins;
+  for (int d = threadIdx.x; d < nbins; d += kTileThreads) row[d] = hist[d];
+}
+
+template <bool BATCH>
+__global__ __launch_bounds__(kScanDigits * kChunkScanSegs) void tile_scan_kernel(
+    BinProblem one, const BinProblem *table, int nprob) {
+  uint32_t blk;
+  const BinProblem &pr = tile_problem<BATCH, kTileScan>(one, table, nprob, blk);
+  chunk_scan(pr, blk);
+}
+
+typedef SubLds<kTileThreads, 1> TileSubLds;
+// LDS of the scatter: the tile starts (nbins + 1), then (list block) the list's.
+static size_t tile_scatter_lds(int nbins) {
+  return sizeof(uint32_t) * (((size_t)nbins + 4) & ~(size_t)3) + sizeof(TileSubLds);
+}
+
+template <bool BATCH>
+__global__ __launch_bounds__(kTileThreads) void tile_scatter_kernel(BinProblem one,
+                                                                    const BinProblem *table,
+                                                                    int nprob) {
+  extern __shared__ uint4 tile_lds[];
+  __shared__ float wmax[kTileThreads / 64];
+  __shared__ uint32_t sh[kTileThreads / 64];
+  uint32_t chunk;
+  const BinProblem &pr = tile_problem<BATCH, kTileScatter>(one, table, nprob, chunk);
+  const int nbins = pr.nbins;
+  const PointArgs &pa = pr.pa;
+  uint32_t *place = (uint32_t *)tile_lds;  // next place of each tile
+  // tile starts: the totals' exclusive scan, a run of tiles per thread
+  for (int d = threadIdx.x; d < nbins; d += kTileThreads) place[d] = pr.tot[d];
+  __syncthreads();
+  {
+    const int per = (nbins + kTileThreads - 1) / kTileThreads;
+    const int d0 = min(nbins, (int)threadIdx.x * per), d1 = min(nbins, d0 + per);
+    uint32_t sum = 0, total;
+    for (int d = d0; d < d1; ++d) sum += place[d];
+    uint32_t at = block_scan_waves<kTileThreads>(sum, sh, total);
+    for (int d = d0; d < d1; ++d) {
+      const uint32_t v = place[d];
+      place[d] = at;
+      at += v;
+    }
+    if (threadIdx.x == 0) place[nbins] = total;
+  }
+  __syncthreads();
+  if (chunk == 0) {
+    subproblems_body<kTileThreads, 1>(*(TileSubLds *)(place + ((nbins + 4) & ~3)), place, nullptr, 0,
+                                      nbins, make_int3(pr.g.nbin[0], pr.g.nbin[1], pr.g.nbin[2]),
+                                      pr.along_x, pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
+    return;
+  }
+  --chunk;
+  {  // consecutive chunks on one XCD (blocks are dealt to the XCDs in turn):
+     // the runs they write in a tile join in its L2 (2e6 points: 79 to 75 us)
+    const uint32_t n = (uint32_t)pr.nchunks, x = chunk & 7u;
+    chunk = x * (n >> 3) + min(x, n & 7u) + (chunk >> 3);
+  }
+  const int64_t end = min(pa.num_points, (int64_t)(chunk + 1) * pr.chunk);
+  int64_t j = (int64_t)chunk * pr.chunk + threadIdx.x;
+  const bool vals = pr.out.v != nullptr;
+  float c[3], cn[3];
+  float2 v = make_float2(0.f, 0.f), vn = v;
+  load_point(pa, 3, j, j < end, c);
+  if (vals) v = pr.values[j < end ? j : 0];
+  if (pr.nchunks > 1) {
+    const uint32_t *coff = pr.cnt + (int64_t)chunk * nbins;
+    for (int d = threadIdx.x; d < nbins; d += kTileThreads) place[d] += coff[d];
+    __syncthreads();
+  }
+  float mx = 0.f;
+  for (; j < end; j += kTileThreads) {
+    const int64_t jn = j + kTileThreads;
+    load_point(pa, 3, jn, jn < end, cn);
+    if (vals) vn = pr.values[jn < end ? jn : 0];
+    float z[3];
+    int off;
+    const uint32_t p = atomicAdd(&place[fold_point<true>(c, pr.g, 3, z, off)], 1u);
+    pr.out.r[p] = make_float4(z[0], z[1], z[2], __int_as_float(off));
+    if (vals) {
+      pr.out.v[p] = v;
+      mx = fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y)));
+    }
+    if (pr.out.i) pr.out.i[p] = (uint32_t)j;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[a] = cn[a];
+    v = vn;
+  }
+  if (vals) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x < 64) value_max(threadIdx.x < kTileThreads / 64 ? wmax[threadIdx.x] : 0.f, pr.cls.vmax);
   }
 }
 
@@ -754,13 +875,12 @@ __global__ __launch_bounds__(kOneThreads) void chunk_scatter_kernel(BinProblem o
 // their own would be 3 to 16 times as many), and the classes are listed inside
 // each subproblem of the tile list: one block per subproblem (at most
 // kClassSub points) ranks every point among those of its class and x offset
-// (stable) and writes the sorted positions in that order (perm) and the
+// (LDS atomics) and writes the sorted positions in that order (perm) and the
 // classes' starts.  The x order lets the kernels leave out the x cells no
 // point of a group reaches.
 constexpr int kClsThreads = 256;
-constexpr int kClsWaves = kClsThreads / 64;
 constexpr int kClsSteps = kClassSub / kClsThreads;
-constexpr int kClsKeys = 256;  // (class, x offset) pairs at most
+constexpr int kClsKeys = kClsThreads;  // (class, x offset) pairs at most
 
 // The problem of this block: the one passed by value (no table), or the last
 // table entry whose first block is at most blockIdx.x.
@@ -782,88 +902,51 @@ __device__ __forceinline__ const BinProblem &piece_problem(const BinProblem &one
 __global__ __launch_bounds__(kClsThreads) void class_sort_kernel(BinProblem one,
                                                                  const BinProblem *table,
                                                                  int nprob) {
-  __shared__ uint32_t cnt[kClsWaves][kClsKeys];  // per wave: points of each key, then their places
-  __shared__ uint32_t sh[kClsWaves];
+  __shared__ uint32_t cnt[kClsKeys];  // points of each key, then its first place
+  __shared__ uint32_t sh[kClsThreads / 64];
   uint32_t piece;
   const BinProblem &pr = piece_problem(one, table, nprob, piece);
   if (piece >= pr.nsub[0]) return;
   const ClassBuffers &cb = pr.cls;
-  const int ncls = cb.ncls, binx = pr.g.bin[0], nkeys = ncls * binx, bits = cb.bits;
+  const int ncls = cb.ncls, binx = pr.g.bin[0], nkeys = ncls * binx;
   const int4 sub = pr.subs[piece];
   const int n = sub.z;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  // each wave ranks one contiguous run of `steps` x 64 points
-  const int steps = (n + kClsThreads - 1) / kClsThreads;
-  const float *ofs = (const float *)pr.out.r + 8 * (int64_t)sub.y + 3;  // point p's offsets: ofs[8 p]
-  const int p0 = wave * steps * 64 + lane;
+  const float *ofs = (const float *)(pr.out.r + sub.y) + 3;  // point p's offsets: ofs[4 p]
   const float inv_cw = 1.0f / (float)cb.cw;
   int o[kClsSteps];
 #pragma unroll
   for (int s = 0; s < kClsSteps; ++s) {
-    const int p = p0 + 64 * s;
-    o[s] = s < steps && p < n ? __float_as_int(ofs[8 * (int64_t)p]) : -1;
+    const int p = threadIdx.x + s * kClsThreads;
+    o[s] = p < n ? __float_as_int(ofs[4 * (int64_t)p]) : -1;
   }
-#pragma unroll
-  for (int w = 0; w < kClsWaves; ++w) cnt[w][threadIdx.x] = 0u;
+  cnt[threadIdx.x] = 0u;
   __syncthreads();
-  uint32_t *row = cnt[wave];
   uint32_t rk[kClsSteps];
 #pragma unroll
   for (int s = 0; s < kClsSteps; ++s) {
-    if (s >= steps) break;
-    const bool valid = o[s] >= 0;
     // class (o1 - 1) / cw of the y offset o1 >= 1 (cell_div's rounding argument)
     const int c = (int)(((float)((o[s] >> 8) & 255) - 0.5f) * inv_cw);
-    const uint32_t k = valid ? (uint32_t)(c * binx + (o[s] & 255)) : 0u;
-    const uint64_t peers = key_peers(k, valid, bits);
-    const uint64_t below = peers & lt;
-    uint32_t b0 = 0;
-    if (valid && below == 0ull) {  // the first lane of each key claims the step's places
-      b0 = row[k];
-      row[k] = b0 + (uint32_t)__popcll(peers);
-    }
-    const int leader = valid ? __ffsll((unsigned long long)peers) - 1 : lane;
-    rk[s] = __shfl(b0, leader) + (uint32_t)__popcll(below);
-    o[s] = valid ? (int)k : -1;
+    const int k = c * binx + (o[s] & 255);
+    rk[s] = o[s] >= 0 ? atomicAdd(&cnt[k], 1u) : 0u;
+    o[s] = o[s] >= 0 ? k : -1;
   }
   __syncthreads();
-  {
-    // first place of each key, then of each wave's points of it
-    const int k = threadIdx.x;
-    uint32_t c[kClsWaves], tot = 0, all;
-#pragma unroll
-    for (int w = 0; w < kClsWaves; ++w) {
-      c[w] = cnt[w][k];
-      tot += c[w];
-    }
-    uint32_t at = block_scan_waves<kClsThreads>(tot, sh, all);
-    if (k < nkeys && k % binx == 0) cb.start[(int64_t)piece * ncls + k / binx] = (uint16_t)at;
-#pragma unroll
-    for (int w = 0; w < kClsWaves; ++w) {
-      cnt[w][k] = at;
-      at += c[w];
-    }
-  }
+  uint32_t all;
+  const int k = threadIdx.x;
+  const uint32_t at = block_scan_waves<kClsThreads>(cnt[k], sh, all);
+  if (k < nkeys && k % binx == 0) cb.start[(int64_t)piece * ncls + k / binx] = (uint16_t)at;
+  cnt[k] = at;
   __syncthreads();
   uint32_t *perm = cb.perm + (int64_t)sub.y;
 #pragma unroll
-  for (int s = 0; s < kClsSteps; ++s) {
-    if (s >= steps) break;
-    if (o[s] >= 0) perm[row[o[s]] + rk[s]] = (uint32_t)sub.y + (uint32_t)(p0 + 64 * s);
-  }
+  for (int s = 0; s < kClsSteps; ++s)
+    if (o[s] >= 0) perm[cnt[o[s]] + rk[s]] = (uint32_t)(sub.y + (int)threadIdx.x + s * kClsThreads);
 }
 
 // Subproblems of a list at most.
 int class_pieces(int64_t n, int nbins, int max_sub) {
   return (int)(std::min<int64_t>(nbins, n) + (n + max_sub - 1) / max_sub);
 }
-// The class list of one problem.
-void launch_class_sort(const BinProblem &pr, int64_t n, int nbins, int max_sub, hipStream_t s) {
-  hipLaunchKernelGGL(class_sort_kernel, dim3(class_pieces(n, nbins, max_sub)), dim3(kClsThreads), 0, s, pr,
-                     (const BinProblem *)nullptr, 1);
-}
-
 // descriptors per table-fill launch (kernarg size)
 constexpr int kBinTableChunk = 8;
 struct BinTableChunk {
@@ -881,34 +964,66 @@ int key_bits(int nbins) {
   return bits;
 }
 
-hipError_t set_scatter_lds(bool rec, bool batch, size_t lds) {
+hipError_t set_lds(const void *fn, size_t lds) {
   if (lds <= 65536) return hipSuccess;
-  const void *fn = rec ? (batch ? (const void *)chunk_scatter_kernel<true, true>
-                                : (const void *)chunk_scatter_kernel<true, false>)
-                       : (batch ? (const void *)chunk_scatter_kernel<false, true>
-                                : (const void *)chunk_scatter_kernel<false, false>);
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+}
+
+// Points of a chunk: two chunks a CU on 256 CUs, in steps of a block (twice
+// and four times as many: 479, 522 and 593 us at 16e6 points, as their counts
+// grow; 75 and 97 at 2e6); up to 4096 points one chunk, whose totals need no
+// scan launch (5 us) for a few steps of a block (1 us each).
+constexpr int kTileChunks = 512;
+int tile_chunk(int64_t n) {
+  if (n <= 4 * kTileThreads) return 4 * kTileThreads;
+  return (int)(((n + kTileChunks - 1) / kTileChunks + kTileThreads - 1) / kTileThreads) * kTileThreads;
+}
+int tile_chunks(int64_t n) { return (int)((n + tile_chunk(n) - 1) / tile_chunk(n)); }
+
+// The tile binning's launches over `chunks` chunks, `scans` scan blocks and
+// `pieces` subproblems at most, of one problem or a table.
+hipError_t launch_tile_binning(const BinProblem &one, const BinProblem *table, int nprob,
+                               int max_bins, uint32_t chunks, uint32_t scans, uint32_t pieces,
+                               hipStream_t s) {
+  const size_t hist = sizeof(uint32_t) * (size_t)max_bins, lds = tile_scatter_lds(max_bins);
+  const void *scatter = table ? (const void *)tile_scatter_kernel<true> : (const void *)tile_scatter_kernel<false>;
+  hipError_t e = set_lds(scatter, lds);
+  if (e != hipSuccess) return e;
+  const dim3 nt(kTileThreads), ns(kScanDigits * kChunkScanSegs), lists(chunks + (uint32_t)nprob);
+  if (table) {
+    if (chunks > 0) hipLaunchKernelGGL(tile_count_kernel<true>, dim3(chunks), nt, hist, s, one, table, nprob);
+    hipLaunchKernelGGL(tile_scan_kernel<true>, dim3(scans), ns, 0, s, one, table, nprob);
+    hipLaunchKernelGGL(tile_scatter_kernel<true>, lists, nt, lds, s, one, table, nprob);
+  } else {
+    hipLaunchKernelGGL(tile_count_kernel<false>, dim3(chunks), nt, hist, s, one, table, nprob);
+    if (scans > 0) hipLaunchKernelGGL(tile_scan_kernel<false>, dim3(scans), ns, 0, s, one, table, nprob);
+    hipLaunchKernelGGL(tile_scatter_kernel<false>, lists, nt, lds, s, one, table, nprob);
+  }
+  if (pieces > 0)
+    hipLaunchKernelGGL(class_sort_kernel, dim3(pieces), dim3(kClsThreads), 0, s, one, table, nprob);
+  return hipGetLastError();
 }
 
 } // namespace
 
 bool sort_one_pass(int nbins) { return nbins <= kOneMaxBins; }
+// (4 bytes of LDS a tile)
+bool tile_binning(int nbins) { return nbins <= kTileMaxBins; }
 
 size_t radix_count_entries(int64_t num_points) {
   const int64_t M = std::max<int64_t>(num_points, 1);
   return (size_t)(kRadix * ((M + kSortChunk - 1) / kSortChunk));
+}
+size_t tile_count_entries(int64_t num_points, int nbins) {
+  return tile_binning(nbins) ? (size_t)nbins * tile_chunks(std::max<int64_t>(num_points, 1)) : 0;
 }
 size_t one_pass_count_entries(int64_t num_points, int nbins) {
   const int64_t M = std::max<int64_t>(num_points, 1);
   return sort_one_pass(nbins) ? (size_t)nbins * (size_t)((M + kOneChunk - 1) / kOneChunk) : 0;
 }
 
-// One-pass binning: see the comment above chunk_count_kernel.
-static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int dim,
-                                       const SortBuffers &sb, hipStream_t s,
-                                       const RecordOut *rec) {
-  const int64_t n = pa.num_points;
-  const int nbins = sb.nbins;
+static BinProblem bin_problem(const PointArgs &pa, const Geom &g, int dim, const SortBuffers &sb,
+                              const RecordOut *rec) {
   BinProblem pr{};
   pr.pa = pa;
   pr.g = g;
@@ -920,27 +1035,37 @@ static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int d
   if (rec) {
     pr.out = rec->out;
     pr.values = rec->values;
+    pr.cls = sb.cls;
   } else {
     pr.keys_out = sb.keys[sb.passes & 1];
     pr.idx_out = sb.idx[sb.passes & 1];
   }
   pr.dim = dim;
-  pr.nbins = nbins;
-  pr.bits = key_bits(nbins);
+  pr.nbins = sb.nbins;
+  pr.bits = key_bits(sb.nbins);
   pr.max_sub = sb.max_sub;
   pr.sub_work = sb.sub_work;
   pr.along_x = sb.along_x;
-  if (rec) pr.cls = sb.cls;
+  return pr;
+}
+
+// One-pass binning: see the comment above chunk_count_kernel.
+static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int dim,
+                                       const SortBuffers &sb, hipStream_t s,
+                                       const RecordOut *rec) {
+  const int64_t n = pa.num_points;
+  const int nbins = sb.nbins;
+  BinProblem pr = bin_problem(pa, g, dim, sb, rec);
   pr.nchunks = (int)((n + kOneChunk - 1) / kOneChunk);
   const int nch = pr.nchunks;
   // with the tile starts in LDS beside the count rows, the scatter launch
   // also writes the list (one more block)
   pr.fused = n > 0 && nbins <= kFusedMaxBins;
   if (n > 0) {
-    hipLaunchKernelGGL(chunk_count_kernel<false>, dim3(nch), dim3(kCountThreads),
-                       sizeof(uint32_t) * nbins, s, pr, (const BinProblem *)nullptr, 1);
-    hipLaunchKernelGGL(chunk_scan_kernel<false>, dim3((nbins + kScanDigits - 1) / kScanDigits),
-                       dim3(kScanDigits * kChunkScanSegs), 0, s, pr, (const BinProblem *)nullptr, 1);
+    hipLaunchKernelGGL(chunk_count_kernel, dim3(nch), dim3(kCountThreads), sizeof(uint32_t) * nbins, s,
+                       pr);
+    hipLaunchKernelGGL(chunk_scan_kernel, dim3((nbins + kScanDigits - 1) / kScanDigits),
+                       dim3(kScanDigits * kChunkScanSegs), 0, s, pr);
   }
   if (!pr.fused) {
     // tile starts and the subproblem list need only the counts
@@ -952,16 +1077,14 @@ static hipError_t sort_points_one_pass(const PointArgs &pa, const Geom &g, int d
   if (n > 0) {
     size_t lds = sizeof(uint16_t) * (size_t)kOneWaves * nbins;
     if (pr.fused) lds = std::max(lds + sizeof(uint32_t) * nbins, sizeof(SubLds<kOneThreads>));
-    hipError_t e = set_scatter_lds(rec != nullptr, false, lds);
+    hipError_t e = set_lds(rec ? (const void *)chunk_scatter_kernel<true>
+                               : (const void *)chunk_scatter_kernel<false>, lds);
     if (e != hipSuccess) return e;
     const int blocks = nch + (pr.fused ? 1 : 0);
     if (rec)
-      hipLaunchKernelGGL((chunk_scatter_kernel<true, false>), dim3(blocks), dim3(kOneThreads), lds,
-                         s, pr, (const BinProblem *)nullptr, 1);
+      hipLaunchKernelGGL(chunk_scatter_kernel<true>, dim3(blocks), dim3(kOneThreads), lds, s, pr);
     else
-      hipLaunchKernelGGL((chunk_scatter_kernel<false, false>), dim3(blocks), dim3(kOneThreads),
-                         lds, s, pr, (const BinProblem *)nullptr, 1);
-    if (pr.cls.ncls > 0) launch_class_sort(pr, n, nbins, sb.max_sub, s);
+      hipLaunchKernelGGL(chunk_scatter_kernel<false>, dim3(blocks), dim3(kOneThreads), lds, s, pr);
   }
   return hipGetLastError();
 }
@@ -970,19 +1093,17 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
   if (nprob <= 0) return hipSuccess;
   uint32_t chunks = 0, scans = 0, pieces = 0;
   int max_bins = 1;
-  bool rec = probs[0].out.r != nullptr;
   for (int i = 0; i < nprob; ++i) {
     BinProblem &pr = probs[i];
-    if (!sort_one_pass(pr.nbins) || (pr.out.r != nullptr) != rec) return hipErrorInvalidValue;
-    pr.bits = key_bits(pr.nbins);
-    pr.nchunks = (int)((pr.pa.num_points + kOneChunk - 1) / kOneChunk);
+    if (!tile_binning(pr.nbins) || pr.cls.ncls == 0) return hipErrorInvalidValue;
+    pr.chunk = tile_chunk(pr.pa.num_points);
+    pr.nchunks = tile_chunks(pr.pa.num_points);
     pr.chunk0 = chunks;
     pr.scan0 = scans;
     pr.piece0 = pieces;
-    if (pr.cls.ncls > 0)
-      pieces += (uint32_t)class_pieces(pr.pa.num_points, pr.nbins, pr.max_sub);
+    pieces += (uint32_t)class_pieces(pr.pa.num_points, pr.nbins, pr.max_sub);
     chunks += (uint32_t)pr.nchunks;
-    if (pr.pa.num_points > 0) scans += (uint32_t)((pr.nbins + kScanDigits - 1) / kScanDigits);
+    scans += (uint32_t)((pr.nbins + kScanDigits - 1) / kScanDigits);
     max_bins = std::max(max_bins, pr.nbins);
   }
   for (int first = 0; first < nprob; first += kBinTableChunk) {
@@ -992,37 +1113,23 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
     for (int i = 0; i < chunk.count; ++i) chunk.probs[i] = probs[first + i];
     hipLaunchKernelGGL(bin_table_kernel, dim3(1), dim3(64), 0, s, chunk, table);
   }
-  const BinProblem none{};
-  if (chunks > 0) {
-    hipLaunchKernelGGL(chunk_count_kernel<true>, dim3(chunks), dim3(kCountThreads),
-                       sizeof(uint32_t) * max_bins, s, none, (const BinProblem *)table, nprob);
-    if (scans > 0)
-      hipLaunchKernelGGL(chunk_scan_kernel<true>, dim3(scans), dim3(kScanDigits * kChunkScanSegs),
-                         0, s, none, (const BinProblem *)table, nprob);
-  }
-  hipLaunchKernelGGL(subproblems_batched_kernel, dim3(nprob), dim3(kSubThreads), 0, s,
-                     (const BinProblem *)table);
-  if (chunks > 0) {
-    const size_t lds = sizeof(uint16_t) * (size_t)kOneWaves * max_bins;
-    hipError_t e = set_scatter_lds(rec, true, lds);
-    if (e != hipSuccess) return e;
-    if (rec)
-      hipLaunchKernelGGL((chunk_scatter_kernel<true, true>), dim3(chunks), dim3(kOneThreads), lds,
-                         s, none, (const BinProblem *)table, nprob);
-    else
-      hipLaunchKernelGGL((chunk_scatter_kernel<false, true>), dim3(chunks), dim3(kOneThreads), lds,
-                         s, none, (const BinProblem *)table, nprob);
-  }
-  if (pieces > 0)
-    hipLaunchKernelGGL(class_sort_kernel, dim3(pieces), dim3(kClsThreads), 0, s, none,
-                       (const BinProblem *)table, nprob);
-  return hipGetLastError();
+  return launch_tile_binning(BinProblem{}, table, nprob, max_bins, chunks, scans, pieces, s);
 }
 
 hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBuffers &sb,
                        hipStream_t s, const RecordOut *rec) {
-  if (sort_one_pass(sb.nbins)) return sort_points_one_pass(pa, g, dim, sb, s, rec);
   const int64_t n = pa.num_points;
+  if (rec && sb.cls.ncls > 0 && n > 0 && tile_binning(sb.nbins)) {
+    BinProblem pr = bin_problem(pa, g, dim, sb, rec);
+    pr.chunk = tile_chunk(n);
+    pr.nchunks = tile_chunks(n);
+    // the totals of a single chunk are its counts
+    uint32_t scans = (uint32_t)((sb.nbins + kScanDigits - 1) / kScanDigits);
+    if (pr.nchunks == 1) pr.tot = pr.cnt, scans = 0;
+    return launch_tile_binning(pr, nullptr, 1, sb.nbins, (uint32_t)pr.nchunks, scans,
+                               (uint32_t)class_pieces(n, sb.nbins, sb.max_sub), s);
+  }
+  if (sort_one_pass(sb.nbins)) return sort_points_one_pass(pa, g, dim, sb, s, rec);
   // with records, the last pass writes rec->out; earlier ones alternate with tmp
   auto dst = [&](int q) { return ((sb.passes - 1 - q) & 1) == 0 ? rec->out : rec->tmp; };
   if (n > 0) {
@@ -1044,9 +1151,10 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
         rm.pa = pa;
         rm.g = g;
         rm.first = p == 0;
+        rm.last = p == sb.passes - 1;
         rm.vmax = p == 0 && rec->values && sb.cls.ncls > 0 ? sb.cls.vmax : nullptr;
         hipLaunchKernelGGL(scatter_kernel<true>, dim3(sb.nchunks), dim3(kSortThreads), 0, s,
-                           sb.keys[0], (const uint32_t *)nullptr, (uint32_t *)nullptr,
+                           sb.keys[0], (const uint32_t *)nullptr, sb.keys[1],
                            (uint32_t *)nullptr, n, p * kRadixBits, sb.cnt, sb.scan_tmp,
                            sb.nchunks, rm);
       } else {
@@ -1057,7 +1165,7 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
       }
     }
   }
-  const KeySrc sorted{sb.keys[sb.passes & 1], rec ? rec->out.r : nullptr};
+  const KeySrc sorted{rec ? sb.keys[1] : sb.keys[sb.passes & 1], nullptr};
   int nb1 = sb.nbins + 1;
   const int3 nb = dim == 3 ? make_int3(g.nbin[0], g.nbin[1], g.nbin[2]) : make_int3(1, 1, 1);
   hipLaunchKernelGGL(bounds_kernel, dim3((nb1 + 255) / 256), dim3(256), 0, s, sorted, n,
@@ -1065,15 +1173,9 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
   hipLaunchKernelGGL(subproblems_kernel, dim3(1), dim3(kSubThreads), 0, s, sb.bin_start,
                      (const uint32_t *)nullptr, 0, sb.nbins, nb, sb.along_x, sb.max_sub, sb.sub_work,
                      sb.sub_ofs + sb.nbins, sb.subs);
-  if (n > 0 && rec && sb.cls.ncls > 0) {
-    BinProblem pr{};
-    pr.g = g;
-    pr.out = rec->out;
-    pr.nsub = sb.sub_ofs + sb.nbins;
-    pr.subs = sb.subs;
-    pr.cls = sb.cls;
-    launch_class_sort(pr, n, sb.nbins, sb.max_sub, s);
-  }
+  if (n > 0 && rec && sb.cls.ncls > 0)
+    hipLaunchKernelGGL(class_sort_kernel, dim3(class_pieces(n, sb.nbins, sb.max_sub)), dim3(kClsThreads),
+                       0, s, bin_problem(pa, g, dim, sb, rec), (const BinProblem *)nullptr, 1);
   return hipGetLastError();
 }
 

@@ -440,15 +440,14 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
   const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
 
   const uint32_t *perm = pa.cperm;
-  const float2 *vals = (const float2 *)zr.r + 2;  // point p's value: vals[4 p]
   Rounds ahead(r, pa);
   float4 ra;
   float2 cv = make_float2(0.f, 0.f);
   // the staging roles move round the waves (SIMDs) from round to round
   int role = wave;
   uint32_t np = perm[ahead.pos(staged_point(role, lane))];
-  ra = zr.r[2 * (int64_t)np];
-  if (role >= 2) cv = vals[4 * (int64_t)np];
+  ra = zr.r[np];
+  if (role >= 2) cv = zr.v[np];
   ahead.advance();
   np = perm[ahead.pos(staged_point((role + 1) & 3, lane))];
   ClassWalk cw(r, pa);
@@ -462,8 +461,8 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
       spread_stage<W>(sh, role, lane, npts, ra, make_float2(cv.x * s_in, cv.y * s_in), poly, t);
       __syncthreads();
       role = (role + 1) & 3;
-      ra = zr.r[2 * (int64_t)np];
-      if (role >= 2) cv = vals[4 * (int64_t)np];
+      ra = zr.r[np];
+      if (role >= 2) cv = zr.v[np];
       ahead.advance();
       np = perm[ahead.pos(staged_point((role + 1) & 3, lane))];
       spread_products<W>(acc, sh, (npts + 31) >> 5, t, wave, i16, g4);
@@ -763,14 +762,13 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
   if (r.begin >= r.end) return;
 
   const uint32_t *perm = pa.cperm;
-  const uint32_t *idx = (const uint32_t *)zr.r + 7;  // point p's input index: idx[8 p]
   Rounds ahead(r, pa);
   uint32_t np = perm[ahead.pos(lane)];
-  float4 ra = zr.r[2 * (int64_t)np];
+  float4 ra = zr.r[np];
   // staging roles (0 x, 1 y, 2 z, 3 writes the outputs) move round the waves
   int role = wave;
   uint32_t j = 0, jn = 0;
-  if (role == 3) jn = idx[8 * (int64_t)np];
+  if (role == 3) jn = zr.i[np];
   ahead.advance();
   np = perm[ahead.pos(lane)];
 
@@ -816,8 +814,8 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
       __syncthreads();
       const bool writer = role == 3;
       role = (role + 1) & 3;
-      ra = zr.r[2 * (int64_t)np];
-      if (role == 3) jn = idx[8 * (int64_t)np];
+      ra = zr.r[np];
+      if (role == 3) jn = zr.i[np];
       ahead.advance();
       np = perm[ahead.pos(lane)];
       for (int gi = 0; gi < (npts + 15) >> 4; ++gi) {
@@ -901,12 +899,13 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
   const uint32_t *perm = pa.cperm;
   Rounds ahead(r, pa);
   uint32_t np = perm[ahead.pos(lane)];
-  float4 ra = zr.r[2 * (int64_t)np];
+  float4 ra = zr.r[np];
   // staging roles (0 x, 1 y, 2 z values, 3 z derivatives) move round the
   // waves; role 2 also writes the outputs
   int role = wave;
-  float4 rb = make_float4(0.f, 0.f, 0.f, 0.f), rbn = rb;  // writer: (u, key, index)
-  if (role == 2) rbn = zr.r[2 * (int64_t)np + 1];
+  float2 u = make_float2(0.f, 0.f), un = u;  // writer: the point's u and index
+  uint32_t j = 0, jn = 0;
+  if (role == 2) un = zr.v[np], jn = zr.i[np];
   ahead.advance();
   np = perm[ahead.pos(lane)];
 
@@ -945,7 +944,8 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
           interp_stage_y<W, false>(WY + p * kIRowY, ok, ra.y, s, &dpoly->p.c[0][0]);
           interp_stage_y<W, true>(DY + p * kIRowY, ok, ra.y, s, &dpoly->p.dc[0][0]);
         } else if (role == 2) {
-          rb = rbn;
+          u = un;
+          j = jn;
           interp_stage_z<W, false>(BH + p * kIRow, BL + p * kIRow, ok, ra.z, ((off >> 16) & 255) + oz,
                                    &dpoly->op[0][0]);
         } else {
@@ -956,8 +956,8 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
       __syncthreads();
       const bool writer = role == 2;
       role = (role + 1) & 3;
-      ra = zr.r[2 * (int64_t)np];
-      if (role == 2) rbn = zr.r[2 * (int64_t)np + 1];
+      ra = zr.r[np];
+      if (role == 2) un = zr.v[np], jn = zr.i[np];
       ahead.advance();
       np = perm[ahead.pos(lane)];
       for (int gi = 0; gi < (npts + 15) >> 4; ++gi) {
@@ -1024,16 +1024,15 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
       }
       __syncthreads();
       if (writer && ok) {
-        const uint32_t j = __float_as_uint(rb.w);
         float sv[6];
 #pragma unroll
         for (int c = 0; c < 6; ++c)
           sv[c] = ((RED[0][c][lane] + RED[1][c][lane]) + (RED[2][c][lane] + RED[3][c][lane])) * s_out *
                   (c < 4 ? kProdUnscale : kProdUnscaleD);
         // Re(conj(u) * (-s) * S) = -s (u.x S.x + u.y S.y)
-        gx[j] = -(float)g.scale[0] * (rb.x * sv[0] + rb.y * sv[1]);
-        if (gy) gy[j] = -(float)g.scale[1] * (rb.x * sv[2] + rb.y * sv[3]);
-        if (gz) gz[j] = -(float)g.scale[2] * (rb.x * sv[4] + rb.y * sv[5]);
+        gx[j] = -(float)g.scale[0] * (u.x * sv[0] + u.y * sv[1]);
+        if (gy) gy[j] = -(float)g.scale[1] * (u.x * sv[2] + u.y * sv[3]);
+        if (gz) gz[j] = -(float)g.scale[2] * (u.x * sv[4] + u.y * sv[5]);
       }
     }
   } while (cw.next());

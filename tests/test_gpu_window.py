@@ -1,5 +1,5 @@
 """Matrix-core window kernels against the vector-ALU kernels at the sizes
-where rounds, groups, classes and subproblems end.
+where rounds, groups, classes, chunks and subproblems end.
 
 Both kernel families form the same FP32 sums and share the FFT.  A point's
 weight is a product of three tap values; each is a polynomial in FP32 (a few
@@ -66,3 +66,24 @@ def test_window_kernels_match_vector_kernels(dev, w, case):
         a, b = a.to("cpu", torch.complex128), b.to("cpu", torch.complex128)
         err = float(torch.linalg.norm(a - b) / torch.linalg.norm(b))
         assert err <= tol, (case, w, err)
+
+
+def test_many_tiles(dev):
+    """More tiles than the stable one-pass binning takes (9216), up to the
+    tile binning's 16384: the same sums as the vector-ALU kernels."""
+    import torch
+    import apollofft_amd as A
+    n, w, M = (120, 116, 120), 8, 20_000
+    rng = np.random.default_rng(9)
+    x = torch.from_numpy(rng.uniform(0, 1, (M, 3)).astype(np.float32)).to(dev)
+    c = torch.from_numpy((rng.standard_normal((M, 2)) @ [1, 1j]).astype(np.complex64)).to(dev)
+    f = torch.from_numpy((rng.standard_normal(n + (2,)) @ [1, 1j]).astype(np.complex64)).to(dev)
+    out = {}
+    for method in ("mfma", "valu"):
+        p = A.NufftPlan3D(*n, *[1.0 / k for k in n], 2, w, kernel_method=method, grid_policy="exact")
+        if method == "mfma":
+            assert 9216 < np.prod([-(-a // b) for a, b in zip(p.meta["m"], p.meta["bin_size"])]) <= 16384
+        out[method] = (p.type1(x, c), p.type2(x, f))
+    for a, b in zip(out["mfma"], out["valu"]):
+        a, b = a.to("cpu", torch.complex128), b.to("cpu", torch.complex128)
+        assert float(torch.linalg.norm(a - b) / torch.linalg.norm(b)) <= TOL
