@@ -244,11 +244,12 @@ __device__ __forceinline__ void load_lines(const FftPass &p, const int64_t *lbas
 }
 
 // LDS lines to the output: kept modes, Bluestein chirp, conjugation for the
-// inverse, scale and deconvolution (DEC), and the bin maxima (bm != null).
+// inverse, scale and deconvolution (DEC).  Returns the thread's largest
+// |re|, |im| written.
 template <bool DEC, int NT>
-__device__ __forceinline__ void store_lines(const FftPass &p, const int64_t *lbase, int nl,
-                                            uint32_t mag_nl, int Lf, bool blue, const float2 *src,
-                                            uint32_t *bm, int nbz) {
+__device__ __forceinline__ float store_lines(const FftPass &p, const int64_t *lbase, int nl,
+                                             uint32_t mag_nl, int Lf, bool blue, const float2 *src) {
+  float mx = 0.f;
   const bool contig = p.out_si == 1;
   const int n = nl * p.nout;
   for (int base = threadIdx.x; base < n; base += NT * kLoadBatch) {
@@ -272,11 +273,10 @@ __device__ __forceinline__ void store_lines(const FftPass &p, const int64_t *lba
       v.x *= s;
       v.y *= s;
       p.out[lbase[p.lb + li] + (int64_t)o * p.out_si] = v;
-      if (bm)
-        atomicMax(&bm[li * nbz + fdiv(o, p.bm_bin[2], p.mag_bmz)],
-                  __float_as_uint(fmaxf(fabsf(v.x), fabsf(v.y))));
+      mx = fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y)));
     }
   }
+  return mx;
 }
 
 template <int NT>
@@ -293,9 +293,8 @@ __global__ __launch_bounds__(NT) void fft_pass_kernel(FftPass p) {
   // input lines (their latency overlaps the line set-up and loads)
   const float2 tw0 = p.tw[min((int)threadIdx.x, Lf - 1)];
   const float2 tw1 = p.tw[min((int)threadIdx.x + NT, Lf - 1)];
-  if (p.zero)
-    for (int i = blockIdx.x * NT + threadIdx.x; i < p.zero_n; i += gridDim.x * NT)
-      p.zero[i] = 0.f;
+  if (p.zero && blockIdx.x == 0 && threadIdx.x < kMaxSlots)
+    p.zero[threadIdx.x * kMaxStride] = 0.f;
   const int64_t l0 = (int64_t)blockIdx.x * lb;
   const int nl = (int)((p.nlines - l0) < lb ? (p.nlines - l0) : lb);
   const uint32_t mag_nl = nl == lb ? p.mag_lb : p.mag_last;  // nl < lb only in the last block
@@ -343,25 +342,19 @@ __global__ __launch_bounds__(NT) void fft_pass_kernel(FftPass p) {
   __syncthreads();
 
   // ---- store (crop, conjugation, scale and deconvolution) ----
-  // with bin maxima: per (line, z bin) maxima in LDS (the free buffer; non-
-  // negative floats order like their bit patterns), then one global atomic
-  // maximum per (line, bin)
-  uint32_t *bm = (uint32_t *)dst;
-  const int nbz = p.bmax ? p.bm_nbin[2] : 0;
-  if (p.bmax) {
-    for (int i = threadIdx.x; i < nl * nbz; i += NT) bm[i] = 0u;
+  const float mx = p.dec_out ? store_lines<true, NT>(p, lbase, nl, mag_nl, Lf, blue, src)
+                             : store_lines<false, NT>(p, lbase, nl, mag_nl, Lf, blue, src);
+  if (p.vmax) {  // (non-negative floats order like their bit patterns)
+    float m = mx;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    float *red = (float *)dst;  // the free buffer
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-  }
-  uint32_t *bmx = p.bmax ? bm : nullptr;
-  if (p.dec_out) store_lines<true, NT>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
-  else store_lines<false, NT>(p, lbase, nl, mag_nl, Lf, blue, src, bmx, nbz);
-  if (p.bmax) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < nl * nbz; i += NT) {
-      const int li = i / nbz, zb = i - li * nbz;
-      const int64_t l = l0 + li, x = l / p.nb, y = l - x * p.nb;
-      const int64_t bin = ((x / p.bm_bin[0]) * p.bm_nbin[1] + y / p.bm_bin[1]) * p.bm_nbin[2] + zb;
-      atomicMax((uint32_t *)p.bmax + bin, bm[i]);
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int w = 1; w < NT / 64; ++w) m = fmaxf(m, red[w]);
+      atomicMax((uint32_t *)p.vmax + (blockIdx.x % kMaxSlots) * kMaxStride, __float_as_uint(m));
     }
   }
 }
@@ -391,7 +384,6 @@ hipError_t launch_fft_pass(const FftPass &pass, hipStream_t s) {
   FftPass p = pass;
   p.mag_nin = div_magic(p.nin);
   p.mag_nout = div_magic(p.nout);
-  p.mag_bmz = div_magic(p.bmax ? p.bm_bin[2] : 1);
   p.mag_lb = div_magic(p.lb);
   p.mag_last = div_magic(p.nlines - (p.nlines - 1) / p.lb * p.lb);
   p.use_mag_nb = p.nlines < ((int64_t)1 << 31) &&

@@ -101,20 +101,26 @@ constexpr uint32_t kSubWork = 48;
 constexpr int kMaxCls = 16;
 constexpr int kClassSub = 4096;  // points of a tile listed by class at once
 
+// A maximum over a launch (strengths, fine grid) is kept in slots, a line of
+// memory each, over which workgroups spread their maxima: thousands of atomics
+// to one line are done one after another (the FFT passes and binning of a
+// gradient step at 64^3: 865 us a step with one line, 804 with 64).
+constexpr int kMaxSlots = 64, kMaxStride = 16;
+
 // The class list of a binning (sort.hip, class_sort_kernel).
 struct ClassBuffers {
   int ncls = 0;      // 0: no class list
   int cw = 1;
   uint32_t *perm;    // list order -> sorted position: a subproblem's points by class and x offset
   uint16_t *start;   // per subproblem: first entry of each class in its part of the list
-  uint32_t *vmax;    // bits of the largest |re|, |im| of the values
+  uint32_t *vmax;    // bits of the largest |re|, |im| of the values (kMaxSlots slots)
 };
 
 struct SortBuffers {
   uint32_t *keys[2];
   uint32_t *idx[2];
   uint32_t *cnt;       // per-chunk digit (one-pass: tile) counts, then offsets
-  uint32_t *scan_tmp;  // digit (one-pass: tile) totals; [nbins] ClassBuffers::vmax
+  uint32_t *scan_tmp;  // digit (one-pass: tile) totals
   uint32_t *bin_start; // nbins + 1
   uint32_t *sub_ofs;   // nbins + 2; [nbins] = number of subproblems, [nbins + 1] = total work
   int4 *subs;          // (bin, start, count, work before it)
@@ -151,23 +157,18 @@ struct FftPass {
   int blue_n;
   const float2 *chirp;   // exp(-i pi n^2 / L), n in [0, L)
   const float2 *bhat;    // FFT_blue_n of the conjugate chirp filter, times 1/blue_n
-  // Bin maxima of the written grid (the last pass of a 3D Type-2, lines
-  // (a, b) = (x, y), output index = z): bmax[bin] = max |re|, |im| over the
-  // bin's cells, with bins of bm_bin cells (bm_nbin per axis); zero[0 ..
-  // zero_n) is cleared by the pass before (the first pass of the chain).
-  float *bmax;
-  int bm_bin[3];
-  int bm_nbin[3];
+  // Largest |re|, |im| written (the last pass of a 3D Type-2), as the maximum
+  // over kMaxSlots slots; zero: slots cleared by this pass (the first).
+  float *vmax;
   float *zero;
-  int zero_n;
   // Division by the pass's runtime divisors as multiply-high by
   // ceil(2^32 / d) (0 for d = 1), set by launch_fft_pass: nin, nout, the
-  // z bin width of the bin maxima, the lines of a full and of the last
+  // lines of a full and of the last
   // block, and per stage f the butterflies per line Lf / fac[f] and the
   // stage span Ns (product of fac[0 .. f-1]); the twiddle step of stage f,
   // Lf / (Ns fac[f]).  mag_nb: the line index split l / nb, used when
   // nlines * nb < 2^32 (use_mag_nb), else the kernel divides in 64 bits.
-  uint32_t mag_nin, mag_nout, mag_bmz, mag_lb, mag_last, mag_nb;
+  uint32_t mag_nin, mag_nout, mag_lb, mag_last, mag_nb;
   int use_mag_nb;
   uint32_t mag_nbf[16], mag_ns[16];
   int twstep[16];
@@ -309,16 +310,12 @@ hipError_t launch_win_spread_batched(int w, const SpreadProblem *host_probs, int
                                      const WinPoly *dpoly, int num_blocks, hipStream_t s);
 int win_interp_groups(int w, int64_t num_points, int cus);
 int win_grad_groups(int w, int64_t num_points, int cus);
-// Tile maxima from the bin maxima the last FFT pass wrote (FftPass::bmax):
-// the scales of the interpolation and gradient windows of class geometry
-// (ncls, cw).
-hipError_t launch_win_tile_max(int w, const float *bmax, float *tmax, const Geom &g, int ncls,
-                               int cw, hipStream_t s);
+// gmax: the grid's kMaxSlots maxima (FftPass::vmax), the scale of the windows.
 hipError_t launch_win_interp(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
-                             const float *tmax, float2 *out, const Geom &g, const WinPoly *dpoly,
+                             const float *gmax, float2 *out, const Geom &g, const WinPoly *dpoly,
                              int num_blocks, hipStream_t s);
 hipError_t launch_win_grad(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
-                           const float *tmax, float *gx, float *gy, float *gz, const Geom &g,
+                           const float *gmax, float *gx, float *gy, float *gz, const Geom &g,
                            const WinPoly *dpoly, int num_blocks, hipStream_t s);
 
 // Direct FP64 sums (direct.hip): type 1 writes every mode, type 2 every point.

@@ -187,7 +187,7 @@ struct StageTimer {
 
 struct Layout {
   size_t keys0 = 0, keys1 = 0, idx0 = 0, idx1 = 0, cnt = 0, scan = 0, bin_start = 0,
-         sub_ofs = 0, subs = 0, rec = 0, xo = 0, zrec = 0, zrec2 = 0, tmax = 0, grid = 0, fftbuf = 0,
+         sub_ofs = 0, subs = 0, rec = 0, xo = 0, zrec = 0, zrec2 = 0, gmax = 0, grid = 0, fftbuf = 0,
          total = 0;
   int nchunks = 0;
 };
@@ -292,7 +292,7 @@ Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
     if (p->dim != 3 || p->kernel_method != kSpreadMfma) cnt_n = std::max(cnt_n, one_n);
     l.cnt = take(4 * cnt_n);
     const bool classes = p->dim == 3 && p->kernel_method == kSpreadMfma;
-    l.scan = take(4 * (size_t)(std::max(kRadix, nb) + 1));  // digit (or tile) totals, value maximum
+    l.scan = take(4 * (size_t)std::max(kRadix, nb));  // digit (or tile) totals
     l.bin_start = take(4 * (size_t)(nb + 1));
     l.sub_ofs = take(4 * (size_t)(nb + 2));  // (nb unused,) list totals
     int64_t nsub = 1;
@@ -310,7 +310,7 @@ Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
       // of the subproblems (2 bytes each, at most 16 a point).  The class list
       // itself takes the place of the permutation, which the records replace.
       l.zrec2 = take(std::max(32 * Mp, 4 * one_n));
-      l.tmax = take(2 * sizeof(float) * (size_t)(p->bi.nbins + 1));  // bin and tile maxima
+      l.gmax = take(sizeof(float) * kMaxSlots * kMaxStride);  // maxima: grid, values
     } else {
       l.rec = take(sizeof(float) * (size_t)point_rec_floats(p->w) * Mp);
       l.xo = take(Mp);
@@ -813,25 +813,19 @@ struct Exec {
                                  blocks(p->bf, pa.num_points, 2), s);
     });
   }
-  // Bin maxima, then tile maxima, of the fine grid (matrix-core kernels).
-  float *bmax() const { return (float *)(ws + lay.tmax); }
-  float *tmax() const { return bmax() + p->bi.nbins; }
-  // The fine grid of `modes` (this workspace), with the tile maxima the
+  // Largest component of the fine grid (matrix-core kernels).
+  float *gmax() const { return (float *)(ws + lay.gmax); }
+  // The fine grid of `modes` (this workspace), with the maximum the
   // matrix-core interpolation and gradient scale by.
   hipError_t fine_grid(const float2 *modes, bool compat) const {
-    const bool mf = p->kernel_method == kSpreadMfma;
-    hipError_t e = timed(ANUFFT_STAGE_FFT, [&] { return modes_to_grid(modes, compat, mf); });
-    if (e != hipSuccess || !mf) return e;
-    return timed(ANUFFT_STAGE_TILE_MAX, [&] {
-      return launch_win_tile_max(p->w, bmax(), tmax(), p->bi.g, p->bi.ncls, p->bi.cw, s);
-    });
+    return timed(ANUFFT_STAGE_FFT, [&] { return modes_to_grid(modes, compat); });
   }
   // Type-2 interpolation and coordinate gradient of binned points from the
   // fine grid in `from`'s workspace.
   hipError_t interp3(const PointArgs &pa, const Exec &from, float2 *out) const {
     return timed(ANUFFT_STAGE_INTERP, [&] {
       if (p->kernel_method == kSpreadMfma)
-        return launch_win_interp(p->w, pa, zrec(pa.num_points), from.grid(), from.tmax(), out, p->bi.g,
+        return launch_win_interp(p->w, pa, zrec(pa.num_points), from.grid(), from.gmax(), out, p->bi.g,
                                  p->d_poly, blocks(p->bi, pa.num_points, win_interp_groups(p->w, pa.num_points, p->cus)), s);
       return launch_interp3d(p->w, pa, from.grid(), out, p->bi.g, p->poly,
                              blocks(p->bi, pa.num_points, 4), s);
@@ -840,7 +834,7 @@ struct Exec {
   hipError_t grad3(const PointArgs &pa, const Exec &from, const float2 *u, float *const g[3]) const {
     return timed(ANUFFT_STAGE_GRAD, [&] {
       if (p->kernel_method == kSpreadMfma)
-        return launch_win_grad(p->w, pa, zrec(pa.num_points), from.grid(), from.tmax(), g[0], g[1], g[2],
+        return launch_win_grad(p->w, pa, zrec(pa.num_points), from.grid(), from.gmax(), g[0], g[1], g[2],
                                p->bi.g, p->d_poly, blocks(p->bi, pa.num_points, win_grad_groups(p->w, pa.num_points, p->cus)), s);
       return launch_grad3d(p->w, pa, from.grid(), u, g[0], g[1], g[2], p->bg.g, p->poly,
                            blocks(p->bg, pa.num_points, 4), s);
@@ -876,7 +870,7 @@ struct Exec {
       c.cw = b.cw;
       c.perm = sb.idx[0];
       c.start = (uint16_t *)(ws + lay.zrec2);
-      c.vmax = sb.scan_tmp + b.nbins;
+      c.vmax = (uint32_t *)gmax() + 1;  // beside the grid's slots
     }
     return sb;
   }
@@ -932,10 +926,9 @@ struct Exec {
     return launch_fft_pass(fx, s);
   }
 
-  // T2 modes -> grid: deconvolve, zero pad, inverse passes x, y, z.  With
-  // bin_max (3D, MFMA interpolation) the passes also leave the bin maxima
-  // of the grid in the first half of the tile-maximum scratch.
-  hipError_t modes_to_grid(const float2 *modes, bool compat, bool bin_max = false) const {
+  // T2 modes -> grid: deconvolve, zero pad, inverse passes x, y, z (matrix-core
+  // plans in 3D: and the largest component of the grid).
+  hipError_t modes_to_grid(const float2 *modes, bool compat) const {
     const int64_t mx = p->m[0], my = p->m[1], mz = p->m[2];
     const int64_t nx = p->n[0], ny = p->n[1], nz = p->n[2];
     float2 *g = grid(), *c = fftbuf();
@@ -948,12 +941,8 @@ struct Exec {
     // x: modes[nx][ny][nz] -> b[mx][ny][nz] (in the grid buffer)
     FftPass fx = make_pass(p, 0, modes, g, (int)nx, (int)mx, ny, nz, nz, 1, ny * nz, nz, 1, ny * nz,
                            true, 1.0);
-    const bool bm = bin_max && p->kernel_method == kSpreadMfma;
-    float *bmax = bm ? (float *)(ws + lay.tmax) : nullptr;
-    if (bm) {
-      fx.zero = bmax;
-      fx.zero_n = p->bi.nbins;
-    }
+    const bool mf = p->kernel_method == kSpreadMfma;
+    if (mf) fx.zero = gmax();
     if ((e = launch_fft_pass(fx, s)) != hipSuccess) return e;
     // y: b[mx][ny][nz] -> c[mx][my][nz]
     FftPass fy = make_pass(p, 1, g, c, (int)ny, (int)my, mx, nz, ny * nz, 1, nz, my * nz, 1, nz,
@@ -962,13 +951,7 @@ struct Exec {
     // z: c[mx][my][nz] -> grid[mx][my][mz]
     FftPass fz = make_pass(p, 2, c, g, (int)nz, (int)mz, mx, my, my * nz, nz, 1, my * mz, mz, 1,
                            true, scale);
-    if (bm) {
-      fz.bmax = bmax;
-      for (int a = 0; a < 3; ++a) {
-        fz.bm_bin[a] = p->bi.g.bin[a];
-        fz.bm_nbin[a] = p->bi.g.nbin[a];
-      }
-    }
+    if (mf) fz.vmax = gmax();
     return launch_fft_pass(fz, s);
   }
 };

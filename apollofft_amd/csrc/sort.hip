@@ -45,7 +45,7 @@ __global__ __launch_bounds__(kSortThreads) void keys_kernel(PointArgs pa, Geom g
                                                             uint32_t *keys, uint32_t *cnt,
                                                             int nchunks, uint32_t *vmax) {
   __shared__ uint32_t hist[kRadix];
-  if (vmax && blockIdx.x == 0 && threadIdx.x == 0) *vmax = 0u;
+  if (vmax && blockIdx.x == 0 && threadIdx.x < kMaxSlots) vmax[threadIdx.x * kMaxStride] = 0u;
   for (int d = threadIdx.x; d < kRadix; d += kSortThreads) hist[d] = 0;
   __syncthreads();
   int64_t base = (int64_t)blockIdx.x * kSortChunk;
@@ -444,14 +444,13 @@ __global__ __launch_bounds__(kSubThreads) void subproblems_kernel(uint32_t *bin_
 // Ties keep input order, so the result equals the LSD passes' (and
 // numpy.argsort(keys, kind="stable")).
 
-// Largest |component| of the values, as bits (non-negative floats order like
-// their bit patterns): one atomic per wave that raises it.
+// Largest |component| of a wave's values into the slot of its block, as bits
+// (non-negative floats order like their bit patterns).
 __device__ __forceinline__ void value_max(float mx, uint32_t *vmax) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  const uint32_t b = __float_as_uint(mx);
-  if ((threadIdx.x & 63) == 0 && b > __hip_atomic_load(vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-    atomicMax(vmax, b);
+  if ((threadIdx.x & 63) == 0)
+    atomicMax(vmax + (blockIdx.x % kMaxSlots) * kMaxStride, __float_as_uint(mx));
 }
 
 // Peers of this lane (lanes of the wave with the same key among `valid`
@@ -754,7 +753,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_count_kernel(BinProblem one
   const BinProblem &pr = tile_problem<BATCH, kTileCount>(one, table, nprob, chunk);
   const int nbins = pr.nbins;
   const PointArgs &pa = pr.pa;
-  if (chunk == 0 && threadIdx.x == 0) *pr.cls.vmax = 0u;
+  if (chunk == 0 && threadIdx.x < kMaxSlots) pr.cls.vmax[threadIdx.x * kMaxStride] = 0u;
   for (int d = threadIdx.x; d < nbins; d += kTileThreads) hist[d] = 0;
   const int64_t end = min(pa.num_points, (int64_t)(chunk + 1) * pr.chunk);
   int64_t j = (int64_t)chunk * pr.chunk + threadIdx.x;

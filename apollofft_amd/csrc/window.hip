@@ -109,7 +109,6 @@ __device__ __forceinline__ void split2(float a, float b, half2v &hi, half2v &lo)
 
 // Window of one class of a tile.
 struct WTile {
-  int bin;          // tile
   int xlo, y0, z0;  // grid cell of column 0, row 0, layer 0
   int o1;           // tile y offset of row 0's first tap
 };
@@ -119,7 +118,6 @@ __device__ __forceinline__ WTile win_tile(const Geom &g, int bin, int cls, int c
   const int bz = bin % g.nbin[2], t = bin / g.nbin[2];
   const int by = t % g.nbin[1], bx = t / g.nbin[1];
   WTile w;
-  w.bin = bin;
   w.o1 = 1 + cls * cw;
   w.xlo = bx * g.bin[0] - W + 1;
   w.y0 = by * g.bin[1] - W + w.o1;
@@ -412,10 +410,11 @@ __device__ __forceinline__ void spread_products(SpreadAcc<W> &acc, const char *s
   }
 }
 
-// Power-of-two scale of the strengths: e with max |c| 2^-e in [1/2, 1),
-// clamped so that both scales stay finite and normal.
-__device__ __forceinline__ int strength_exp(const uint32_t *vmax) {
-  const float mx = __uint_as_float(*vmax);
+// Power-of-two exponent of a maximum kept in slots: e with max 2^-e in
+// [1/2, 1), clamped so that the scale and its inverse stay finite and normal.
+__device__ __forceinline__ int max_exp(const float *slots, int lane) {
+  static_assert(kMaxSlots == 64, "a slot a lane");
+  const float mx = wave_max(slots[lane * kMaxStride]);
   int e = 0;
   if (mx > 0.f) (void)frexpf(mx, &e);
   return __builtin_amdgcn_readfirstlane(max(-120, min(120, e)));
@@ -436,7 +435,7 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
   for (int q = 0; q < WN::XW; ++q)
 #pragma unroll
     for (int b = 0; b < 4; ++b) acc[q][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int e = strength_exp(pa.vmax);
+  const int e = max_exp((const float *)pa.vmax, lane);
   const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
 
   const uint32_t *perm = pa.cperm;
@@ -540,64 +539,19 @@ __global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu<W>()) void win_spr
   }
 }
 
-// ---- tile maxima of the grid (scales of the interpolation windows) -----------
-//
-// bmax[b] = largest |re| or |im| over the cells of bin b (written by the last
-// FFT pass); tmax[b] = largest bmax over the bins that the windows of tile b
-// overlap, i.e. an upper bound of the largest component of those windows.
-//
-// Tile maxima: for the tile of bin b, the maximum of bmax over the bins that
-// meet its cells [b * bin + org, + ext) along each axis (periodic).  One
-// wave per tile: lanes 0-2 list the bins of one axis each in LDS, then the
-// lanes share the combinations.
-constexpr int kTileMaxList = 32;
-__device__ __forceinline__ int axis_bins(int b, int bw, int m, int org, int ext, int *out) {
-  int c = b * bw + org;
-  while (c < 0) c += m;
-  while (c >= m) c -= m;
-  int n = 0, left = ext;
-  while (left > 0 && n < kTileMaxList) {
-    const int bin = c / bw;
-    if (n == 0 || out[n - 1] != bin) out[n++] = bin;
-    const int step = min(left, min((bin + 1) * bw, m) - c);  // to the next bin or the grid end
-    left -= step;
-    c += step;
-    if (c >= m) c -= m;
-  }
-  return n;
-}
-
-__global__ __launch_bounds__(64) void tile_max_kernel(const float *bmax, Geom g, int3 org,
-                                                      int3 ext, float *tmax) {
-  __shared__ int lst[3][kTileMaxList];
-  __shared__ int cnt[3];
-  const int bin = blockIdx.x;
-  const int b3[3] = {bin / (g.nbin[2] * g.nbin[1]), (bin / g.nbin[2]) % g.nbin[1], bin % g.nbin[2]};
-  const int o3[3] = {org.x, org.y, org.z}, e3[3] = {ext.x, ext.y, ext.z};
-  if (threadIdx.x < 3) {
-    const int a = threadIdx.x;
-    cnt[a] = axis_bins(b3[a], g.bin[a], g.m[a], o3[a], e3[a], lst[a]);
-  }
-  __syncthreads();
-  const int nx = cnt[0], ny = cnt[1], nz = cnt[2];
-  float mx = 0.f;
-  for (int c = threadIdx.x; c < nx * ny * nz; c += 64) {
-    const int k = c % nz, j = (c / nz) % ny, i = c / (nz * ny);
-    mx = fmaxf(mx, bmax[((int64_t)lst[0][i] * g.nbin[1] + lst[1][j]) * g.nbin[2] + lst[2][k]]);
-  }
-  mx = wave_max(mx);
-  if (threadIdx.x == 0) tmax[bin] = mx;
-}
-
 // ---- interpolation and coordinate gradient -------------------------------------
 //
 // The window of the grid lives in registers as FP16 hi + lo A operands: lane
 // (i16, g4) of a wave holds ring row i16 (row y at y mod 16), z cells 8 g4 ..
 // 8 g4 + 7 of the window's 32, for each of the wave's x cells.  It is scaled
-// by the power of two of its tile's largest component (tile maxima), so rows
-// carry over while the window slides inside one tile; a new tile loads all
-// rows.  Only rows the window gains are loaded (the lanes of the others sit
-// the loads out).
+// by the power of two of the grid's largest component, which leaves 22 bits to
+// cells down to 2^-15 of it and an absolute 2^-37 of it below, far under the
+// rounding of the FFT that wrote the grid; so rows carry over while the window
+// slides along a pencil of tiles.  Only rows the window gains are loaded (the
+// lanes of the others sit the loads out).  (Scales of each tile's own maximum
+// took LDS atomics in the last FFT pass and a launch of their own: Type-2 of
+// 2e6 points, w = 7, 394 us and now 371, 200,000 ragged ones, w = 4, 113 and
+// 95.)
 constexpr int kIRow = 40;   // row stride (halves) of a staged point's z weights (32 cells)
 constexpr int kIRowY = 20;  // row stride (floats) of its y weights (16 ring rows)
 template <int W>
@@ -666,14 +620,6 @@ __device__ __forceinline__ float sum_groups(float a, float b) {
   const float s = __uint_as_float(h[0]) + __uint_as_float(h[1]);
   const uint2v r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Power-of-two exponent of a tile's largest component, clamped so that the
-// scale and its inverse stay finite and normal.
-__device__ __forceinline__ int tile_exp(float mx) {
-  int e = 0;
-  if (mx > 0.f) (void)frexpf(mx, &e);
-  return __builtin_amdgcn_readfirstlane(max(-120, min(120, e)));
 }
 
 // The x cells reached by each group of 16 of the staged points (cells_reached).
@@ -746,7 +692,7 @@ constexpr int interp_groups_per_cu() { return Win<W>::XW <= 4 ? 4 : 3; }
 
 template <int W>
 __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_interp_kernel(
-    PointArgs pa, ZRec zr, const float2 *grid, const float *tmax, float2 *out, Geom g,
+    PointArgs pa, ZRec zr, const float2 *grid, const float *gmax, float2 *out, Geom g,
     const WinPoly *__restrict__ dpoly) {
   using WN = Win<W>;
   using L = ILds<W>;
@@ -773,21 +719,17 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
   np = perm[ahead.pos(lane)];
 
   GridWin<W> win;
-  float s_in = 0.f, s_out = 0.f;
+  const int e = max_exp(gmax, lane);
+  const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
   ClassWalk cw(r, pa);
   WTile t{};
-  t.bin = -1;
+  bool open = false;
   do {
     const WTile n = win_tile<W>(g, cw.bin, cw.cls, pa.cw);
-    // rows carry over inside one tile (one scale), ascending classes
-    int first = 0;
-    if (n.bin == t.bin && n.y0 >= t.y0) first = 16 - min(16, n.y0 - t.y0);
+    // rows carry over along a pencil, ascending classes
+    const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
+    open = true;
     t = n;
-    if (first == 0) {
-      const int e = tile_exp(tmax[t.bin]);
-      s_in = ldexpf(kOpScale, -e);
-      s_out = ldexpf(kProdUnscale, e);
-    }
     if (first < 16) win.load(grid, g, t, first, s_in, wave, i16, g4);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
@@ -879,7 +821,7 @@ constexpr int grad_groups_per_cu() { return 2; }
 
 template <int W>
 __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_kernel(
-    PointArgs pa, ZRec zr, const float2 *grid, const float *tmax, float *gx, float *gy, float *gz,
+    PointArgs pa, ZRec zr, const float2 *grid, const float *gmax, float *gx, float *gy, float *gz,
     Geom g, const WinPoly *__restrict__ dpoly) {
   using WN = Win<W>;
   using L = ILds<W>;
@@ -910,21 +852,17 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
   np = perm[ahead.pos(lane)];
 
   GridWin<W> win;
-  float s_in = 0.f, s_out = 0.f;
+  const int e = max_exp(gmax, lane);
+  const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(1.0f, e);
   ClassWalk cw(r, pa);
   WTile t{};
-  t.bin = -1;
+  bool open = false;
   do {
     const WTile n = win_tile<W>(g, cw.bin, cw.cls, pa.cw);
-    // rows carry over inside one tile (one scale), ascending classes
-    int first = 0;
-    if (n.bin == t.bin && n.y0 >= t.y0) first = 16 - min(16, n.y0 - t.y0);
+    // rows carry over along a pencil, ascending classes
+    const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
+    open = true;
     t = n;
-    if (first == 0) {
-      const int e = tile_exp(tmax[t.bin]);
-      s_in = ldexpf(kOpScale, -e);
-      s_out = ldexpf(1.0f, e);
-    }
     if (first < 16) win.load(grid, g, t, first, s_in, wave, i16, g4);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
@@ -1076,26 +1014,10 @@ struct WinSpreadBatched {
 };
 
 template <int W>
-struct WinTileMax {
-  static hipError_t run(const float *bmax, float *tmax, const Geom &g, int ncls, int cw,
-                        hipStream_t s) {
-    const int3 org = make_int3(1 - W, 1 - W, -W);
-    const int3 ext = make_int3(Win<W>::PX, (ncls - 1) * cw + 16, 33);
-    // tile_max_kernel lists at most kTileMaxList bins per axis
-    if (ext.x / g.bin[0] + 2 > kTileMaxList || ext.y / g.bin[1] + 2 > kTileMaxList ||
-        ext.z / g.bin[2] + 2 > kTileMaxList)
-      return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tile_max_kernel, dim3(g.nbin[0] * g.nbin[1] * g.nbin[2]), dim3(64), 0, s, bmax,
-                       g, org, ext, tmax);
-    return hipGetLastError();
-  }
-};
-
-template <int W>
 struct WinInterp {
-  static hipError_t run(const PointArgs &pa, ZRec zr, const float2 *grid, const float *tmax,
+  static hipError_t run(const PointArgs &pa, ZRec zr, const float2 *grid, const float *gmax,
                         float2 *out, const Geom &g, const WinPoly *dpoly, int nblk, hipStream_t s) {
-    hipLaunchKernelGGL(win_interp_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, tmax,
+    hipLaunchKernelGGL(win_interp_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, gmax,
                        out, g, dpoly);
     return hipGetLastError();
   }
@@ -1103,10 +1025,10 @@ struct WinInterp {
 
 template <int W>
 struct WinGrad {
-  static hipError_t run(const PointArgs &pa, ZRec zr, const float2 *grid, const float *tmax,
+  static hipError_t run(const PointArgs &pa, ZRec zr, const float2 *grid, const float *gmax,
                         float *gx, float *gy, float *gz, const Geom &g, const WinPoly *dpoly,
                         int nblk, hipStream_t s) {
-    hipLaunchKernelGGL(win_grad_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, tmax, gx,
+    hipLaunchKernelGGL(win_grad_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, gmax, gx,
                        gy, gz, g, dpoly);
     return hipGetLastError();
   }
@@ -1159,19 +1081,15 @@ int win_spread_groups(int w, int64_t num_points, int cus) { return win_groups(0,
 int win_interp_groups(int w, int64_t num_points, int cus) { return win_groups(1, w, num_points, cus); }
 int win_grad_groups(int w, int64_t num_points, int cus) { return win_groups(2, w, num_points, cus); }
 
-hipError_t launch_win_tile_max(int w, const float *bmax, float *tmax, const Geom &g, int ncls,
-                               int cw, hipStream_t s) {
-  return dispatch_w<WinTileMax>(w, bmax, tmax, g, ncls, cw, s);
-}
 hipError_t launch_win_interp(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
-                             const float *tmax, float2 *out, const Geom &g, const WinPoly *dpoly,
+                             const float *gmax, float2 *out, const Geom &g, const WinPoly *dpoly,
                              int num_blocks, hipStream_t s) {
-  return dispatch_w<WinInterp>(w, pa, zr, grid, tmax, out, g, dpoly, num_blocks, s);
+  return dispatch_w<WinInterp>(w, pa, zr, grid, gmax, out, g, dpoly, num_blocks, s);
 }
 hipError_t launch_win_grad(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
-                           const float *tmax, float *gx, float *gy, float *gz, const Geom &g,
+                           const float *gmax, float *gx, float *gy, float *gz, const Geom &g,
                            const WinPoly *dpoly, int num_blocks, hipStream_t s) {
-  return dispatch_w<WinGrad>(w, pa, zr, grid, tmax, gx, gy, gz, g, dpoly, num_blocks, s);
+  return dispatch_w<WinGrad>(w, pa, zr, grid, gmax, gx, gy, gz, g, dpoly, num_blocks, s);
 }
 
 hipError_t launch_win_spread(int w, const PointArgs &pa, ZRec zr, float2 *grid, const Geom &g,
