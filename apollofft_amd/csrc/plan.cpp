@@ -185,6 +185,17 @@ struct StageTimer {
   }
 };
 
+// Memory that a plan keeps between its host-pointer calls: device buffers and
+// workspace, and pinned staging.  Allocating and freeing them took 70 of a
+// call's 405 us (32^3 modes, 100,000 points), copying from pageable memory
+// waits for each copy.  At most kArenaDev and kArenaPin bytes are kept, until
+// the plan is destroyed; a larger call frees its memory when it ends.
+struct HostArena {
+  char *dev = nullptr, *pin = nullptr;
+  size_t dev_bytes = 0, pin_bytes = 0;
+};
+constexpr size_t kArenaDev = (size_t)64 << 20, kArenaPin = (size_t)16 << 20;
+
 struct Layout {
   size_t keys0 = 0, keys1 = 0, idx0 = 0, idx1 = 0, cnt = 0, scan = 0, bin_start = 0,
          sub_ofs = 0, subs = 0, rec = 0, xo = 0, zrec = 0, zrec2 = 0, gmax = 0, grid = 0, fftbuf = 0,
@@ -238,6 +249,8 @@ struct anufft_plan {
   int lds_max = 163840; // gfx950 LDS per workgroup
   int kernel_method = kSpreadMfma;
   hipStream_t host_stream = nullptr;
+  mutable std::mutex arena_mu;  // held by the host call that uses the arena
+  mutable HostArena arena;
   // Second stream for the Type-2 FFT passes, which run concurrently with the
   // binning of the points (fork/join through the two events; the mutex keeps
   // concurrent callers from interleaving their record/wait pairs).
@@ -479,6 +492,8 @@ void destroy_plan(anufft_plan *p) {
       if (p->d_bhat[a]) (void)hipFree(p->d_bhat[a]);
     }
     if (p->d_poly) (void)hipFree(p->d_poly);
+    if (p->arena.dev) (void)hipFree(p->arena.dev);
+    if (p->arena.pin) (void)hipHostFree(p->arena.pin);
     if (p->host_stream) (void)hipStreamDestroy(p->host_stream);
     if (p->aux_stream) (void)hipStreamDestroy(p->aux_stream);
     if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
@@ -1206,7 +1221,7 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
     // The grid is zeroed before the binning: beside it, on the second stream,
     // the 2 us (64^3 cells) to 19 us (254^3) cost more in the fork and join,
     // about 25 us.  Not so right after the copies of a host call, where the
-    // fork costs nothing (the call: 403 us with it, 458 without).
+    // fork costs nothing (the call: 246 us with it, 254 without).
     if (blocks) {
       e = ex.fork_join(fill, bin);
     } else {
@@ -1768,38 +1783,66 @@ float f16_to_f32(uint16_t h) {
   return f;
 }
 
-void to_c64(int storage, const void *src, int64_t n, std::vector<float2> &dst) {
-  dst.resize((size_t)std::max<int64_t>(n, 1));
-  for (int64_t i = 0; i < n; ++i) {
-    if (storage == ANUFFT_STORAGE_C128) {
-      const double *s = (const double *)src;
-      dst[i] = make_float2((float)s[2 * i], (float)s[2 * i + 1]);
-    } else if (storage == ANUFFT_STORAGE_C64) {
-      const float *s = (const float *)src;
-      dst[i] = make_float2(s[2 * i], s[2 * i + 1]);
-    } else {
-      const uint16_t *s = (const uint16_t *)src;
-      dst[i] = make_float2(f16_to_f32(s[2 * i]), f16_to_f32(s[2 * i + 1]));
-    }
+void to_c64(int storage, const void *src, int64_t n, float2 *dst) {
+  if (storage == ANUFFT_STORAGE_C128) {
+    const double *s = (const double *)src;
+    for (int64_t i = 0; i < n; ++i) dst[i] = make_float2((float)s[2 * i], (float)s[2 * i + 1]);
+  } else if (storage == ANUFFT_STORAGE_C64) {
+    const float *s = (const float *)src;
+    for (int64_t i = 0; i < n; ++i) dst[i] = make_float2(s[2 * i], s[2 * i + 1]);
+  } else {
+    const uint16_t *s = (const uint16_t *)src;
+    for (int64_t i = 0; i < n; ++i) dst[i] = make_float2(f16_to_f32(s[2 * i]), f16_to_f32(s[2 * i + 1]));
   }
 }
 
-void from_c64(int storage, const std::vector<float2> &src, int64_t n, void *dst) {
-  for (int64_t i = 0; i < n; ++i) {
-    if (storage == ANUFFT_STORAGE_C128) {
-      double *d = (double *)dst;
+void from_c64(int storage, const float2 *src, int64_t n, void *dst) {
+  if (storage == ANUFFT_STORAGE_C128) {
+    double *d = (double *)dst;
+    for (int64_t i = 0; i < n; ++i) {
       d[2 * i] = src[i].x;
       d[2 * i + 1] = src[i].y;
-    } else if (storage == ANUFFT_STORAGE_C64) {
-      float *d = (float *)dst;
+    }
+  } else if (storage == ANUFFT_STORAGE_C64) {
+    float *d = (float *)dst;
+    for (int64_t i = 0; i < n; ++i) {
       d[2 * i] = src[i].x;
       d[2 * i + 1] = src[i].y;
-    } else {
-      uint16_t *d = (uint16_t *)dst;
+    }
+  } else {
+    uint16_t *d = (uint16_t *)dst;
+    for (int64_t i = 0; i < n; ++i) {
       d[2 * i] = f32_to_f16(src[i].x);
       d[2 * i + 1] = f32_to_f16(src[i].y);
     }
   }
+}
+
+// Device and pinned host memory of a host call, at least db and pb bytes;
+// without pinned memory (pin NULL) the call stages in pageable memory.
+hipError_t grow_arena(HostArena &a, size_t db, size_t pb) {
+  hipError_t e = hipSuccess;
+  if (a.dev_bytes < db) {
+    if (a.dev) (void)hipFree(a.dev);
+    a.dev = nullptr;
+    a.dev_bytes = 0;
+    if ((e = hipMalloc((void **)&a.dev, db)) != hipSuccess) return e;
+    a.dev_bytes = db;
+  }
+  if (a.pin_bytes < pb) {
+    if (a.pin) (void)hipHostFree(a.pin);
+    a.pin = nullptr;
+    a.pin_bytes = 0;
+    if (hipHostMalloc((void **)&a.pin, pb, hipHostMallocDefault) == hipSuccess) a.pin_bytes = pb;
+    else (void)hipGetLastError();
+  }
+  return e;
+}
+void free_arena(HostArena &a) {
+  if (a.dev) (void)hipFree(a.dev);
+  if (a.pin) (void)hipHostFree(a.pin);
+  a.dev = a.pin = nullptr;
+  a.dev_bytes = a.pin_bytes = 0;
 }
 
 anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t profile,
@@ -1821,42 +1864,63 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   hipStream_t s = p->host_stream;
   const int64_t N = p->modes();
   const int64_t nin = type == 1 ? M : N, nout = type == 1 ? N : M;
-  std::vector<float2> hin, hout((size_t)std::max<int64_t>(nout, 1));
-  to_c64(storage, in, nin, hin);
-  std::vector<float> hc((size_t)std::max<int64_t>(M, 1) * p->dim);
-  for (int a = 0; a < p->dim; ++a)
-    for (int64_t j = 0; j < M; ++j) hc[(size_t)a * M + j] = (float)coords[a][j * stride];
   // FP64 results keep one summation order (block_spread.hip)
   const bool blocks = type == 1 && storage == ANUFFT_STORAGE_C128 && p->dim == 3 &&
                       p->kernel_method == kSpreadMfma;
   const Layout lay = layout(p, M, blocks);
   const size_t wsb = lay.total;
-  char *buf = nullptr;
-  size_t b_in = align_up(8 * (size_t)std::max<int64_t>(nin, 1));
-  size_t b_out = align_up(8 * (size_t)std::max<int64_t>(nout, 1));
-  size_t b_c = align_up(4 * hc.size());
-  hipError_t e = hipMalloc(&buf, b_in + b_out + b_c + wsb);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc");
-  float2 *d_in = (float2 *)buf, *d_out = (float2 *)(buf + b_in);
-  float *d_c = (float *)(buf + b_in + b_out);
-  void *d_ws = buf + b_in + b_out + b_c;
+  const size_t nc = (size_t)std::max<int64_t>(M, 1) * p->dim;
+  const size_t b_in = align_up(8 * (size_t)std::max<int64_t>(nin, 1));
+  const size_t b_out = align_up(8 * (size_t)std::max<int64_t>(nout, 1));
+  const size_t b_c = align_up(4 * nc);
+  // The plan's memory, or (in use by another thread's call) this call's own.
+  HostArena own;
+  std::unique_lock<std::mutex> lk(p->arena_mu, std::try_to_lock);
+  HostArena &ar = lk.owns_lock() ? p->arena : own;
+  const bool keep = lk.owns_lock() && b_in + b_out + b_c + wsb <= kArenaDev && b_in + b_out + b_c <= kArenaPin;
+  hipError_t e = grow_arena(ar, b_in + b_out + b_c + wsb, b_in + b_out + b_c);
+  if (e != hipSuccess) {
+    free_arena(ar);
+    return hip_fail(e, "hipMalloc");
+  }
+  std::vector<char> pageable;
+  char *h = ar.pin;
+  if (!h) {
+    pageable.resize(b_in + b_out + b_c);
+    h = pageable.data();
+  }
+  float2 *h_in = (float2 *)h, *h_out = (float2 *)(h + b_in);
+  float *h_c = (float *)(h + b_in + b_out);
+  float2 *d_in = (float2 *)ar.dev, *d_out = (float2 *)(ar.dev + b_in);
+  float *d_c = (float *)(ar.dev + b_in + b_out);
+  void *d_ws = ar.dev + b_in + b_out + b_c;
+  // interleaved coordinates are converted and taken as they are
+  const bool inter = p->dim == 3 && stride == 3 && M > 0 && coords[1] == coords[0] + 1 && coords[2] == coords[0] + 2;
+  const float *dc[3] = {d_c, inter ? d_c + 1 : p->dim == 3 ? d_c + M : d_c,
+                        inter ? d_c + 2 : p->dim == 3 ? d_c + 2 * M : d_c};
+  const int64_t st_c = inter ? 3 : 1;
   anufft_status st = ANUFFT_OK;
   do {
-    if ((e = hipMemcpyAsync(d_in, hin.data(), 8 * (size_t)nin, hipMemcpyHostToDevice, s)) != hipSuccess) break;
-    if ((e = hipMemcpyAsync(d_c, hc.data(), 4 * hc.size(), hipMemcpyHostToDevice, s)) != hipSuccess) break;
-    const float *dc[3] = {d_c, p->dim == 3 ? d_c + M : d_c, p->dim == 3 ? d_c + 2 * M : d_c};
-    st = blocks    ? run_type1(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, lay, s, true)
-         : type == 1 ? anufft_execute_type1(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, wsb, s)
-                   : anufft_execute_type2(p, M, dc, 1, (const float *)d_in, (float *)d_out, d_ws, wsb, s);
+    to_c64(storage, in, nin, h_in);
+    if ((e = hipMemcpyAsync(d_in, h_in, 8 * (size_t)nin, hipMemcpyHostToDevice, s)) != hipSuccess) break;
+    if (inter)
+      for (int64_t j = 0; j < 3 * M; ++j) h_c[j] = (float)coords[0][j];
+    else
+      for (int a = 0; a < p->dim; ++a)
+        for (int64_t j = 0; j < M; ++j) h_c[(size_t)a * M + j] = (float)coords[a][j * stride];
+    if ((e = hipMemcpyAsync(d_c, h_c, 4 * nc, hipMemcpyHostToDevice, s)) != hipSuccess) break;
+    st = blocks    ? run_type1(p, M, dc, st_c, (const float *)d_in, (float *)d_out, d_ws, lay, s, true)
+         : type == 1 ? anufft_execute_type1(p, M, dc, st_c, (const float *)d_in, (float *)d_out, d_ws, wsb, s)
+                     : anufft_execute_type2(p, M, dc, st_c, (const float *)d_in, (float *)d_out, d_ws, wsb, s);
     if (st != ANUFFT_OK) break;
-    if ((e = hipMemcpyAsync(hout.data(), d_out, 8 * (size_t)nout, hipMemcpyDeviceToHost, s)) != hipSuccess) break;
+    if ((e = hipMemcpyAsync(h_out, d_out, 8 * (size_t)nout, hipMemcpyDeviceToHost, s)) != hipSuccess) break;
     e = hipStreamSynchronize(s);
   } while (0);
-  (void)hipStreamSynchronize(s);
-  (void)hipFree(buf);
+  if (st != ANUFFT_OK || e != hipSuccess) (void)hipStreamSynchronize(s);
+  if (st == ANUFFT_OK && e == hipSuccess) from_c64(storage, h_out, nout, out);
+  if (!keep) free_arena(ar);
   if (st != ANUFFT_OK) return st;
   if (e != hipSuccess) return hip_fail(e, "host execute");
-  from_c64(storage, hout, nout, out);
   return ANUFFT_OK;
 }
 
