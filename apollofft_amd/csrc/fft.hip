@@ -402,10 +402,11 @@ hipError_t launch_fft_pass(const FftPass &pass, hipStream_t s) {
   int64_t blocks = (p.nlines + p.lb - 1) / p.lb;
   const int Lf = p.blue_n > 0 ? p.blue_n : p.L;
   size_t lds = (2 * (size_t)p.lb + 1) * Lf * sizeof(float2) + 2 * (size_t)p.lb * sizeof(int64_t);
-  // 256 threads for the usual 1024 points of a block, 1024 from 2048 points
-  // on: a single long line is a chain of stages and loads on one CU (one
-  // line of 4096 points, Bluestein: 62 us at 256 threads in a stage by itself, 32 at 1024).
-  const bool wide = (int64_t)p.lb * Lf >= 2048;
+  // 256 threads for the usual 1024 points of a block; 1024 where few blocks
+  // hold 2048 points and more: a long line by itself is a chain of stages and
+  // loads on one CU (one line of 4096 points, Bluestein: 62 us at 256 threads
+  // in a stage by itself, 32 at 1024; with every CU busy 256 are faster).
+  const bool wide = (int64_t)p.lb * Lf >= 2048 && blocks <= 256;
   const void *fn = wide ? (const void *)fft_pass_kernel<1024> : (const void *)fft_pass_kernel<256>;
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -714,12 +714,16 @@ FftPass make_pass(const anufft_plan *p, int axis, const float2 *in, float2 *out,
   f.blue_n = p->blue_n[axis];
   f.chirp = p->d_chirp[axis];
   f.bhat = p->d_bhat[axis];
-  // lines per block: two LDS buffers of lb*Lf complex within 16 KiB (more,
-  // smaller blocks keep more loads in flight: 9 % faster than 64 KiB at
-  // 128^3), and enough blocks to cover the chip when there are few lines.
+  // lines per block: a multiple of 8, so that passes across lines move whole
+  // 64-byte sectors: 8 as long as the two LDS buffers stay within 32 KiB (2048
+  // points; 100^3 modes, 200 a line, 92 us with 1024 points and 85; 128^3 159
+  // and 130; 48^3 26.2 and 23.7; 127^3, Bluestein of 512, 2 and 4 lines, 460
+  // and 393; more leave too few blocks on a CU, 128^3 with 16 lines 164),
+  // more of short lines (1024 points; 1024 x 16 x 16 modes with 8 lines 57 us,
+  // 40) unless too few blocks are left to cover the chip.
   const int Lf = f.blue_n ? f.blue_n : f.L;
-  int lb = std::max(1, 1024 / Lf);
-  while (lb > 8 && (f.nlines + lb - 1) / lb < 2 * (int64_t)p->cus) lb >>= 1;
+  int lb = std::max(1, std::max(std::min(8, 2048 / Lf), 1024 / Lf / 8 * 8));
+  while (lb > 8 && (f.nlines + lb - 1) / lb < 2 * (int64_t)p->cus) lb = lb / 16 * 8;
   // plan setting: lines per workgroup, within 64 KiB of LDS buffers
   if (p->opts.fft_lines > 0) lb = std::max(1, std::min(p->opts.fft_lines, 4096 / Lf));
   f.lb = (int)std::max<int64_t>(1, std::min<int64_t>(lb, f.nlines));
