@@ -1094,7 +1094,8 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
   int max_bins = 1;
   for (int i = 0; i < nprob; ++i) {
     BinProblem &pr = probs[i];
-    if (!tile_binning(pr.nbins) || pr.cls.ncls == 0) return hipErrorInvalidValue;
+    if (!tile_binning(pr.nbins) || pr.cls.ncls == 0 || pr.cls.ncls * pr.g.bin[0] > kClsKeys)
+      return hipErrorInvalidValue;
     pr.chunk = tile_chunk(pr.pa.num_points);
     pr.nchunks = tile_chunks(pr.pa.num_points);
     pr.chunk0 = chunks;
@@ -1118,6 +1119,7 @@ hipError_t sort_points_batched(BinProblem *probs, int nprob, BinProblem *table, 
 hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBuffers &sb,
                        hipStream_t s, const RecordOut *rec) {
   const int64_t n = pa.num_points;
+  if (sb.cls.ncls * g.bin[0] > kClsKeys) return hipErrorInvalidValue;
   if (rec && sb.cls.ncls > 0 && n > 0 && tile_binning(sb.nbins)) {
     BinProblem pr = bin_problem(pa, g, dim, sb, rec);
     pr.chunk = tile_chunk(n);
