@@ -296,9 +296,9 @@ hipError_t launch_grad3d(int w, const PointArgs &pa, const float2 *grid, const f
                          hipStream_t s);
 // Matrix-core kernels on 16-row windows (window.hip), on the class list of
 // the binning (PointArgs::cperm, cstart) and its records.
-int win_bin_x(int w);          // tile interior along x
+int win_bin_x(int w, bool wide = false);  // tile interior along x
 // workgroups per CU of the launches
-int win_spread_groups(int w, int64_t num_points, int cus);
+int win_spread_groups(int w, const Geom &g, int64_t num_points, int cus);
 hipError_t launch_win_spread(int w, const PointArgs &pa, ZRec zr, float2 *grid, const Geom &g,
                              const WinPoly *dpoly, int num_blocks, hipStream_t s);
 // On 32 x 32 blocks (block_spread.hip), on a tile list along x.

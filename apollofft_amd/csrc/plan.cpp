@@ -230,7 +230,7 @@ struct anufft_plan {
   // gradient (LDS tile).  Each execute sorts with the geometry it uses.
   struct Binning {
     Geom g{};
-    int nbins = 1;
+    int nbins = 0;
     int passes = 1;
     int max_sub = 1024;
     // 3D matrix-core tiles: y-offset classes per tile, offsets per class
@@ -246,6 +246,24 @@ struct anufft_plan {
     }
   } bs, bi, bg;
   Binning bf;  // blocks of the FP64 host Type-1 (3D, matrix cores)
+  Binning bw;  // wide spreading windows (3D, matrix cores)
+  // Type-1 tiles of M points.  With few points to a cell spreading is bound by
+  // the cells its windows flush, each up to 2 PX / BINX times, and wide windows
+  // flush fewer; with many by its products, for which the narrow windows leave
+  // room for one more workgroup on a CU.  Spreading to 128^3 cells, narrow and
+  // wide (us): w = 8, 0.05 points a cell 261 and 199, 0.95 378 and 346; w = 7,
+  // 0.05 124 and 104, 0.5 170 and 166, 0.95 253 and 264; w = 6, 0.05 120 and 88,
+  // 0.5 156 and 151, 0.95 235 and 260; w = 5, 0.05 87 and 75, 0.3 104 and 106;
+  // w = 4, 0.05 76 and 61, 0.3 98 and 88, 0.5 103 and 111.  On small grids, or
+  // with a few thousand points, too few wide windows are left to keep the
+  // chip's workgroups busy (w = 6, 32^3 cells 22 and 29, 64^3 37 and 35; w = 8,
+  // 96^3, 4000 points 68 and 75, 60,000 115 and 101).
+  const Binning &spread_bins(int64_t M) const {
+    const double cells = (double)m[0] * (double)m[1] * (double)m[2];
+    const bool wide = (double)M < cells * (w >= 8 ? 1.0 : w >= 6 ? 0.5 : 0.25) && M >= 8192 &&
+                      bw.nbins * bw.ncls >= (w >= 8 ? 4096 : 256);
+    return wide ? bw : bs;
+  }
   int lds_max = 163840; // gfx950 LDS per workgroup
   int kernel_method = kSpreadMfma;
   hipStream_t host_stream = nullptr;
@@ -292,8 +310,8 @@ Layout layout(const anufft_plan *p, int64_t M, bool blocks = false) {
     l.keys1 = take(4 * Mp);
     l.idx0 = take(4 * Mp);
     l.idx1 = take(4 * Mp);
-    const anufft_plan::Binning *const all[] = {&p->bs, &p->bi, &p->bg, &p->bf};
-    const int kinds = blocks ? 4 : 3;
+    const anufft_plan::Binning *const all[] = {&p->bs, &p->bi, &p->bg, &p->bw, &p->bf};
+    const int kinds = blocks ? 5 : p->bw.ncls > 0 ? 4 : 3;
     int nb = 1;
     size_t cnt_n = radix_count_entries(M), one_n = 0;
     for (int i = 0; i < kinds; ++i) {
@@ -580,6 +598,9 @@ void choose_bins(anufft_plan *p) {
     set_geom(p->bf, p, bf);
     p->bf.max_sub = p->bs.max_sub;
     p->bf.along_x = true;
+    p->bw = p->bs;
+    const int bw[3] = {win_bin_x(p->w, true), bsp[1], bsp[2]};
+    set_geom(p->bw, p, bw);
   }
 
   // LDS-tile geometry (gradient; interpolation on the vector-ALU path)
@@ -808,15 +829,16 @@ struct Exec {
     });
   }
   // Type-1 spreading of binned points (records, then the tile kernel).
-  hipError_t spread3(const PointArgs &pa, const float2 *values, float2 *grid) const {
+  hipError_t spread3(const anufft_plan::Binning &b, const PointArgs &pa, const float2 *values,
+                     float2 *grid) const {
     if (p->kernel_method != kSpreadMfma) {
       hipError_t e = prep(p->bs, pa, values);
       if (e != hipSuccess) return e;
     }
     return timed(ANUFFT_STAGE_SPREAD, [&] {
       if (p->kernel_method == kSpreadMfma)
-        return launch_win_spread(p->w, pa, zrec(pa.num_points), grid, p->bs.g, p->d_poly,
-                                 blocks(p->bs, pa.num_points, win_spread_groups(p->w, pa.num_points, p->cus)), s);
+        return launch_win_spread(p->w, pa, zrec(pa.num_points), grid, b.g, p->d_poly,
+                                 blocks(b, pa.num_points, win_spread_groups(p->w, b.g, pa.num_points, p->cus)), s);
       return launch_spread3d(p->w, pa, rec(), xo(), grid, p->bs.g, p->poly,
                              blocks(p->bs, pa.num_points, 2), s);
     });
@@ -1209,7 +1231,7 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
                                const Layout &lay, hipStream_t stream, bool blocks) {
   DeviceGuard guard(p->device);
   Exec ex{p, stream, (char *)ws, lay};
-  const anufft_plan::Binning &bs = blocks ? p->bf : p->bs;
+  const anufft_plan::Binning &bs = blocks ? p->bf : p->spread_bins(M);
   hipError_t e = hipSuccess;
   if (M > 0 && p->dim == 1) {
     e = ex.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ex.grid(), p->cells(), ex.s); });
@@ -1233,7 +1255,7 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
       if (e == hipSuccess) e = bin();
     }
     if (e != hipSuccess) return hip_fail(e, "fill / binning");
-    e = blocks ? ex.spread_blocks(pa, ex.grid()) : ex.spread3(pa, (const float2 *)values, ex.grid());
+    e = blocks ? ex.spread_blocks(pa, ex.grid()) : ex.spread3(bs, pa, (const float2 *)values, ex.grid());
     if (e != hipSuccess) return hip_fail(e, "spread");
   } else {
     e = ex.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ex.grid(), p->cells(), ex.s); });
@@ -1384,7 +1406,7 @@ anufft_status anufft_execute_type2_backward(const anufft_plan *p, int64_t M,
       },
       [&] { return ex.bin(p->bs, pa, (const float2 *)g, Exec::kValues | Exec::kIndices); });
   if (e != hipSuccess) return hip_fail(e, "fft / fill / binning");
-  e = ex.spread3(pa, (const float2 *)g, ex.grid());
+  e = ex.spread3(p->bs, pa, (const float2 *)g, ex.grid());
   if (e != hipSuccess) return hip_fail(e, "spread");
   e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.grid_to_modes((float2 *)grad_modes); });
   if (e != hipSuccess) return hip_fail(e, "fft");
@@ -1537,7 +1559,7 @@ anufft_status anufft_debug_spread(const anufft_plan *p, int64_t M, const float *
   if (p->dim == 3) {
     e = ex.bin(p->bs, pa, (const float2 *)values, Exec::kValues);
     if (e != hipSuccess) return hip_fail(e, "binning");
-    e = ex.spread3(pa, (const float2 *)values, (float2 *)grid);
+    e = ex.spread3(p->bs, pa, (const float2 *)values, (float2 *)grid);
   } else {
     e = ex.spread1(pa, (const float2 *)values, (float2 *)grid);
   }
@@ -1709,7 +1731,7 @@ anufft_status anufft_execute_type1_batched(const anufft_plan *const *plans, int3
     });
     if (e != hipSuccess) return hip_fail(e, "spread records");
   }
-  const int per_cu = mf ? win_spread_groups(p0->w, points, p0->cus) : 2;
+  const int per_cu = mf ? win_spread_groups(p0->w, p0->bs.g, points, p0->cus) : 2;
   const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(sub_upper, per_cu * (int64_t)p0->cus));
   e = e0.timed(ANUFFT_STAGE_SPREAD, [&] {
     if (mf)

@@ -50,14 +50,18 @@
 namespace anufft {
 namespace {
 
-template <int W>
+// x cells per wave: of the windows, and of the wide spreading windows for
+// few points a cell (anufft_plan::spread_bins).
+constexpr int win_cells(int w) { return w >= 7 ? 5 : (w >= 5 ? 4 : 3); }
+constexpr int wide_cells(int w) { return w >= 5 ? 7 : 6; }
+
+template <int W, int XC = win_cells(W)>
 struct Win {
   static constexpr int T = 2 * W;
   static constexpr int CW = 17 - T;  // y offsets of a class at most
   static constexpr int NW = 4;       // waves
   static constexpr int NT = 64 * NW;
-  // x cells per wave
-  static constexpr int XW = W >= 7 ? 5 : (W >= 5 ? 4 : 3);
+  static constexpr int XW = XC;      // x cells per wave
   static constexpr int PX = NW * XW;
   static constexpr int BINX = PX - T + 1;
   static_assert(BINX >= 1 && CW >= 1, "window shape");
@@ -221,8 +225,8 @@ struct SLds {
   static constexpr int R = B + 2 * 64 * kSLd * 2;         // int [groups]: x cells reached
   static constexpr int SIZE = R + 16;
 };
-template <int W>
-using SpreadAcc = f32x4[Win<W>::XW][4];  // [slot][block of 8 z cells]
+template <int W, int XC>
+using SpreadAcc = f32x4[XC][4];  // [slot][block of 8 z cells]
 
 // Ring rows and z cells of the accumulators.  Register r of lane (i16, g4)
 // of a block is ring row 4 r + g4, so that the (few, consecutive) rows of a
@@ -237,11 +241,11 @@ using SpreadAcc = f32x4[Win<W>::XW][4];  // [slot][block of 8 z cells]
 //
 // Add rows [0, nrow) of the window t to the grid (scaled by s_out) and zero
 // them.
-template <int W>
-__device__ __forceinline__ void win_flush(SpreadAcc<W> &acc, float2 *grid, const Geom &g,
+template <int W, int XC>
+__device__ __forceinline__ void win_flush(SpreadAcc<W, XC> &acc, float2 *grid, const Geom &g,
                                           const WTile &t, int wave, int i16, int g4, int nrow,
                                           float s_out) {
-  using WN = Win<W>;
+  using WN = Win<W, XC>;
   int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
   int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
   asm volatile("" : "+v"(i16), "+v"(g4), "+s"(m0), "+s"(m1), "+s"(m2));
@@ -313,10 +317,10 @@ __device__ __forceinline__ int cells_reached(int off, int first, int last) {
 // point; 2 and 3 the B operands of the first and second 32 points, lanes 0-31
 // re and 32-63 im (staged_point).  Lanes past the round's points leave their
 // column of the tables zero.
-template <int W>
+template <int W, int XC>
 __device__ __forceinline__ void spread_stage(char *sh, int role, int lane, int npts, float4 ra,
                                              float2 cv, const WinPoly *poly, const WTile &w) {
-  using WN = Win<W>;
+  using WN = Win<W, XC>;
   constexpr int T = WN::T, PX = WN::PX;
   using L = SLds<PX>;
   const int off = __float_as_int(ra.w);
@@ -361,10 +365,10 @@ __device__ __forceinline__ int staged_point(int role, int lane) {
 // i16 (the ring row whose sums its lane group keeps, win_flush) and B column
 // i16 for the points 8 g4 .. 8 g4 + 7.  x cells the 32 points do not reach
 // are left out.
-template <int W>
-__device__ __forceinline__ void spread_products(SpreadAcc<W> &acc, const char *sh, int ng,
+template <int W, int XC>
+__device__ __forceinline__ void spread_products(SpreadAcc<W, XC> &acc, const char *sh, int ng,
                                                 const WTile &t, int wave, int i16, int g4) {
-  using WN = Win<W>;
+  using WN = Win<W, XC>;
   using L = SLds<WN::PX>;
   constexpr int XW = WN::XW;
   asm volatile("" : "+v"(i16), "+v"(g4));
@@ -421,16 +425,16 @@ __device__ __forceinline__ int max_exp(const float *slots, int lane) {
 }
 
 // Spread the share r of one problem's list.
-template <int W>
+template <int W, int XC>
 __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, float2 *grid,
                                            const Geom &g, const XcdChunk &r, const WinPoly *poly,
                                            char *sh) {
-  using WN = Win<W>;
+  using WN = Win<W, XC>;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i16 = lane & 15, g4 = lane >> 4;
   if (r.begin >= r.end) return;
-  SpreadAcc<W> acc;
+  SpreadAcc<W, XC> acc;
 #pragma unroll
   for (int q = 0; q < WN::XW; ++q)
 #pragma unroll
@@ -457,14 +461,14 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
     chain += n;
     for (int c0 = 0; c0 < n; c0 += kWinPts) {
       const int npts = min(kWinPts, n - c0);
-      spread_stage<W>(sh, role, lane, npts, ra, make_float2(cv.x * s_in, cv.y * s_in), poly, t);
+      spread_stage<W, XC>(sh, role, lane, npts, ra, make_float2(cv.x * s_in, cv.y * s_in), poly, t);
       __syncthreads();
       role = (role + 1) & 3;
       ra = zr.r[np];
       if (role >= 2) cv = zr.v[np];
       ahead.advance();
       np = perm[ahead.pos(staged_point((role + 1) & 3, lane))];
-      spread_products<W>(acc, sh, (npts + 31) >> 5, t, wave, i16, g4);
+      spread_products<W, XC>(acc, sh, (npts + 31) >> 5, t, wave, i16, g4);
       __syncthreads();
     }
     if (!cw.next()) break;
@@ -474,26 +478,25 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
     asm volatile("" : "+v"(ra.x), "+v"(ra.w), "+v"(cv.x), "+v"(np));
     const bool slide = w.xlo == t.xlo && w.z0 == t.z0 && w.y0 >= t.y0 && chain + cw.hi - cw.lo <= kMaxChain;
     const int nrow = slide ? min(16, w.y0 - t.y0) : 16;
-    if (nrow > 0) win_flush<W>(acc, grid, g, t, wave, i16, g4, nrow, s_out);
+    if (nrow > 0) win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, nrow, s_out);
     if (nrow == 16) chain = 0;
     t = w;
   }
-  win_flush<W>(acc, grid, g, t, wave, i16, g4, 16, s_out);
+  win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, 16, s_out);
 }
 
 // Workgroups resident on a CU: as many as the registers hold without
 // spilling.  Spreading's accumulators (16 XW registers a lane) allow 3, from
 // w = 4 down 4 (2e6 points on 64^3, w = 4: 166 to 158 us; w = 6 at 4: 226 to
 // 306, the spills queue behind the atomics).
-template <int W>
-constexpr int spread_groups_per_cu() { return Win<W>::XW <= 3 ? 4 : 3; }
+constexpr int spread_groups_per_cu(int cells) { return cells <= 3 ? 4 : cells <= 5 ? 3 : 2; }
 
-template <int W>
-__global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu<W>()) void win_spread_kernel(
+template <int W, int XC>
+__global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu(XC)) void win_spread_kernel(
     PointArgs pa, ZRec zr, float2 *grid, Geom g, const WinPoly *__restrict__ dpoly) {
-  __shared__ __align__(16) char sh[SLds<Win<W>::PX>::SIZE];
+  __shared__ __align__(16) char sh[SLds<Win<W, XC>::PX>::SIZE];
   const XcdChunk r(pa);
-  spread_run<W>(pa, zr, grid, g, r, dpoly, sh);
+  spread_run<W, XC>(pa, zr, grid, g, r, dpoly, sh);
 }
 
 // A descriptor read through the scalar cache (its fields stay in scalar
@@ -513,10 +516,10 @@ __device__ __forceinline__ T load_scalar(const T *p) {
 
 // Batched form: one persistent launch over the lists of all problems
 // (wpre[p] = work of the problems before p, wpre[nprob] = total).
-template <int W>
-__global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu<W>()) void win_spread_batched_kernel(
+template <int W, int XC>
+__global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu(XC)) void win_spread_batched_kernel(
     const SpreadProblem *probs, const uint32_t *wpre, int nprob, const WinPoly *__restrict__ dpoly) {
-  __shared__ __align__(16) char sh[SLds<Win<W>::PX>::SIZE];
+  __shared__ __align__(16) char sh[SLds<Win<W, XC>::PX>::SIZE];
   uint32_t w0, w1;
   xcd_work_range(wpre[nprob], w0, w1);
   if (w0 >= w1) return;
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu<W>()) void win_spr
     if (hi <= w0) continue;  // no work of this problem in the range
     const SpreadProblem pr = load_scalar(probs + p);
     const XcdChunk part(pr.pa.subs, pr.pa.nsub[0], hi - lo, max(w0, lo) - lo, min(w1, hi) - lo);
-    spread_run<W>(pr.pa, pr.zr, pr.grid, pr.g, part, dpoly, sh);
+    spread_run<W, XC>(pr.pa, pr.zr, pr.grid, pr.g, part, dpoly, sh);
   }
 }
 
@@ -997,8 +1000,12 @@ template <int W>
 struct WinSpread {
   static hipError_t run(const PointArgs &pa, ZRec zr, float2 *grid, const Geom &g,
                         const WinPoly *dpoly, int nblk, hipStream_t s) {
-    hipLaunchKernelGGL(win_spread_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, g,
-                       dpoly);
+    if (g.bin[0] > Win<W>::BINX)
+      hipLaunchKernelGGL((win_spread_kernel<W, wide_cells(W)>), dim3(nblk), dim3(Win<W>::NT), 0, s, pa,
+                         zr, grid, g, dpoly);
+    else
+      hipLaunchKernelGGL((win_spread_kernel<W, win_cells(W)>), dim3(nblk), dim3(Win<W>::NT), 0, s, pa,
+                         zr, grid, g, dpoly);
     return hipGetLastError();
   }
 };
@@ -1007,7 +1014,7 @@ template <int W>
 struct WinSpreadBatched {
   static hipError_t run(const SpreadProblem *probs, const uint32_t *wpre, int nprob,
                         const WinPoly *dpoly, int nblk, hipStream_t s) {
-    hipLaunchKernelGGL(win_spread_batched_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, probs,
+    hipLaunchKernelGGL((win_spread_batched_kernel<W, win_cells(W)>), dim3(nblk), dim3(Win<W>::NT), 0, s, probs,
                        wpre, nprob, dpoly);
     return hipGetLastError();
   }
@@ -1036,17 +1043,17 @@ struct WinGrad {
 
 template <int W>
 struct WinShape {
-  static hipError_t run(int *binx) {
-    *binx = Win<W>::BINX;
+  static hipError_t run(bool wide, int *binx) {
+    *binx = wide ? Win<W, wide_cells(W)>::BINX : Win<W>::BINX;
     return hipSuccess;
   }
 };
 
 } // namespace
 
-int win_bin_x(int w) {
+int win_bin_x(int w, bool wide) {
   int v = 1;
-  (void)dispatch_w<WinShape>(w, &v);
+  (void)dispatch_w<WinShape>(w, wide, &v);
   return v;
 }
 
@@ -1064,7 +1071,7 @@ static int groups(int64_t num_points, int cus, int resident, int most) {
 template <int W>
 struct WinGroups {
   static hipError_t run(int which, int64_t num_points, int cus, int *v) {
-    constexpr int R = spread_groups_per_cu<W>(), I = interp_groups_per_cu<W>(),
+    constexpr int R = spread_groups_per_cu(win_cells(W)), I = interp_groups_per_cu<W>(),
                   G = grad_groups_per_cu<W>();
     *v = which == 0   ? groups(num_points, cus, R, W >= 7 ? 5 * R : W >= 5 ? 2 * R : R)
          : which == 1 ? groups(num_points, cus, I, 16 / I * I)
@@ -1077,7 +1084,10 @@ static int win_groups(int which, int w, int64_t num_points, int cus) {
   (void)dispatch_w<WinGroups>(w, which, num_points, cus, &v);
   return v;
 }
-int win_spread_groups(int w, int64_t num_points, int cus) { return win_groups(0, w, num_points, cus); }
+int win_spread_groups(int w, const Geom &g, int64_t num_points, int cus) {
+  if (g.bin[0] > win_bin_x(w)) return spread_groups_per_cu(wide_cells(w));  // few points
+  return win_groups(0, w, num_points, cus);
+}
 int win_interp_groups(int w, int64_t num_points, int cus) { return win_groups(1, w, num_points, cus); }
 int win_grad_groups(int w, int64_t num_points, int cus) { return win_groups(2, w, num_points, cus); }
 
