@@ -308,7 +308,7 @@ hipError_t launch_block_spread(int w, const PointArgs &pa, ZRec zr, float2 *grid
 hipError_t launch_win_spread_batched(int w, const SpreadProblem *host_probs, int nprob,
                                      SpreadProblem *dev_table, uint32_t *dev_prefix,
                                      const WinPoly *dpoly, int num_blocks, hipStream_t s);
-int win_interp_groups(int w, int64_t num_points, int cus);
+int win_interp_groups(int w, int cw, int64_t num_points, int cus);
 int win_grad_groups(int w, int64_t num_points, int cus);
 // gmax: the grid's kMaxSlots maxima (FftPass::vmax), the scale of the windows.
 hipError_t launch_win_interp(int w, const PointArgs &pa, ZRec zr, const float2 *grid,

@@ -247,6 +247,7 @@ struct anufft_plan {
   } bs, bi, bg;
   Binning bf;  // blocks of the FP64 host Type-1 (3D, matrix cores)
   Binning bw;  // wide spreading windows (3D, matrix cores)
+  Binning bt;  // tall interpolation windows: bi with one class a tile
   // Type-1 tiles of M points.  With few points to a cell spreading is bound by
   // the cells its windows flush, each up to 2 PX / BINX times, and wide windows
   // flush fewer; with many by its products, for which the narrow windows leave
@@ -263,6 +264,17 @@ struct anufft_plan {
     const bool wide = (double)M < cells * (w >= 8 ? 1.0 : w >= 6 ? 0.5 : 0.25) && M >= 8192 &&
                       bw.nbins * bw.ncls >= (w >= 8 ? 4096 : 256);
     return wide ? bw : bs;
+  }
+  // Type-2 tiles of M points.  Classes of a few points each leave rounds of
+  // kWinPts points nearly empty, and w = 7 and 8 have 5 and 16 classes a tile;
+  // tall windows take a tile's points as one class, for twice the products a
+  // point.  Interpolation from 128^3 cells, 16-row and tall windows (us): w = 8,
+  // 4 points a class 314 and 133, 23 353 and 211, 38 356 and 275; w = 7, 1.5 a
+  // class 112 and 94, 15 123 and 115 (clustered 124 and 126), 44 143 and 157.
+  // (w = 6: 2 a class 91 and 97, 20 104 and 119.)
+  const Binning &interp_bins(int64_t M) const {
+    const int per_class = w >= 8 ? 48 : w == 7 ? 8 : 0;
+    return bt.ncls > 0 && M < (int64_t)per_class * bi.nbins * bi.ncls ? bt : bi;
   }
   int lds_max = 163840; // gfx950 LDS per workgroup
   int kernel_method = kSpreadMfma;
@@ -636,6 +648,11 @@ void choose_bins(anufft_plan *p) {
     p->bi.max_sub = p->bs.max_sub;
     p->bi.ncls = p->bs.ncls;
     p->bi.cw = p->bs.cw;
+    if (p->bi.ncls > 1) {
+      p->bt = p->bi;
+      p->bt.ncls = 1;
+      p->bt.cw = p->bi.g.bin[1];
+    }
   } else {
     p->bi = p->bg;
   }
@@ -863,11 +880,12 @@ struct Exec {
   }
   // Type-2 interpolation and coordinate gradient of binned points from the
   // fine grid in `from`'s workspace.
-  hipError_t interp3(const PointArgs &pa, const Exec &from, float2 *out) const {
+  hipError_t interp3(const anufft_plan::Binning &b, const PointArgs &pa, const Exec &from,
+                     float2 *out) const {
     return timed(ANUFFT_STAGE_INTERP, [&] {
       if (p->kernel_method == kSpreadMfma)
-        return launch_win_interp(p->w, pa, zrec(pa.num_points), from.grid(), from.gmax(), out, p->bi.g,
-                                 p->d_poly, blocks(p->bi, pa.num_points, win_interp_groups(p->w, pa.num_points, p->cus)), s);
+        return launch_win_interp(p->w, pa, zrec(pa.num_points), from.grid(), from.gmax(), out, b.g, p->d_poly,
+                                 blocks(b, pa.num_points, win_interp_groups(p->w, b.cw, pa.num_points, p->cus)), s);
       return launch_interp3d(p->w, pa, from.grid(), out, p->bi.g, p->poly,
                              blocks(p->bi, pa.num_points, 4), s);
     });
@@ -1314,16 +1332,17 @@ anufft_status anufft_execute_type2(const anufft_plan *p, int64_t M, const float 
   Exec ex{p, (hipStream_t)stream, (char *)ws, lay};
   hipError_t e;
   if (p->dim == 3) {
-    PointArgs pa = ex.point_args(p->bi, M, coords, stride);
+    const anufft_plan::Binning &b = p->interp_bins(M);
+    PointArgs pa = ex.point_args(b, M, coords, stride);
     // the FFT passes (modes -> grid) and the binning (points) are independent:
     // the FFT goes to the plan's second stream, joined before interpolation
     e = ex.fork_join(
         [&](const Exec &ea) {
           return ea.fine_grid((const float2 *)modes, p->opts.compat_reference_type2_3d_scaling != 0);
         },
-        [&] { return ex.bin(p->bi, pa, nullptr, Exec::kIndices); });
+        [&] { return ex.bin(b, pa, nullptr, Exec::kIndices); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
-    e = ex.interp3(pa, ex, (float2 *)out);
+    e = ex.interp3(b, pa, ex, (float2 *)out);
   } else {
     e = ex.timed(ANUFFT_STAGE_FFT, [&] { return ex.modes_to_grid((const float2 *)modes, false); });
     if (e != hipSuccess) return hip_fail(e, "fft");
@@ -1438,7 +1457,7 @@ anufft_status anufft_execute_type1_backward(const anufft_plan *p, int64_t M,
       [&](const Exec &ea) { return ea.fine_grid((const float2 *)G, false); },
       [&] { return ex.bin(p->bi, pa, (const float2 *)values, Exec::kValues | Exec::kIndices); });
   if (e != hipSuccess) return hip_fail(e, "fft / binning");
-  e = ex.interp3(pa, ex, (float2 *)grad_values);
+  e = ex.interp3(p->bi, pa, ex, (float2 *)grad_values);
   if (e != hipSuccess) return hip_fail(e, "interp");
   e = ex.grad3(pa, ex, (const float2 *)values, grad_x);
   if (e != hipSuccess) return hip_fail(e, "grad");

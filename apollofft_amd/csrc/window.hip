@@ -556,7 +556,7 @@ __global__ __launch_bounds__(Win<W>::NT, spread_groups_per_cu(XC)) void win_spre
 // 2e6 points, w = 7, 394 us and now 371, 200,000 ragged ones, w = 4, 113 and
 // 95.)
 constexpr int kIRow = 40;   // row stride (halves) of a staged point's z weights (32 cells)
-constexpr int kIRowY = 20;  // row stride (floats) of its y weights (16 ring rows)
+constexpr int kIRowY = 20;  // row stride (floats) of its y weights (16 ring rows; 32: + 16)
 template <int W>
 struct ILds {
   using WN = Win<W>;
@@ -566,19 +566,27 @@ struct ILds {
 // (z offsets start at 1: no tap of the tile lies in a skipped first cell).
 __device__ __forceinline__ int even_z0(int z0) { return z0 + (z0 & 1); }
 
-template <int W>
+// H windows of 16 rows on top of each other: H = 2, tall windows, hold every
+// point of a tile (bin_y + 2 W <= 32 rows) for twice the products a point; row
+// y at y mod 16 H.
+template <int W, int H>
 struct GridWin {
   static constexpr int XW = Win<W>::XW;
-  half8 rh[XW], rl[XW], ih[XW], il[XW];
+  half8 rh[H][XW], rl[H][XW], ih[H][XW], il[H][XW];
 
-  // Load rows `first` .. 15 of window t (scaled by s); the other rows keep
-  // their content.
+  // Load rows `first` .. 16 H - 1 of window t (scaled by s); the other rows
+  // keep their content.
   __device__ __forceinline__ void load(const float2 *grid, const Geom &g, const WTile &t, int first,
                                        float s, int wave, int i16, int g4) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) load_half(h, grid, g, t, first, s, wave, i16, g4);
+  }
+  __device__ __forceinline__ void load_half(int h, const float2 *grid, const Geom &g, const WTile &t,
+                                            int first, float s, int wave, int i16, int g4) {
     int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
     int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
     asm volatile("" : "+v"(i16), "+v"(g4), "+s"(m0), "+s"(m1), "+s"(m2));
-    const int row = (i16 - t.y0) & 15;
+    const int row = (16 * h + i16 - t.y0) & (16 * H - 1);
     if (row < first) return;
     const int z0 = even_z0(t.z0) + 8 * g4;
     const uint32_t y = (uint32_t)wrap(t.y0 + row, m1) * (uint32_t)m2;
@@ -609,8 +617,8 @@ struct GridWin {
         tr[j] = v[j].x * s;
         ti[j] = v[j].y * s;
       }
-      split8(tr, rh[q], rl[q]);
-      split8(ti, ih[q], il[q]);
+      split8(tr, rh[h][q], rl[h][q]);
+      split8(ti, ih[h][q], il[h][q]);
     }
   }
 };
@@ -649,15 +657,15 @@ __device__ __forceinline__ void interp_stage_x(float *row, bool ok, float z, int
     for (int i = 0; i < 2 * W; ++i) row[i] = v[i];
   }
 }
-template <int W, bool ODD>
+template <int W, int H, bool ODD>
 __device__ __forceinline__ void interp_stage_y(float *row, bool ok, float z, int first, const float *poly) {
 #pragma unroll
-  for (int i = 0; i < 16; i += 4) *(float4 *)(row + i) = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i = 0; i < 16 * H; i += 4) *(float4 *)(row + i) = make_float4(0.f, 0.f, 0.f, 0.f);
   float v[2 * W];
   taps_scalar<W, ODD>((ConstFloatPtr)poly, z, v);
   if (ok) {
-    const int r0 = first & 15, cut = 16 - r0;  // taps from `cut` on wrap around
-    float *a = row + r0, *b = a - 16;
+    const int r0 = first & (16 * H - 1), cut = 16 * H - r0;  // taps from `cut` on wrap around
+    float *a = row + r0, *b = a - 16 * H;
 #pragma unroll
     for (int i = 0; i < 2 * W; ++i) (i < cut ? a : b)[i] = v[i];
   }
@@ -690,18 +698,18 @@ __device__ __forceinline__ void interp_stage_z(_Float16 *rh, _Float16 *rl, bool 
 
 // As many workgroups on a CU as the registers hold: 4 up to w = 6 (2e6 points
 // on 64^3, w = 6: 252 to 230 us), 3 above (w = 7 at 4: 296 to 372, spilled).
-template <int W>
-constexpr int interp_groups_per_cu() { return Win<W>::XW <= 4 ? 4 : 3; }
+// Tall windows need twice the operand registers.
+constexpr int interp_groups_per_cu(int cells, int h) { return (cells <= 4 ? 4 : 3) - (h - 1); }
 
-template <int W>
-__global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_interp_kernel(
+template <int W, int H>
+__global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) void win_interp_kernel(
     PointArgs pa, ZRec zr, const float2 *grid, const float *gmax, float2 *out, Geom g,
     const WinPoly *__restrict__ dpoly) {
   using WN = Win<W>;
   using L = ILds<W>;
-  constexpr int XW = WN::XW;
+  constexpr int XW = WN::XW, ROWY = kIRowY + 16 * (H - 1);
   __shared__ __align__(16) _Float16 BH[kWinPts * kIRow], BL[kWinPts * kIRow];
-  __shared__ __align__(16) float WY[kWinPts * kIRowY], WX[kWinPts * L::ROWX];
+  __shared__ __align__(16) float WY[kWinPts * ROWY], WX[kWinPts * L::ROWX];
   __shared__ float RED[4][2][kWinPts];  // per wave: re, im of each point
   __shared__ __align__(16) int REACH[kWinPts / 16];   // x cells each group of 16 points reaches
   const int lane = threadIdx.x & 63;
@@ -721,7 +729,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
   ahead.advance();
   np = perm[ahead.pos(lane)];
 
-  GridWin<W> win;
+  GridWin<W, H> win;
   const int e = max_exp(gmax, lane);
   const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
   ClassWalk cw(r, pa);
@@ -730,10 +738,11 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
   do {
     const WTile n = win_tile<W>(g, cw.bin, cw.cls, pa.cw);
     // rows carry over along a pencil, ascending classes
-    const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
+    const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0
+                          ? 16 * H - min(16 * H, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16) win.load(grid, g, t, first, s_in, wave, i16, g4);
+    if (first < 16 * H) win.load(grid, g, t, first, s_in, wave, i16, g4);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
     for (int c0 = 0; c0 < npt; c0 += kWinPts) {
@@ -747,7 +756,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
           stage_reach<W>(REACH, off, npts, lane);
           interp_stage_x<W, false>(WX + p * L::ROWX, ok, ra.x, off & 255, &dpoly->p.c[0][0]);
         } else if (role == 1) {
-          interp_stage_y<W, false>(WY + p * kIRowY, ok, ra.y, ((off >> 8) & 255) - t.o1 + t.y0,
+          interp_stage_y<W, H, false>(WY + p * ROWY, ok, ra.y, ((off >> 8) & 255) - t.o1 + t.y0,
                                    &dpoly->p.c[0][0]);
         } else if (role == 2) {
           interp_stage_z<W, false>(BH + p * kIRow, BL + p * kIRow, ok, ra.z, ((off >> 16) & 255) + oz,
@@ -767,8 +776,11 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
         const int k = 16 * gi + i16;  // this lane's point
         const half8 bh = *(const half8 *)(BH + k * kIRow + 8 * g4);
         const half8 bl = *(const half8 *)(BL + k * kIRow + 8 * g4);
-        // wy at this lane's D rows (ring rows 4 g4 .. 4 g4 + 3), wx at the wave's cells
-        const float4 wy = *(const float4 *)(WY + k * kIRowY + 4 * g4);
+        // wy at this lane's D rows (ring rows 4 g4 .. 4 g4 + 3 of each half), wx
+        // at the wave's cells
+        float4 wy[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) wy[h] = *(const float4 *)(WY + k * ROWY + 16 * h + 4 * g4);
         float wx[XW];
 #pragma unroll
         for (int q = 0; q < XW; ++q) wx[q] = WX[k * L::ROWX + 4 * q + wave];
@@ -779,24 +791,28 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu<W>()) void win_int
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         reached_cells<XW>(c0, c1, [&](auto q0, auto q1) {
           f32x4 dr[2], di[2];
-          // products of cell q + 1 are issued before the contraction of cell q
+          // products of one cell (and half) are issued before the contraction of
+          // the one before
 #pragma unroll
-          for (int q = q0; q <= q1; ++q) {
-            if (q < q1) {
-              f32x4 &a = dr[q & 1], &b = di[q & 1];
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], bh, zero, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], bh, zero, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], bl, a, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], bl, b, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[q], bh, a, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[q], bh, b, 0, 0, 0);
+          for (int u = q0 * H; u <= q1 * H; ++u) {
+            if (u < q1 * H) {
+              const int q = u / H, h = u % H;
+              f32x4 &a = dr[u & 1], &b = di[u & 1];
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[h][q], bh, zero, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[h][q], bh, zero, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[h][q], bl, a, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[h][q], bl, b, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[h][q], bh, a, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[h][q], bh, b, 0, 0, 0);
             }
-            if (q > q0) {
-              const f32x4 &a = dr[(q - 1) & 1], &b = di[(q - 1) & 1];
-              const float pr = fmaf(wy.x, a[0], fmaf(wy.y, a[1], fmaf(wy.z, a[2], wy.w * a[3])));
-              const float pi = fmaf(wy.x, b[0], fmaf(wy.y, b[1], fmaf(wy.z, b[2], wy.w * b[3])));
-              accr = fmaf(wx[q - 1], pr, accr);
-              acci = fmaf(wx[q - 1], pi, acci);
+            if (u > q0 * H) {
+              const int q = (u - 1) / H, h = (u - 1) % H;
+              const f32x4 &a = dr[(u - 1) & 1], &b = di[(u - 1) & 1];
+              const float4 y = wy[h];
+              const float pr = fmaf(y.x, a[0], fmaf(y.y, a[1], fmaf(y.z, a[2], y.w * a[3])));
+              const float pi = fmaf(y.x, b[0], fmaf(y.y, b[1], fmaf(y.z, b[2], y.w * b[3])));
+              accr = fmaf(wx[q], pr, accr);
+              acci = fmaf(wx[q], pi, acci);
             }
           }
         });
@@ -854,7 +870,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
   ahead.advance();
   np = perm[ahead.pos(lane)];
 
-  GridWin<W> win;
+  GridWin<W, 1> win;
   const int e = max_exp(gmax, lane);
   const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(1.0f, e);
   ClassWalk cw(r, pa);
@@ -882,8 +898,8 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
           interp_stage_x<W, true>(DX + p * L::ROWX, ok, ra.x, off & 255, &dpoly->p.dc[0][0]);
         } else if (role == 1) {
           const int s = ((off >> 8) & 255) - t.o1 + t.y0;
-          interp_stage_y<W, false>(WY + p * kIRowY, ok, ra.y, s, &dpoly->p.c[0][0]);
-          interp_stage_y<W, true>(DY + p * kIRowY, ok, ra.y, s, &dpoly->p.dc[0][0]);
+          interp_stage_y<W, 1, false>(WY + p * kIRowY, ok, ra.y, s, &dpoly->p.c[0][0]);
+          interp_stage_y<W, 1, true>(DY + p * kIRowY, ok, ra.y, s, &dpoly->p.dc[0][0]);
         } else if (role == 2) {
           u = un;
           j = jn;
@@ -925,18 +941,18 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
           for (int q = q0; q <= q1; ++q) {
             if (q < q1) {
               f32x4 &a = dr[q & 1], &b = di[q & 1], &c = er[q & 1], &d = ei[q & 1];
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], bh, zero, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], bh, zero, 0, 0, 0);
-              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], dh, zero, 0, 0, 0);
-              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], dh, zero, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], bl, a, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], bl, b, 0, 0, 0);
-              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[q], dl, c, 0, 0, 0);
-              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[q], dl, d, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[q], bh, a, 0, 0, 0);
-              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[q], bh, b, 0, 0, 0);
-              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[q], dh, c, 0, 0, 0);
-              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[q], dh, d, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[0][q], bh, zero, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[0][q], bh, zero, 0, 0, 0);
+              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[0][q], dh, zero, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[0][q], dh, zero, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[0][q], bl, a, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[0][q], bl, b, 0, 0, 0);
+              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rh[0][q], dl, c, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.ih[0][q], dl, d, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[0][q], bh, a, 0, 0, 0);
+              b = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[0][q], bh, b, 0, 0, 0);
+              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.rl[0][q], dh, c, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(win.il[0][q], dh, d, 0, 0, 0);
             }
             if (q > q0) {
               const f32x4 &a = dr[(q - 1) & 1], &b = di[(q - 1) & 1];
@@ -1024,8 +1040,16 @@ template <int W>
 struct WinInterp {
   static hipError_t run(const PointArgs &pa, ZRec zr, const float2 *grid, const float *gmax,
                         float2 *out, const Geom &g, const WinPoly *dpoly, int nblk, hipStream_t s) {
-    hipLaunchKernelGGL(win_interp_kernel<W>, dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid, gmax,
-                       out, g, dpoly);
+    if constexpr (W >= 7) {  // (anufft_plan::interp_bins takes them from there on)
+      if (pa.cw > Win<W>::CW) {
+        hipLaunchKernelGGL((win_interp_kernel<W, 2>), dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid,
+                           gmax, out, g, dpoly);
+        return hipGetLastError();
+      }
+    }
+    if (pa.cw > Win<W>::CW) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((win_interp_kernel<W, 1>), dim3(nblk), dim3(Win<W>::NT), 0, s, pa, zr, grid,
+                       gmax, out, g, dpoly);
     return hipGetLastError();
   }
 };
@@ -1071,7 +1095,7 @@ static int groups(int64_t num_points, int cus, int resident, int most) {
 template <int W>
 struct WinGroups {
   static hipError_t run(int which, int64_t num_points, int cus, int *v) {
-    constexpr int R = spread_groups_per_cu(win_cells(W)), I = interp_groups_per_cu<W>(),
+    constexpr int R = spread_groups_per_cu(win_cells(W)), I = interp_groups_per_cu(win_cells(W), 1),
                   G = grad_groups_per_cu<W>();
     *v = which == 0   ? groups(num_points, cus, R, W >= 7 ? 5 * R : W >= 5 ? 2 * R : R)
          : which == 1 ? groups(num_points, cus, I, 16 / I * I)
@@ -1088,7 +1112,10 @@ int win_spread_groups(int w, const Geom &g, int64_t num_points, int cus) {
   if (g.bin[0] > win_bin_x(w)) return spread_groups_per_cu(wide_cells(w));  // few points
   return win_groups(0, w, num_points, cus);
 }
-int win_interp_groups(int w, int64_t num_points, int cus) { return win_groups(1, w, num_points, cus); }
+int win_interp_groups(int w, int cw, int64_t num_points, int cus) {
+  if (cw > 17 - 2 * w) return interp_groups_per_cu(win_cells(w), 2);  // few points
+  return win_groups(1, w, num_points, cus);
+}
 int win_grad_groups(int w, int64_t num_points, int cus) { return win_groups(2, w, num_points, cus); }
 
 hipError_t launch_win_interp(int w, const PointArgs &pa, ZRec zr, const float2 *grid,
