@@ -189,12 +189,13 @@ struct StageTimer {
 // workspace, and pinned staging.  Allocating and freeing them took 70 of a
 // call's 405 us (32^3 modes, 100,000 points), copying from pageable memory
 // waits for each copy.  At most kArenaDev and kArenaPin bytes are kept, until
-// the plan is destroyed; a larger call frees its memory when it ends.
+// the plan is destroyed; a larger call allocates and frees its own, or stages
+// in pageable memory.
 struct HostArena {
   char *dev = nullptr, *pin = nullptr;
   size_t dev_bytes = 0, pin_bytes = 0;
 };
-constexpr size_t kArenaDev = (size_t)64 << 20, kArenaPin = (size_t)16 << 20;
+constexpr size_t kArenaDev = (size_t)256 << 20, kArenaPin = (size_t)32 << 20;
 
 struct Layout {
   size_t keys0 = 0, keys1 = 0, idx0 = 0, idx1 = 0, cnt = 0, scan = 0, bin_start = 0,
@@ -1864,7 +1865,7 @@ void from_c64(int storage, const float2 *src, int64_t n, void *dst) {
 }
 
 // Device and pinned host memory of a host call, at least db and pb bytes;
-// without pinned memory (pin NULL) the call stages in pageable memory.
+// where memory cannot be pinned the call stages in pageable memory.
 hipError_t grow_arena(HostArena &a, size_t db, size_t pb) {
   hipError_t e = hipSuccess;
   if (a.dev_bytes < db) {
@@ -1922,23 +1923,26 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   HostArena own;
   std::unique_lock<std::mutex> lk(p->arena_mu, std::try_to_lock);
   HostArena &ar = lk.owns_lock() ? p->arena : own;
-  const bool keep = lk.owns_lock() && b_in + b_out + b_c + wsb <= kArenaDev && b_in + b_out + b_c <= kArenaPin;
-  hipError_t e = grow_arena(ar, b_in + b_out + b_c + wsb, b_in + b_out + b_c);
+  const size_t staged = b_in + b_out + b_c;
+  const bool keep = lk.owns_lock() && staged + wsb <= kArenaDev;
+  // (pinning memory takes longer than a copy from pageable memory: only what
+  // is kept is pinned)
+  hipError_t e = grow_arena(ar, staged + wsb, lk.owns_lock() && staged <= kArenaPin ? staged : 0);
   if (e != hipSuccess) {
     free_arena(ar);
     return hip_fail(e, "hipMalloc");
   }
   std::vector<char> pageable;
-  char *h = ar.pin;
+  char *h = ar.pin_bytes >= staged ? ar.pin : nullptr;
   if (!h) {
-    pageable.resize(b_in + b_out + b_c);
+    pageable.resize(staged);
     h = pageable.data();
   }
   float2 *h_in = (float2 *)h, *h_out = (float2 *)(h + b_in);
   float *h_c = (float *)(h + b_in + b_out);
   float2 *d_in = (float2 *)ar.dev, *d_out = (float2 *)(ar.dev + b_in);
   float *d_c = (float *)(ar.dev + b_in + b_out);
-  void *d_ws = ar.dev + b_in + b_out + b_c;
+  void *d_ws = ar.dev + staged;
   // interleaved coordinates are converted and taken as they are
   const bool inter = p->dim == 3 && stride == 3 && M > 0 && coords[1] == coords[0] + 1 && coords[2] == coords[0] + 2;
   const float *dc[3] = {d_c, inter ? d_c + 1 : p->dim == 3 ? d_c + M : d_c,
@@ -1963,7 +1967,11 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   } while (0);
   if (st != ANUFFT_OK || e != hipSuccess) (void)hipStreamSynchronize(s);
   if (st == ANUFFT_OK && e == hipSuccess) from_c64(storage, h_out, nout, out);
-  if (!keep) free_arena(ar);
+  if (!keep) {
+    if (ar.dev) (void)hipFree(ar.dev);
+    ar.dev = nullptr;
+    ar.dev_bytes = 0;
+  }
   if (st != ANUFFT_OK) return st;
   if (e != hipSuccess) return hip_fail(e, "host execute");
   return ANUFFT_OK;
