@@ -130,6 +130,8 @@ struct SortBuffers {
   int max_sub;
   int sub_work;        // fixed cost of a subproblem in kWorkUnit units
   bool along_x;        // pencils of the list run along x (else y)
+  float2 *zero;        // a grid to zero beside the binning (zero_n values, 0: none)
+  int64_t zero_n;
   ClassBuffers cls;
 };
 
@@ -234,6 +236,8 @@ struct BinProblem {
   ClassBuffers cls;
   int chunk;                // tile binning: points of a chunk
   uint32_t chunk0, scan0, piece0;
+  float2 *zero;             // single tile binning: a grid zeroed beside the counting
+  int64_t zero_n;
   int fused;                // one pass: the scatter launch also writes the list
 };
 

@@ -813,6 +813,17 @@ struct Exec {
     hipError_t ej = hipStreamWaitEvent(s, p->ev_join, 0);
     return em != hipSuccess ? em : ej;
   }
+  // The FFT passes of a grid (aux) beside the binning of M points (main), or,
+  // where both are short, before it: a fork and join cost about 10 us of a
+  // call.  Type-2, forked and in turn (us): 24^3 cells, 2000 points 63 and 53;
+  // 48^3, 20,000 74 and 71; 80^3, 100,000 111 and 107, 400,000 126 and 129;
+  // 128^3, 100,000 163 and 164, 400,000 170 and 179.
+  template <typename A, typename B>
+  hipError_t fft_and_binning(int64_t M, A aux, B main) const {
+    if (p->cells() > (int64_t)1 << 19 || M > 200000) return fork_join(aux, main);
+    hipError_t e = aux(*this);
+    return e == hipSuccess ? main() : e;
+  }
   float2 *grid() const { return (float2 *)(ws + lay.grid); }
   float *rec() const { return (float *)(ws + lay.rec); }
   uint8_t *xo() const { return (uint8_t *)(ws + lay.xo); }
@@ -832,9 +843,13 @@ struct Exec {
   // Binning; with records (MFMA kernels) the sort passes also build the
   // compact per-point records in sorted order.
   hipError_t bin(const anufft_plan::Binning &b, const PointArgs &pa, const float2 *values,
-                 int fields) const {
+                 int fields, bool zero_grid = false) const {
     return timed(ANUFFT_STAGE_BIN, [&] {
-      const SortBuffers sb = sort_buffers(b);
+      SortBuffers sb = sort_buffers(b);
+      if (zero_grid) {
+        sb.zero = grid();
+        sb.zero_n = p->cells();
+      }
       if (p->kernel_method != kSpreadMfma) return sort_points(pa, b.g, p->dim, sb, s);
       const RecordOut ro = record_out(pa.num_points, values, fields);
       return sort_points(pa, b.g, p->dim, sb, s, &ro);
@@ -1259,20 +1274,17 @@ static anufft_status run_type1(const anufft_plan *p, int64_t M, const float *con
     if (e != hipSuccess) return hip_fail(e, "spread");
   } else if (M > 0) {
     PointArgs pa = ex.point_args(bs, M, coords, stride);
-    auto fill = [&](const Exec &ea) {
-      return ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
-    };
-    auto bin = [&] { return ex.bin(bs, pa, (const float2 *)values, Exec::kValues); };
-    // The grid is zeroed before the binning: beside it, on the second stream,
-    // the 2 us (64^3 cells) to 19 us (254^3) cost more in the fork and join,
-    // about 25 us.  Not so right after the copies of a host call, where the
-    // fork costs nothing (the call: 246 us with it, 254 without).
-    if (blocks) {
-      e = ex.fork_join(fill, bin);
-    } else {
-      e = fill(ex);
-      if (e == hipSuccess) e = bin();
-    }
+    // The binning's first launch zeroes the grid as well.  The host calls'
+    // zeroes it on the second stream, where the fork right after their copies
+    // costs nothing (the call: 246 us with it, 254 with a launch before).
+    if (blocks)
+      e = ex.fork_join(
+          [&](const Exec &ea) {
+            return ea.timed(ANUFFT_STAGE_FILL, [&] { return launch_fill(ea.grid(), p->cells(), ea.s); });
+          },
+          [&] { return ex.bin(bs, pa, (const float2 *)values, Exec::kValues); });
+    else
+      e = ex.bin(bs, pa, (const float2 *)values, Exec::kValues, true);
     if (e != hipSuccess) return hip_fail(e, "fill / binning");
     e = blocks ? ex.spread_blocks(pa, ex.grid()) : ex.spread3(bs, pa, (const float2 *)values, ex.grid());
     if (e != hipSuccess) return hip_fail(e, "spread");
@@ -1337,8 +1349,7 @@ anufft_status anufft_execute_type2(const anufft_plan *p, int64_t M, const float 
     PointArgs pa = ex.point_args(b, M, coords, stride);
     // the FFT passes (modes -> grid) and the binning (points) are independent:
     // the FFT goes to the plan's second stream, joined before interpolation
-    e = ex.fork_join(
-        [&](const Exec &ea) {
+    e = ex.fft_and_binning(M, [&](const Exec &ea) {
           return ea.fine_grid((const float2 *)modes, p->opts.compat_reference_type2_3d_scaling != 0);
         },
         [&] { return ex.bin(b, pa, nullptr, Exec::kIndices); });
@@ -1375,7 +1386,7 @@ anufft_status anufft_execute_grad_points(const anufft_plan *p, int64_t M,
     const anufft_plan::Binning &b = gm ? p->bi : p->bg;
     PointArgs pa = ex.point_args(b, M, coords, stride);
     // FFT passes (second stream) concurrent with the binning
-    e = ex.fork_join([&](const Exec &ea) { return ea.fine_grid((const float2 *)modes_h, false); },
+    e = ex.fft_and_binning(M, [&](const Exec &ea) { return ea.fine_grid((const float2 *)modes_h, false); },
                      [&] { return ex.bin(b, pa, (const float2 *)u, Exec::kValues | Exec::kIndices); });
     if (e != hipSuccess) return hip_fail(e, "fft / binning");
     e = ex.grad3(pa, ex, (const float2 *)u, grad);
@@ -1454,8 +1465,7 @@ anufft_status anufft_execute_type1_backward(const anufft_plan *p, int64_t M,
   // with the same tiles: one FFT (second stream) and one binning carrying
   // the values c (ignored by the interpolation, u of the gradient)
   PointArgs pa = ex.point_args(p->bi, M, coords, stride);
-  hipError_t e = ex.fork_join(
-      [&](const Exec &ea) { return ea.fine_grid((const float2 *)G, false); },
+  hipError_t e = ex.fft_and_binning(M, [&](const Exec &ea) { return ea.fine_grid((const float2 *)G, false); },
       [&] { return ex.bin(p->bi, pa, (const float2 *)values, Exec::kValues | Exec::kIndices); });
   if (e != hipSuccess) return hip_fail(e, "fft / binning");
   e = ex.interp3(p->bi, pa, ex, (float2 *)grad_values);

@@ -751,6 +751,16 @@ __global__ __launch_bounds__(kTileThreads) void tile_count_kernel(BinProblem one
   extern __shared__ uint32_t hist[];  // nbins
   uint32_t chunk;
   const BinProblem &pr = tile_problem<BATCH, kTileCount>(one, table, nprob, chunk);
+  if (!BATCH && chunk >= (uint32_t)pr.nchunks) {  // blocks past the chunks zero pr.zero
+    const int64_t st = (int64_t)(gridDim.x - pr.nchunks) * kTileThreads;
+    float4 *q = (float4 *)pr.zero;
+    const int64_t n4 = pr.zero_n / 2;
+    for (int64_t i = (int64_t)(chunk - pr.nchunks) * kTileThreads + threadIdx.x; i < n4; i += st)
+      q[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (chunk == (uint32_t)pr.nchunks && threadIdx.x == 0 && (pr.zero_n & 1))
+      pr.zero[pr.zero_n - 1] = make_float2(0.f, 0.f);
+    return;
+  }
   const int nbins = pr.nbins;
   const PointArgs &pa = pr.pa;
   if (chunk == 0 && threadIdx.x < kMaxSlots) pr.cls.vmax[threadIdx.x * kMaxStride] = 0u;
@@ -946,6 +956,116 @@ __global__ __launch_bounds__(kClsThreads) void class_sort_kernel(BinProblem one,
 int class_pieces(int64_t n, int nbins, int max_sub) {
   return (int)(std::min<int64_t>(nbins, n) + (n + max_sub - 1) / max_sub);
 }
+// The whole binning of at most kSmallPoints points by one workgroup: counts of
+// (tile, class, x offset) keys in LDS, their scan, the subproblem list, the
+// class starts, and the records at once in their final order (the class list
+// is the identity).  The launch's other workgroups zero pr.zero.  In place of
+// four launches that each wait for the one before (2000 points on 32^3 cells:
+// fill, count, scatter and class list 19 us, this kernel 11; a Type-1 call 51
+// and 46).
+constexpr int kSmallPer = 4;
+constexpr int kSmallPoints = kSmallPer * kTileThreads;
+constexpr size_t kSmallLds = 148 * 1024;
+static int small_keys(const Geom &g, int nbins, int ncls) { return nbins * ncls * g.bin[0]; }
+// LDS: key counts (then places), tile starts, the list's.
+static size_t small_lds(int nkeys, int nbins) {
+  return sizeof(uint32_t) * (((size_t)nkeys + 4) & ~(size_t)3) +
+         sizeof(uint32_t) * (((size_t)nbins + 4) & ~(size_t)3) + sizeof(TileSubLds);
+}
+
+__global__ __launch_bounds__(kTileThreads) void small_binning_kernel(BinProblem pr) {
+  extern __shared__ uint4 tile_lds[];
+  __shared__ uint32_t sh[kTileThreads / 64];
+  __shared__ float wmax[kTileThreads / 64];
+  if (blockIdx.x > 0) {
+    const int64_t st = (int64_t)(gridDim.x - 1) * kTileThreads;
+    for (int64_t i = (int64_t)(blockIdx.x - 1) * kTileThreads + threadIdx.x; i < pr.zero_n; i += st)
+      pr.zero[i] = make_float2(0.f, 0.f);
+    return;
+  }
+  const PointArgs &pa = pr.pa;
+  const ClassBuffers &cb = pr.cls;
+  const int nbins = pr.nbins, ncls = cb.ncls, binx = pr.g.bin[0], tk = ncls * binx, nkeys = nbins * tk;
+  const int n = (int)pa.num_points;
+  uint32_t *cnt = (uint32_t *)tile_lds, *starts = cnt + ((nkeys + 4) & ~3);
+  const bool vals = pr.out.v != nullptr;
+  float c[kSmallPer][3];
+  float2 v[kSmallPer];
+#pragma unroll
+  for (int s = 0; s < kSmallPer; ++s) {
+    const int j = (int)threadIdx.x + s * kTileThreads;
+    load_point(pa, 3, j, j < n, c[s]);
+    v[s] = vals ? pr.values[j < n ? j : 0] : make_float2(0.f, 0.f);
+  }
+  for (int d = threadIdx.x; d < nkeys; d += kTileThreads) cnt[d] = 0u;
+  __syncthreads();
+  const float inv_cw = 1.0f / (float)cb.cw;
+  float z[kSmallPer][3], mx = 0.f;
+  int off[kSmallPer];
+  uint32_t key[kSmallPer], rk[kSmallPer];
+#pragma unroll
+  for (int s = 0; s < kSmallPer; ++s) {
+    const uint32_t tile = fold_point<true>(c[s], pr.g, 3, z[s], off[s]);
+    const int cls = (int)(((float)((off[s] >> 8) & 255) - 0.5f) * inv_cw);  // as class_sort_kernel
+    key[s] = tile * (uint32_t)tk + (uint32_t)(cls * binx + (off[s] & 255));
+    rk[s] = 0u;
+    if ((int)threadIdx.x + s * kTileThreads < n) {
+      rk[s] = atomicAdd(&cnt[key[s]], 1u);
+      mx = fmaxf(mx, fmaxf(fabsf(v[s].x), fabsf(v[s].y)));
+    }
+  }
+  __syncthreads();
+  {
+    // first place of each key: exclusive scan, a run of keys per thread
+    const int per = (nkeys + kTileThreads - 1) / kTileThreads;
+    const int d0 = min(nkeys, (int)threadIdx.x * per), d1 = min(nkeys, d0 + per);
+    uint32_t sum = 0, total;
+    for (int d = d0; d < d1; ++d) sum += cnt[d];
+    uint32_t at = block_scan_waves<kTileThreads>(sum, sh, total);
+    for (int d = d0; d < d1; ++d) {
+      const uint32_t k = cnt[d];
+      cnt[d] = at;
+      at += k;
+    }
+  }
+  __syncthreads();
+  // the records, in their final order
+#pragma unroll
+  for (int s = 0; s < kSmallPer; ++s) {
+    const int j = (int)threadIdx.x + s * kTileThreads;
+    if (j >= n) continue;
+    const uint32_t p = cnt[key[s]] + rk[s];
+    pr.out.r[p] = make_float4(z[s][0], z[s][1], z[s][2], __int_as_float(off[s]));
+    if (vals) pr.out.v[p] = v[s];
+    if (pr.out.i) pr.out.i[p] = (uint32_t)j;
+    cb.perm[j] = (uint32_t)j;
+  }
+  for (int d = threadIdx.x; d <= nbins; d += kTileThreads) starts[d] = d < nbins ? cnt[d * tk] : (uint32_t)n;
+  if (vals) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  if (vals && threadIdx.x < kMaxSlots) {  // (one block: one slot, the others zero)
+    float m = 0.f;
+    for (int w = 0; w < kTileThreads / 64; ++w) m = fmaxf(m, wmax[w]);
+    cb.vmax[threadIdx.x * kMaxStride] = threadIdx.x == 0 ? __float_as_uint(m) : 0u;
+  }
+  subproblems_body<kTileThreads, 1>(*(TileSubLds *)(starts + ((nbins + 4) & ~3)), starts, nullptr, 0, nbins,
+                                    make_int3(pr.g.nbin[0], pr.g.nbin[1], pr.g.nbin[2]), pr.along_x,
+                                    pr.max_sub, pr.sub_work, pr.nsub, pr.subs);
+  __syncthreads();
+  // classes of the subproblems: a tile's class starts, cut to the subproblem
+  const int nsub = (int)pr.nsub[0];
+  for (int i = threadIdx.x; i < nsub * ncls; i += kTileThreads) {
+    const int piece = i / ncls, k = i - piece * ncls;
+    const int4 sub = pr.subs[piece];
+    const int first = (int)cnt[sub.x * tk + k * binx] - sub.y;
+    cb.start[i] = (uint16_t)max(0, min(sub.z, first));
+  }
+}
+
 // descriptors per table-fill launch (kernarg size)
 constexpr int kBinTableChunk = 8;
 struct BinTableChunk {
@@ -979,6 +1099,7 @@ int tile_chunk(int64_t n) {
 }
 int tile_chunks(int64_t n) { return (int)((n + tile_chunk(n) - 1) / tile_chunk(n)); }
 
+// (pr.zero: 16-byte aligned, as workspaces are laid out)
 // The tile binning's launches over `chunks` chunks, `scans` scan blocks and
 // `pieces` subproblems at most, of one problem or a table.
 hipError_t launch_tile_binning(const BinProblem &one, const BinProblem *table, int nprob,
@@ -994,7 +1115,8 @@ hipError_t launch_tile_binning(const BinProblem &one, const BinProblem *table, i
     hipLaunchKernelGGL(tile_scan_kernel<true>, dim3(scans), ns, 0, s, one, table, nprob);
     hipLaunchKernelGGL(tile_scatter_kernel<true>, lists, nt, lds, s, one, table, nprob);
   } else {
-    hipLaunchKernelGGL(tile_count_kernel<false>, dim3(chunks), nt, hist, s, one, table, nprob);
+    const uint32_t fill = (uint32_t)std::min<int64_t>((one.zero_n + 8 * kTileThreads - 1) / (8 * kTileThreads), 2048);
+    hipLaunchKernelGGL(tile_count_kernel<false>, dim3(chunks + fill), nt, hist, s, one, table, nprob);
     if (scans > 0) hipLaunchKernelGGL(tile_scan_kernel<false>, dim3(scans), ns, 0, s, one, table, nprob);
     hipLaunchKernelGGL(tile_scatter_kernel<false>, lists, nt, lds, s, one, table, nprob);
   }
@@ -1045,6 +1167,8 @@ static BinProblem bin_problem(const PointArgs &pa, const Geom &g, int dim, const
   pr.max_sub = sb.max_sub;
   pr.sub_work = sb.sub_work;
   pr.along_x = sb.along_x;
+  pr.zero = sb.zero;
+  pr.zero_n = sb.zero_n;
   return pr;
 }
 
@@ -1122,6 +1246,15 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
   if (sb.cls.ncls * g.bin[0] > kClsKeys) return hipErrorInvalidValue;
   if (rec && sb.cls.ncls > 0 && n > 0 && tile_binning(sb.nbins)) {
     BinProblem pr = bin_problem(pa, g, dim, sb, rec);
+    const int nkeys = small_keys(g, sb.nbins, sb.cls.ncls);
+    const size_t lds = small_lds(nkeys, sb.nbins);
+    if (n <= kSmallPoints && lds <= kSmallLds) {
+      hipError_t e = set_lds((const void *)small_binning_kernel, lds);
+      if (e != hipSuccess) return e;
+      const int fill = (int)std::min<int64_t>((pr.zero_n + 4 * kTileThreads - 1) / (4 * kTileThreads), 1024);
+      hipLaunchKernelGGL(small_binning_kernel, dim3(1 + fill), dim3(kTileThreads), lds, s, pr);
+      return hipGetLastError();
+    }
     pr.chunk = tile_chunk(n);
     pr.nchunks = tile_chunks(n);
     // the totals of a single chunk are its counts
@@ -1129,6 +1262,10 @@ hipError_t sort_points(const PointArgs &pa, const Geom &g, int dim, const SortBu
     if (pr.nchunks == 1) pr.tot = pr.cnt, scans = 0;
     return launch_tile_binning(pr, nullptr, 1, sb.nbins, (uint32_t)pr.nchunks, scans,
                                (uint32_t)class_pieces(n, sb.nbins, sb.max_sub), s);
+  }
+  if (sb.zero_n > 0) {
+    const hipError_t e = launch_fill(sb.zero, sb.zero_n, s);
+    if (e != hipSuccess) return e;
   }
   if (sort_one_pass(sb.nbins)) return sort_points_one_pass(pa, g, dim, sb, s, rec);
   // with records, the last pass writes rec->out; earlier ones alternate with tmp

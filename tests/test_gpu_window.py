@@ -42,8 +42,9 @@ def _points(case, n, w, rng):
     return (t / np.array(m)).astype(np.float32)
 
 
-# (random 3000 and 60000: few and many points a cell, wide and narrow windows)
-CASES = [("random", 1), ("random", 65), ("random", 3000), ("random", 60000), ("one_cell", 31), ("one_cell", 64),
+# (random 3000 and 60000: few and many points a cell, wide and narrow windows;
+# up to 4096 points one workgroup bins them all)
+CASES = [("random", 1), ("random", 65), ("random", 3000), ("random", 4096), ("random", 60000), ("one_cell", 31), ("one_cell", 64),
          ("one_cell", 4097), ("columns", 0), ("corner", 129)]
 
 
