@@ -33,11 +33,11 @@
 // 32.  What bounds the kernels is the matrix work and the vector work beside
 // it, which overlap little on a SIMD, then the flush of spreading (17 G
 // 64-byte atomic requests a second) and the loading of interpolation's
-// windows (50 of 290 us).  Measured, blocks or the class lists that each
+// windows.  Measured, blocks or the class lists that each
 // interpolation workgroup built for itself, and now: spreading 2e6 points,
 // 64^3 modes, w = 7, 400 and 250 us; 16e6 points, 127^3 modes, w = 4, 2650
-// and 1250; interpolation 2e6, w = 7, 400 and 290; 16e6, 100^3, w = 8, 5310
-// and 2440; gradient 1e6, 64^3, w = 6, 447 and 284.
+// and 1250; interpolation 2e6, w = 7, 400 and 280; 16e6, 100^3, w = 8, 5310
+// and 2440; gradient 1e6, 64^3, w = 6, 447 and 258.
 //
 // Points are staged kWinPts at a time; each wave evaluates the taps of one
 // axis for them (a lane is a point), with the polynomial coefficients in
@@ -569,47 +569,93 @@ __device__ __forceinline__ int even_z0(int z0) { return z0 + (z0 & 1); }
 // H windows of 16 rows on top of each other: H = 2, tall windows, hold every
 // point of a tile (bin_y + 2 W <= 32 rows) for twice the products a point; row
 // y at y mod 16 H.
+constexpr int kWinBuf = 256;  // 16 rows of 16 pairs
 template <int W, int H>
 struct GridWin {
   static constexpr int XW = Win<W>::XW;
   half8 rh[H][XW], rl[H][XW], ih[H][XW], il[H][XW];
 
   // Load rows `first` .. 16 H - 1 of window t (scaled by s); the other rows
-  // keep their content.
+  // keep their content.  buf: kWinBuf float4 of LDS, the wave's own.
+  //
+  // A lane needs 64 bytes of its row (z cells 8 g4 .. 8 g4 + 7), but 64 lanes
+  // each reading 16 bytes 64 apart are 64 accesses of the first-level cache,
+  // one a clock: they bound calls of few points a window (1.3 M loads of 29
+  // accesses, 150k of 230k clocks, at 17,000 points on 128^3).  So 16 lanes
+  // load a row's 32 cells (4 rows a load, only rows that are new), and the
+  // wave turns them in LDS (XORed places: no bank conflicts).  Lanes as the
+  // products need them, and so: interpolation of 17,000 points 95 and 57 us,
+  // 1e6 on 128^3, w = 6, 155 and 129, 2e6, w = 7, 310 and 287; gradient 1e6
+  // 267 and 258.  AHEAD: the next cell's loads run during this one's turn,
+  // where registers are left for them (w = 5, 6 at 4 workgroups: 25 spilled).
+  template <bool AHEAD>
   __device__ __forceinline__ void load(const float2 *grid, const Geom &g, const WTile &t, int first,
-                                       float s, int wave, int i16, int g4) {
+                                       float s, int wave, int i16, int g4, float4 *buf) {
 #pragma unroll
-    for (int h = 0; h < H; ++h) load_half(h, grid, g, t, first, s, wave, i16, g4);
+    for (int h = 0; h < H; ++h) load_half<AHEAD>(h, grid, g, t, first, s, wave, i16, g4, buf);
   }
+  template <bool AHEAD>
   __device__ __forceinline__ void load_half(int h, const float2 *grid, const Geom &g, const WTile &t,
-                                            int first, float s, int wave, int i16, int g4) {
+                                            int first, float s, int wave, int i16, int g4,
+                                            float4 *buf) {
     int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
     int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
     asm volatile("" : "+v"(i16), "+v"(g4), "+s"(m0), "+s"(m1), "+s"(m2));
-    const int row = (16 * h + i16 - t.y0) & (16 * H - 1);
-    if (row < first) return;
-    const int z0 = even_z0(t.z0) + 8 * g4;
-    const uint32_t y = (uint32_t)wrap(t.y0 + row, m1) * (uint32_t)m2;
+    // as a loader: cells z, z + 1 of ring rows 16 h + 4 r + g4
+    const int z = wrap(even_z0(t.z0) + 2 * i16, m2);
+    const bool pairs = (m2 & 1) == 0;  // aligned, and none crosses the end
+    const int next = z + 1 < m2 ? 8 : 8 - 8 * m2;  // bytes from z to z + 1
+    int at[4];  // byte offset in a plane (below 2^27), -1: not loaded
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = (16 * h + 4 * r + g4 - t.y0) & (16 * H - 1);
+      at[r] = row < first ? -1 : 8 * (wrap(t.y0 + row, m1) * m2 + z);
+    }
+    const bool mine = ((16 * h + i16 - t.y0) & (16 * H - 1)) >= first;
+    auto fetch = [&](int q, float4 (&u)[4]) {
+      const char *plane = (const char *)(grid + (int64_t)wrap(t.xlo + 4 * q + wave, m0) * m1 * m2);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (at[r] < 0) continue;
+        if (pairs) {
+          u[r] = *(const float4 *)(plane + (uint32_t)at[r]);
+        } else {
+          const float2 a = *(const float2 *)(plane + (uint32_t)at[r]);
+          const float2 b = *(const float2 *)(plane + (uint32_t)(at[r] + next));
+          u[r] = make_float4(a.x, a.y, b.x, b.y);
+        }
+      }
+    };
+    float4 u[4], un[4];
+    if (AHEAD) fetch(0, un);
 #pragma unroll
     for (int q = 0; q < XW; ++q) {
-      const int64_t plane = (int64_t)wrap(t.xlo + 4 * q + wave, m0) * m1 * m2;
-      const float2 *rowp = grid + plane + y;
-      float2 v[8];
-      if (z0 >= 0 && z0 + 8 <= m2 && (((uint32_t)plane + y) & 1) == 0) {
-        const float4 *src = (const float4 *)(rowp + z0);
+      if (AHEAD) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4 u = src[j];
-          v[2 * j] = make_float2(u.x, u.y);
-          v[2 * j + 1] = make_float2(u.z, u.w);
-        }
+        for (int r = 0; r < 4; ++r) u[r] = un[r];
+        if (q + 1 < XW) fetch(q + 1, un);
       } else {
-        int z = wrap(z0, m2);
+        fetch(q, u);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      int i = i16, k = g4;
+      if (!AHEAD) asm volatile("" : "+v"(i), "+v"(k));  // places not kept: no registers left
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[j] = rowp[z];
-          z = z + 1 < m2 ? z + 1 : 0;
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * r + k;
+        if (at[r] >= 0) buf[16 * row + (i ^ row)] = u[r];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (!mine) continue;
+      float2 v[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 c = buf[16 * i + ((4 * k + j) ^ i)];
+        v[2 * j] = make_float2(c.x, c.y);
+        v[2 * j + 1] = make_float2(c.z, c.w);
       }
       float tr[8], ti[8];
 #pragma unroll
@@ -711,6 +757,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
   __shared__ __align__(16) _Float16 BH[kWinPts * kIRow], BL[kWinPts * kIRow];
   __shared__ __align__(16) float WY[kWinPts * ROWY], WX[kWinPts * L::ROWX];
   __shared__ float RED[4][2][kWinPts];  // per wave: re, im of each point
+  __shared__ float4 WB[4 * kWinBuf];    // window rows on their way to the lanes
   __shared__ __align__(16) int REACH[kWinPts / 16];   // x cells each group of 16 points reaches
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -742,7 +789,8 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
                           ? 16 * H - min(16 * H, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16 * H) win.load(grid, g, t, first, s_in, wave, i16, g4);
+    if (first < 16 * H) win.template load<interp_groups_per_cu(XW, H) < 4 || XW < 4>(grid, g, t, first, s_in, wave,
+                                                                   i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
     for (int c0 = 0; c0 < npt; c0 += kWinPts) {
@@ -850,6 +898,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
   __shared__ __align__(16) float WY[kWinPts * kIRowY], WX[kWinPts * L::ROWX];
   __shared__ __align__(16) float DY[kWinPts * kIRowY], DX[kWinPts * L::ROWX];
   __shared__ float RED[4][6][kWinPts];
+  __shared__ float4 WB[4 * kWinBuf];
   __shared__ __align__(16) int REACH[kWinPts / 16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -882,7 +931,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
     const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16) win.load(grid, g, t, first, s_in, wave, i16, g4);
+    if (first < 16) win.template load<true>(grid, g, t, first, s_in, wave, i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
     for (int c0 = 0; c0 < npt; c0 += kWinPts) {

@@ -89,3 +89,24 @@ def test_many_tiles(dev):
     for a, b in zip(out["mfma"], out["valu"]):
         a, b = a.to("cpu", torch.complex128), b.to("cpu", torch.complex128)
         assert float(torch.linalg.norm(a - b) / torch.linalg.norm(b)) <= TOL
+
+
+@pytest.mark.parametrize("w", [5, 7, 8])
+def test_odd_grid_lengths(dev, w):
+    """Grids of odd length along z (2 w + 1 cells): rows whose pairs of cells
+    are not aligned, and windows longer than the grid."""
+    import torch
+    import apollofft_amd as A
+    n = (9, 21, 5)
+    rng = np.random.default_rng(w)
+    x = torch.from_numpy(rng.uniform(0, 1, (500, 3)).astype(np.float32)).to(dev)
+    c = torch.from_numpy((rng.standard_normal((500, 2)) @ [1, 1j]).astype(np.complex64)).to(dev)
+    f = torch.from_numpy((rng.standard_normal(n + (2,)) @ [1, 1j]).astype(np.complex64)).to(dev)
+    out = {}
+    for method in ("mfma", "valu"):
+        p = A.NufftPlan3D(*n, *[1.0 / k for k in n], 2, w, kernel_method=method, grid_policy="exact")
+        assert p.meta["m"][2] == 2 * w + 1
+        out[method] = (p.type2(x, f), p.grad_points(x, c, f))
+    for a, b, tol in zip(out["mfma"], out["valu"], (TOL, TOL_GRAD)):
+        a, b = a.to("cpu", torch.complex128), b.to("cpu", torch.complex128)
+        assert float(torch.linalg.norm(a - b) / torch.linalg.norm(b)) <= tol
