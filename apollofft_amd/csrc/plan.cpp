@@ -270,11 +270,11 @@ struct anufft_plan {
   // kWinPts points nearly empty, and w = 7 and 8 have 5 and 16 classes a tile;
   // tall windows take a tile's points as one class, for twice the products a
   // point.  Interpolation from 128^3 cells, 16-row and tall windows (us): w = 8,
-  // 4 points a class 314 and 133, 23 353 and 211, 38 356 and 275; w = 7, 1.5 a
-  // class 112 and 94, 15 123 and 115 (clustered 124 and 126), 44 143 and 157.
-  // (w = 6: 2 a class 91 and 97, 20 104 and 119.)
+  // 4 points a class 270 and 69, 38 314 and 216, 75 403 and 374 (clustered 488
+  // and 429), 150 614 and 719; w = 7, 1.5 a class 68 and 44, 15 74 and 61, 30
+  // (64^3 cells) 39 and 30, 44 86 and 92, 88 120 and 141.
   const Binning &interp_bins(int64_t M) const {
-    const int per_class = w >= 8 ? 48 : w == 7 ? 8 : 0;
+    const int per_class = w >= 8 ? 88 : w == 7 ? 32 : 0;
     return bt.ncls > 0 && M < (int64_t)per_class * bi.nbins * bi.ncls ? bt : bi;
   }
   int lds_max = 163840; // gfx950 LDS per workgroup
