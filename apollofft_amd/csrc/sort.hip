@@ -1135,8 +1135,14 @@ size_t radix_count_entries(int64_t num_points) {
   const int64_t M = std::max<int64_t>(num_points, 1);
   return (size_t)(kRadix * ((M + kSortChunk - 1) / kSortChunk));
 }
+// The chunks at most of up to num_points points (tile_chunks falls where the
+// chunks grow by a step, from 512 at 524288 points to 257 at one more), so that
+// a workspace for many points serves fewer.
 size_t tile_count_entries(int64_t num_points, int nbins) {
-  return tile_binning(nbins) ? (size_t)nbins * tile_chunks(std::max<int64_t>(num_points, 1)) : 0;
+  if (!tile_binning(nbins)) return 0;
+  const int64_t chunks = num_points <= 4 * kTileThreads
+                             ? 1 : std::min<int64_t>((num_points + kTileThreads - 1) / kTileThreads, kTileChunks);
+  return (size_t)nbins * (size_t)chunks;
 }
 size_t one_pass_count_entries(int64_t num_points, int nbins) {
   const int64_t M = std::max<int64_t>(num_points, 1);

@@ -309,3 +309,26 @@ def test_launch_settings_and_autotune_argument_checks():
     bad = N.ptr_array([None] * 3)
     assert lib.anufft_autotune3d(*args, 1000, bad, 3, 3, None, ctypes.byref(out),
                                  ctypes.byref(ms)) == N.INVALID_ARG
+
+
+@pytest.mark.parametrize("n,w,policy", [((128, 128, 128), 6, "reference"), ((128, 128, 128), 8, "reference"),
+                                        ((120, 116, 120), 8, "exact"), ((64, 64, 64), 7, "reference"),
+                                        ((256, 256, 256), 8, "reference")])
+def test_workspace_for_many_points_serves_fewer(n, w, policy):
+    """A workspace sized for some number of points serves every smaller call,
+    also where the binning's chunks grow by a step (4096 points, then every
+    524288) and for more tiles than 8192, whose chunk counts outgrow 32 bytes
+    a point.  Single calls and batches."""
+    p = A.NufftPlan3D(*n, *(_d(k) for k in n), 2, w, grid_policy=policy, kernel_method="mfma")
+    counts = sorted({max(0, base + d) for base in (0, 1024, 4096, 8192, 524288, 600000, 734003, 1048576, 1572864)
+                     for d in (-1025, -1, 0, 1, 1025)})
+    sizes = [p.workspace_size(M) for M in counts]
+    assert sizes == sorted(sizes), [c for c, a, b in zip(counts, sizes[1:], sizes) if a < b]
+    b = ctypes.c_size_t()
+    batch = []
+    for M in counts:
+        plans = (ctypes.c_void_p * 2)(p.handle, p.handle)
+        Ms = (ctypes.c_int64 * 2)(M, M)
+        N.check(N.lib().anufft_batch_workspace_size(plans, 2, Ms, ctypes.byref(b)), "batch")
+        batch.append(b.value)
+    assert batch == sorted(batch)
