@@ -68,7 +68,7 @@ constexpr float kOpScale = 4096.0f;
 constexpr float kOpScaleD = 256.0f;
 constexpr float kFacScale = 64.0f;
 constexpr float kProdUnscale = 1.0f / (4096.0f * 4096.0f);
-constexpr float kProdUnscaleD = 1.0f / (4096.0f * 256.0f);
+constexpr int kOpBits = 12, kProdBits = 24, kProdBitsD = 20;  // exponents: an operand's, the products'
 
 // Geometry of the oversampled grid and the spreading tiles.
 struct Geom {

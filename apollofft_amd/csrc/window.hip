@@ -239,12 +239,12 @@ using SpreadAcc = f32x4[XC][4];  // [slot][block of 8 z cells]
 // whatever they hold (61 M floats: 222 us in aligned 64-byte requests, 370
 // misaligned, 442 in 32-byte ones).
 //
-// Add rows [0, nrow) of the window t to the grid (scaled by s_out) and zero
+// Add rows [0, nrow) of the window t to the grid (times 2^e_out) and zero
 // them.
 template <int W, int XC>
 __device__ __forceinline__ void win_flush(SpreadAcc<W, XC> &acc, float2 *grid, const Geom &g,
                                           const WTile &t, int wave, int i16, int g4, int nrow,
-                                          float s_out) {
+                                          int e_out) {
   using WN = Win<W, XC>;
   int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
   int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
@@ -266,7 +266,7 @@ __device__ __forceinline__ void win_flush(SpreadAcc<W, XC> &acc, float2 *grid, c
       for (int q = 0; q < WN::XW; ++q)
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          const float v = acc[q][b][r] * s_out;
+          const float v = ldexpf(acc[q][b][r], e_out);
           if (v != 0.f) unsafeAtomicAdd((float *)(plane[q] + (y + z[b])), v);
           acc[q][b][r] = 0.f;
         }
@@ -415,13 +415,15 @@ __device__ __forceinline__ void spread_products(SpreadAcc<W, XC> &acc, const cha
 }
 
 // Power-of-two exponent of a maximum kept in slots: e with max 2^-e in
-// [1/2, 1), clamped so that the scale and its inverse stay finite and normal.
+// [1/2, 1), 128 for an infinite one.  Operands are scaled by ldexpf(v, bits - e):
+// over the range of finite floats neither 2^(bits - e) nor its inverse need be
+// one (strengths of 1e-36).
 __device__ __forceinline__ int max_exp(const float *slots, int lane) {
   static_assert(kMaxSlots == 64, "a slot a lane");
   const float mx = wave_max(slots[lane * kMaxStride]);
   int e = 0;
   if (mx > 0.f) (void)frexpf(mx, &e);
-  return __builtin_amdgcn_readfirstlane(max(-120, min(120, e)));
+  return __builtin_amdgcn_readfirstlane(mx < INFINITY ? e : 128);
 }
 
 // Spread the share r of one problem's list.
@@ -440,7 +442,7 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
 #pragma unroll
     for (int b = 0; b < 4; ++b) acc[q][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int e = max_exp((const float *)pa.vmax, lane);
-  const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
+  const int e_in = kOpBits - e, e_out = e - kProdBits;
 
   const uint32_t *perm = pa.cperm;
   Rounds ahead(r, pa);
@@ -461,7 +463,7 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
     chain += n;
     for (int c0 = 0; c0 < n; c0 += kWinPts) {
       const int npts = min(kWinPts, n - c0);
-      spread_stage<W, XC>(sh, role, lane, npts, ra, make_float2(cv.x * s_in, cv.y * s_in), poly, t);
+      spread_stage<W, XC>(sh, role, lane, npts, ra, make_float2(ldexpf(cv.x, e_in), ldexpf(cv.y, e_in)), poly, t);
       __syncthreads();
       role = (role + 1) & 3;
       ra = zr.r[np];
@@ -478,11 +480,11 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
     asm volatile("" : "+v"(ra.x), "+v"(ra.w), "+v"(cv.x), "+v"(np));
     const bool slide = w.xlo == t.xlo && w.z0 == t.z0 && w.y0 >= t.y0 && chain + cw.hi - cw.lo <= kMaxChain;
     const int nrow = slide ? min(16, w.y0 - t.y0) : 16;
-    if (nrow > 0) win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, nrow, s_out);
+    if (nrow > 0) win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, nrow, e_out);
     if (nrow == 16) chain = 0;
     t = w;
   }
-  win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, 16, s_out);
+  win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, 16, e_out);
 }
 
 // Workgroups resident on a CU: as many as the registers hold without
@@ -575,7 +577,7 @@ struct GridWin {
   static constexpr int XW = Win<W>::XW;
   half8 rh[H][XW], rl[H][XW], ih[H][XW], il[H][XW];
 
-  // Load rows `first` .. 16 H - 1 of window t (scaled by s); the other rows
+  // Load rows `first` .. 16 H - 1 of window t (times 2^e); the other rows
   // keep their content.  buf: kWinBuf float4 of LDS, the wave's own.
   //
   // A lane needs 64 bytes of its row (z cells 8 g4 .. 8 g4 + 7), but 64 lanes
@@ -590,13 +592,13 @@ struct GridWin {
   // where registers are left for them (w = 5, 6 at 4 workgroups: 25 spilled).
   template <bool AHEAD>
   __device__ __forceinline__ void load(const float2 *grid, const Geom &g, const WTile &t, int first,
-                                       float s, int wave, int i16, int g4, float4 *buf) {
+                                       int e, int wave, int i16, int g4, float4 *buf) {
 #pragma unroll
-    for (int h = 0; h < H; ++h) load_half<AHEAD>(h, grid, g, t, first, s, wave, i16, g4, buf);
+    for (int h = 0; h < H; ++h) load_half<AHEAD>(h, grid, g, t, first, e, wave, i16, g4, buf);
   }
   template <bool AHEAD>
   __device__ __forceinline__ void load_half(int h, const float2 *grid, const Geom &g, const WTile &t,
-                                            int first, float s, int wave, int i16, int g4,
+                                            int first, int e, int wave, int i16, int g4,
                                             float4 *buf) {
     int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
     int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
@@ -660,8 +662,8 @@ struct GridWin {
       float tr[8], ti[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        tr[j] = v[j].x * s;
-        ti[j] = v[j].y * s;
+        tr[j] = ldexpf(v[j].x, e);
+        ti[j] = ldexpf(v[j].y, e);
       }
       split8(tr, rh[h][q], rl[h][q]);
       split8(ti, ih[h][q], il[h][q]);
@@ -778,7 +780,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
 
   GridWin<W, H> win;
   const int e = max_exp(gmax, lane);
-  const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(kProdUnscale, e);
+  const int e_in = kOpBits - e, e_out = e - kProdBits;
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
@@ -789,7 +791,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
                           ? 16 * H - min(16 * H, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16 * H) win.template load<interp_groups_per_cu(XW, H) < 4 || XW < 4>(grid, g, t, first, s_in, wave,
+    if (first < 16 * H) win.template load<interp_groups_per_cu(XW, H) < 4 || XW < 4>(grid, g, t, first, e_in, wave,
                                                                    i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
@@ -871,7 +873,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
       if (writer && ok) {
         const float re = (RED[0][0][lane] + RED[1][0][lane]) + (RED[2][0][lane] + RED[3][0][lane]);
         const float im = (RED[0][1][lane] + RED[1][1][lane]) + (RED[2][1][lane] + RED[3][1][lane]);
-        out[j] = make_float2(re * s_out, im * s_out);
+        out[j] = make_float2(ldexpf(re, e_out), ldexpf(im, e_out));
       }
     }
   } while (cw.next());
@@ -921,7 +923,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
 
   GridWin<W, 1> win;
   const int e = max_exp(gmax, lane);
-  const float s_in = ldexpf(kOpScale, -e), s_out = ldexpf(1.0f, e);
+  const int e_in = kOpBits - e, e_out = e - kProdBits, e_outd = e - kProdBitsD;
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
@@ -931,7 +933,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
     const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16) win.template load<true>(grid, g, t, first, s_in, wave, i16, g4, WB + wave * kWinBuf);
+    if (first < 16) win.template load<true>(grid, g, t, first, e_in, wave, i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
     for (int c0 = 0; c0 < npt; c0 += kWinPts) {
@@ -1033,8 +1035,8 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
         float sv[6];
 #pragma unroll
         for (int c = 0; c < 6; ++c)
-          sv[c] = ((RED[0][c][lane] + RED[1][c][lane]) + (RED[2][c][lane] + RED[3][c][lane])) * s_out *
-                  (c < 4 ? kProdUnscale : kProdUnscaleD);
+          sv[c] = ldexpf((RED[0][c][lane] + RED[1][c][lane]) + (RED[2][c][lane] + RED[3][c][lane]),
+                         c < 4 ? e_out : e_outd);
         // Re(conj(u) * (-s) * S) = -s (u.x S.x + u.y S.y)
         gx[j] = -(float)g.scale[0] * (u.x * sv[0] + u.y * sv[1]);
         if (gy) gy[j] = -(float)g.scale[1] * (u.x * sv[2] + u.y * sv[3]);
