@@ -54,21 +54,27 @@ struct KbPoly {
 // copies times the powers of two the operands enter the FP16 split with.
 struct WinPoly {
   KbPoly p;
-  float fac[kPolyCoefs][kMaxTaps];  // c * kFacScale
   float op[kPolyCoefs][kMaxTaps];   // c * kOpScale
   float dop[kPolyCoefs][kMaxTaps];  // dc * kOpScaleD
 };
-// Operands enter the FP16 split multiplied by 2^12 (exact), so that the low
-// halves of operands down to 2^-14 of the largest stay FP16-normal (11
-// significant bits): values in [0, 1] become [0, 4096] (FP16 max 65504).
-// Products carry 2^24, removed with the output scale.  Kernel derivatives
-// (|phi'| < 64 for w <= 8) use 2^8.  The x and y weights of spreading enter
-// their split multiplied by 2^6 each, so that their product carries 2^12.
+// Operands enter the FP16 split (hi = fp16(a), lo = fp16(a - hi), 22 bits)
+// multiplied by powers of two, which drop out of the scaled sums exactly.  An
+// operand of 2^-2 or more after scaling has a lo half whose rounding is below
+// 2^-22 of it; smaller ones meet the spacing 2^-24 of the FP16 subnormals.
+//   weights in [0, 1]          2^12: 22 bits from 2^-14 of the largest up
+//   their derivatives          2^8 (|phi'| < 64 for w <= 8)
+//   strengths times z weights  2^(15 - e), and grid cells, 2^e the first power
+//                              of two above the largest strength or cell of the
+//                              call: below 2^15 (FP16 max 65504), 22 bits from
+//                              2^-17 of the largest up, 2^-40 of it below
+// 2^-40 of the largest cell lies far under the rounding of the FFT that wrote
+// the grid, which is spread evenly over the cells (some 2^-24 of their root mean
+// square, and the largest of N modes' cells is at most sqrt(N) of that); and the
+// FFT after spreading mixes all cells.
 constexpr float kOpScale = 4096.0f;
 constexpr float kOpScaleD = 256.0f;
-constexpr float kFacScale = 64.0f;
-constexpr float kProdUnscale = 1.0f / (4096.0f * 4096.0f);
-constexpr int kOpBits = 12, kProdBits = 24, kProdBitsD = 20;  // exponents: an operand's, the products'
+constexpr float kProdUnscale = 1.0f / (4096.0f * 4096.0f);  // block_spread.hip
+constexpr int kValBits = 15, kProdBits = 12 + kValBits, kProdBitsD = 8 + kValBits;
 
 // Geometry of the oversampled grid and the spreading tiles.
 struct Geom {

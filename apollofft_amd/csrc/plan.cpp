@@ -474,7 +474,6 @@ anufft_status build_tables(anufft_plan *p) {
     wp.p = p->poly;
     for (int d = 0; d < kPolyCoefs; ++d)
       for (int i = 0; i < kMaxTaps; ++i) {
-        wp.fac[d][i] = p->poly.c[d][i] * kFacScale;
         wp.op[d][i] = p->poly.c[d][i] * kOpScale;
         wp.dop[d][i] = p->poly.dc[d][i] * kOpScaleD;
       }

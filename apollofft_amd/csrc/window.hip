@@ -216,12 +216,13 @@ __device__ __forceinline__ void reached_cells(int c0, int c1, F body) {
 }
 
 // ---- spreading ---------------------------------------------------------------
-constexpr int kSLd = kWinPts + 8;  // row stride (halves) of the operand tables
+constexpr int kSLd = kWinPts + 8;   // row stride (halves) of the B operand table
+constexpr int kSLdF = kWinPts + 4;  // row stride (floats) of the weight tables
 template <int PX>
 struct SLds {
-  static constexpr int X = 0;                             // half [hi, lo][PX][kSLd]: x weights
-  static constexpr int Y = X + 2 * PX * kSLd * 2;         // half [hi, lo][16][kSLd]: y weights
-  static constexpr int B = Y + 2 * 16 * kSLd * 2;         // half [hi, lo][32 z][re, im][kSLd]
+  static constexpr int X = 0;                             // float [PX][kSLdF]: x weights
+  static constexpr int Y = X + PX * kSLdF * 4;            // float [16][kSLdF]: y weights
+  static constexpr int B = Y + 16 * kSLdF * 4;            // half [hi, lo][32 z][re, im][kSLd]
   static constexpr int R = B + 2 * 64 * kSLd * 2;         // int [groups]: x cells reached
   static constexpr int SIZE = R + 16;
 };
@@ -278,19 +279,17 @@ __device__ __forceinline__ void win_flush(SpreadAcc<W, XC> &acc, float2 *grid, c
 // (bounds the FP32 rounding of a cell's sum).
 constexpr int kMaxChain = 8192;
 
-// Clear N rows (of kWinPts halves, `stride` apart) by one wave.
+// Clear N rows (N a multiple of 4) of the weight tables by one wave.
 template <int N>
-__device__ __forceinline__ void clear_rows(_Float16 *f, int stride, int lane) {
+__device__ __forceinline__ void clear_rows(float *f, int lane) {
+  static_assert(N % 4 == 0 && kWinPts == 64, "four rows a store of the wave");
 #pragma unroll
-  for (int i = 0; i < N / 8; ++i)
-    *(float4 *)(f + (8 * i + (lane >> 3)) * stride + (lane & 7) * 8) = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (N % 8 != 0 && lane < N % 8 * 8)
-    *(float4 *)(f + (N / 8 * 8 + (lane >> 3)) * stride + (lane & 7) * 8) = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i = 0; i < N / 4; ++i)
+    *(float4 *)(f + (4 * i + (lane >> 4)) * kSLdF + (lane & 15) * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// hi and lo of s v[i] to rows i, STEP rows of kSLd apart; the lo table
-// follows the hi table of R rows.
-template <int T, int R, int STEP>
+// hi and lo of s v[i] to z cell i of the B table (re or im rows).
+template <int T>
 __device__ __forceinline__ void store_split(_Float16 *f, const float (&v)[T], float s) {
 #pragma unroll
   for (int i = 0; i < T; i += 2) {
@@ -298,8 +297,8 @@ __device__ __forceinline__ void store_split(_Float16 *f, const float (&v)[T], fl
     split2(v[i] * s, v[i + 1] * s, h, l);
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
-      f[(i + d) * STEP * kSLd] = h[d];
-      f[(R + i + d) * STEP * kSLd] = l[d];
+      f[(i + d) * 2 * kSLd] = h[d];
+      f[(32 + i + d) * 2 * kSLd] = l[d];
     }
   }
 }
@@ -334,16 +333,15 @@ __device__ __forceinline__ void spread_stage(char *sh, int role, int lane, int n
   asm volatile("" : "+v"(lane));
   const bool ok = lane < npts;
   float v[T];
-  if (role == 0) {
-    _Float16 *F = (_Float16 *)(sh + L::X);
-    clear_rows<2 * PX>(F, kSLd, lane);
-    taps_scalar<W>((ConstFloatPtr)&poly->fac[0][0], ra.x, v);
-    if (ok) store_split<T, PX, 1>(F + (off & 255) * kSLd + lane, v, 1.0f);
-  } else if (role == 1) {
-    _Float16 *F = (_Float16 *)(sh + L::Y);
-    clear_rows<2 * 16>(F, kSLd, lane);
-    taps_scalar<W>((ConstFloatPtr)&poly->fac[0][0], ra.y, v);
-    if (ok) store_split<T, 16, 1>(F + (((off >> 8) & 255) - w.o1) * kSLd + lane, v, 1.0f);
+  if (role < 2) {  // (the x weights carry the product's scale)
+    float *F = (float *)(sh + (role == 0 ? L::X : L::Y));
+    if (role == 0) clear_rows<PX>(F, lane);
+    else clear_rows<16>(F, lane);
+    taps_scalar<W>((ConstFloatPtr)(role == 0 ? &poly->op[0][0] : &poly->p.c[0][0]), role == 0 ? ra.x : ra.y, v);
+    F += (role == 0 ? off & 255 : ((off >> 8) & 255) - w.o1) * kSLdF + lane;
+    if (ok)
+#pragma unroll
+      for (int i = 0; i < T; ++i) F[i * kSLdF] = v[i];
   } else if (32 * (role - 2) < npts) {
     _Float16 *B = (_Float16 *)(sh + L::B) + 32 * (role - 2);
 #pragma unroll
@@ -351,8 +349,8 @@ __device__ __forceinline__ void spread_stage(char *sh, int role, int lane, int n
       *(float4 *)(B + (16 * i + (lane >> 2)) * kSLd + (lane & 3) * 8) = make_float4(0.f, 0.f, 0.f, 0.f);
     taps_scalar<W>((ConstFloatPtr)&poly->p.c[0][0], ra.z, v);
     if (32 * (role - 2) + (lane & 31) < npts)
-      store_split<T, 32, 2>(B + (((off >> 16) & 255) * 2 + (lane >> 5)) * kSLd + (lane & 31), v,
-                            lane < 32 ? cv.x : cv.y);
+      store_split<T>(B + (((off >> 16) & 255) * 2 + (lane >> 5)) * kSLd + (lane & 31), v,
+                     lane < 32 ? cv.x : cv.y);
   }
 }
 
@@ -372,9 +370,9 @@ __device__ __forceinline__ void spread_products(SpreadAcc<W, XC> &acc, const cha
   using L = SLds<WN::PX>;
   constexpr int XW = WN::XW;
   asm volatile("" : "+v"(i16), "+v"(g4));
-  const _Float16 *X = (const _Float16 *)(sh + L::X) + wave * kSLd;
+  const float *X = (const float *)(sh + L::X) + wave * kSLdF;
   // ring row 4 (i16 % 4) + i16 / 4 and z cell 8 b + i16 / 2, window relative
-  const _Float16 *Y = (const _Float16 *)(sh + L::Y) + ((4 * (i16 & 3) + (i16 >> 2) - t.y0) & 15) * kSLd;
+  const float *Y = (const float *)(sh + L::Y) + ((4 * (i16 & 3) + (i16 >> 2) - t.y0) & 15) * kSLdF;
   const _Float16 *B[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b)
@@ -389,20 +387,24 @@ __device__ __forceinline__ void spread_products(SpreadAcc<W, XC> &acc, const cha
       bh[b] = *(const half8 *)(B[b] + kb);
       bl[b] = *(const half8 *)(B[b] + 64 * kSLd + kb);
     }
-    const half8 yh = *(const half8 *)(Y + kb);
-    const half8 yl = *(const half8 *)(Y + 16 * kSLd + kb);
+    float y[8];
+    *(float4 *)y = *(const float4 *)(Y + kb);
+    *(float4 *)(y + 4) = *(const float4 *)(Y + kb + 4);
 #pragma unroll
     for (int q = 0; q < XW; ++q) {
       if (4 * q < c0 || 4 * q >= c1) continue;
-      const half8 xh = *(const half8 *)(X + 4 * q * kSLd + kb);
-      const half8 xl = *(const half8 *)(X + (WN::PX + 4 * q) * kSLd + kb);
-      // A = wx wy from the split factors: hi = fp16(xh yh), lo = the exact
-      // rest of that product + xh yl + xl yh (packed FP16 FMAs; xl yl is
-      // below 2^-22 of the product)
-      const half8 ah = xh * yh;
-      half8 al = __builtin_elementwise_fma(xh, yh, -ah);
-      al = __builtin_elementwise_fma(xh, yl, al);
-      al = __builtin_elementwise_fma(xl, yh, al);
+      // A = wx wy, the FP32 product split once.  (Split factors multiplied
+      // with FP16 FMAs take 16 vector instructions a cell instead of 24, but
+      // lose bits: against 64 bits 2000 points on 32^3 cells 2.8e-7 and 2.6e-7;
+      // and their staging takes what the products save: a Type-1 call of 2e6
+      // points, w = 7, 353 us and 354, w = 4, 244 and 244.)
+      float a[8];
+      *(float4 *)a = *(const float4 *)(X + 4 * q * kSLdF + kb);
+      *(float4 *)(a + 4) = *(const float4 *)(X + 4 * q * kSLdF + kb + 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] *= y[j];
+      half8 ah, al;
+      split8(a, ah, al);
       // four independent chains of three products
 #pragma unroll
       for (int b = 0; b < 4; ++b) acc[q][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[b], acc[q][b], 0, 0, 0);
@@ -442,7 +444,7 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
 #pragma unroll
     for (int b = 0; b < 4; ++b) acc[q][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int e = max_exp((const float *)pa.vmax, lane);
-  const int e_in = kOpBits - e, e_out = e - kProdBits;
+  const int e_in = kValBits - e, e_out = e - kProdBits;
 
   const uint32_t *perm = pa.cperm;
   Rounds ahead(r, pa);
@@ -780,7 +782,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
 
   GridWin<W, H> win;
   const int e = max_exp(gmax, lane);
-  const int e_in = kOpBits - e, e_out = e - kProdBits;
+  const int e_in = kValBits - e, e_out = e - kProdBits;
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
@@ -923,7 +925,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
 
   GridWin<W, 1> win;
   const int e = max_exp(gmax, lane);
-  const int e_in = kOpBits - e, e_out = e - kProdBits, e_outd = e - kProdBitsD;
+  const int e_in = kValBits - e, e_out = e - kProdBits, e_outd = e - kProdBitsD;
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
