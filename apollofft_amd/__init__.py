@@ -11,7 +11,7 @@ from ._native import (CapacityExceeded, DeviceUnavailable, HipError, InvalidArgu
                       U32Overflow, Unsupported)
 from .api import (DEFAULT_NUFFT_KERNEL_WIDTH, DEFAULT_NUFFT_OVERSAMPLING, nufft_type1_1d,
                   nufft_type1_1d_fast, nufft_type1_3d, nufft_type1_3d_fast, nufft_type2_1d,
-                  nufft_type2_1d_fast, nufft_type2_3d, nufft_type2_3d_fast)
+                  nufft_type2_1d_fast, nufft_type2_3d, nufft_type2_3d_fast, trim_host_memory)
 from .plan import NufftPlan1D, NufftPlan3D, autotune3d, execute_type1_batched
 
 __version__ = "0.1.0"
@@ -20,6 +20,7 @@ __all__ = [
     "NufftPlan1D", "NufftPlan3D", "autotune3d", "execute_type1_batched",
     "nufft_type1_1d", "nufft_type2_1d", "nufft_type1_3d", "nufft_type2_3d",
     "nufft_type1_1d_fast", "nufft_type2_1d_fast", "nufft_type1_3d_fast", "nufft_type2_3d_fast",
+    "trim_host_memory",
     "DEFAULT_NUFFT_KERNEL_WIDTH", "DEFAULT_NUFFT_OVERSAMPLING",
     "NufftError", "InvalidArgument", "ShapeMismatch", "ProfileMismatch", "CapacityExceeded",
     "U32Overflow", "DeviceUnavailable", "HipError", "Unsupported", "NativeLibraryMissing",

@@ -41,7 +41,7 @@ EXPORTS = [
     "anufft_execute_type1_backward",
     "anufft_batch_workspace_size",
     "anufft_execute_type1_batched", "anufft_execute_type1_host",
-    "anufft_execute_type2_host", "anufft_direct_type1", "anufft_direct_type2",
+    "anufft_execute_type2_host", "anufft_host_memory_trim", "anufft_direct_type1", "anufft_direct_type2",
     "anufft_direct_type1_host", "anufft_direct_type2_host", "anufft_direct_type1_select",
     "anufft_last_error", "anufft_version",
     "anufft_debug_num_bins", "anufft_debug_sort", "anufft_debug_spread",
@@ -183,6 +183,7 @@ def lib():
                                                vp, sz, vp]),
         "anufft_execute_type1_host": (i32, [vp, i32, i32, i64, P(vp), i64, vp, vp]),
         "anufft_execute_type2_host": (i32, [vp, i32, i32, i64, P(vp), i64, vp, vp]),
+        "anufft_host_memory_trim": (i32, []),
         "anufft_direct_type1": (i32, [vp, i64, P(vp), i64, vp, vp, vp]),
         "anufft_direct_type2": (i32, [vp, i64, P(vp), i64, vp, vp, vp]),
         "anufft_direct_type1_host": (i32, [vp, i64, P(vp), i64, vp, vp]),

@@ -151,8 +151,14 @@ def nufft_type2_3d_fast(positions, modes, dx, dy, dz, kernel_width=DEFAULT_NUFFT
                            modes.astype(np.complex128, copy=False))
 
 
+def trim_host_memory():
+    """Free the device and pinned memory the library keeps between the numpy
+    functions' calls (at most 256 MiB and 32 MiB per GPU)."""
+    N.check(N.lib().anufft_host_memory_trim(), "host_memory_trim")
+
+
 __all__ = [
-    "DEFAULT_NUFFT_KERNEL_WIDTH", "DEFAULT_NUFFT_OVERSAMPLING",
+    "DEFAULT_NUFFT_KERNEL_WIDTH", "DEFAULT_NUFFT_OVERSAMPLING", "trim_host_memory",
     "nufft_type1_1d", "nufft_type2_1d", "nufft_type1_3d", "nufft_type2_3d",
     "nufft_type1_1d_fast", "nufft_type2_1d_fast", "nufft_type1_3d_fast", "nufft_type2_3d_fast",
     "N",

@@ -17,6 +17,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -185,17 +187,129 @@ struct StageTimer {
   }
 };
 
-// Memory that a plan keeps between its host-pointer calls: device buffers and
-// workspace, and pinned staging.  Allocating and freeing them took 70 of a
-// call's 405 us (32^3 modes, 100,000 points), copying from pageable memory
-// waits for each copy.  At most kArenaDev and kArenaPin bytes are kept, until
-// the plan is destroyed; a larger call allocates and frees its own, or stages
-// in pageable memory.
-struct HostArena {
-  char *dev = nullptr, *pin = nullptr;
-  size_t dev_bytes = 0, pin_bytes = 0;
+// Memory kept between host-pointer calls, for all plans of a GPU: device memory
+// (buffers and workspace) and pinned staging.  Allocating and freeing them took
+// 70 of a call's 405 us (32^3 modes, 100,000 points), copying from pageable
+// memory waits for each copy.  The blocks lent out and idle together stay within
+// kKeptDev and kKeptPin bytes; a call they leave no room for allocates and frees
+// its own device memory and stages in pageable memory.  Idle blocks go back when
+// the GPU's last plan is destroyed, when an allocation of a host call fails, and
+// with anufft_host_memory_trim.
+constexpr size_t kKeptDev = (size_t)256 << 20, kKeptPin = (size_t)32 << 20;
+struct Block {
+  char *p = nullptr;
+  size_t bytes = 0;
+  bool kept = false;  // counted, and handed back to the pool
 };
-constexpr size_t kArenaDev = (size_t)256 << 20, kArenaPin = (size_t)32 << 20;
+class BlockPool {
+ public:
+  BlockPool(bool pinned, size_t cap) : pinned_(pinned), cap_(cap) {}
+  // A kept block of at least `bytes`, if there is one or there is room for it.
+  Block take(size_t bytes) {
+    Block out, drop[kIdle];
+    int ndrop = 0;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      int best = -1;
+      size_t lent = total_;
+      for (int i = 0; i < n_; ++i) {
+        lent -= idle_[i].bytes;
+        if (idle_[i].bytes >= bytes && (best < 0 || idle_[i].bytes < idle_[best].bytes)) best = i;
+      }
+      if (best >= 0) return remove(best);
+      if (bytes > cap_ || lent > cap_ - bytes) return out;
+      while (n_ > 0 && (total_ > cap_ - bytes || n_ == kIdle)) {  // the longest idle first
+        drop[ndrop] = remove(0);
+        total_ -= drop[ndrop++].bytes;
+      }
+      total_ += bytes;
+    }
+    for (int i = 0; i < ndrop; ++i) release(drop[i]);
+    out.p = allocate(bytes);
+    out.bytes = out.p ? bytes : 0;
+    out.kept = out.p != nullptr;
+    if (!out.p) {
+      std::lock_guard<std::mutex> lk(mu_);
+      total_ -= bytes;
+    }
+    return out;
+  }
+  // The work on the block is done (its stream has been waited for).
+  void give(const Block &b) {
+    Block drop = b;
+    if (b.kept) {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (n_ < kIdle) {
+        idle_[n_++] = b;
+        return;
+      }
+      drop = remove(0);
+      idle_[n_++] = b;
+      total_ -= drop.bytes;
+    }
+    release(drop);
+  }
+  // Free the idle blocks.
+  void trim() {
+    for (;;) {
+      Block b;
+      {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (n_ == 0) return;
+        b = remove(0);
+        total_ -= b.bytes;
+      }
+      release(b);
+    }
+  }
+  char *allocate(size_t bytes) const {
+    void *q = nullptr;
+    const hipError_t e = pinned_ ? hipHostMalloc(&q, bytes, hipHostMallocDefault) : hipMalloc(&q, bytes);
+    if (e == hipSuccess) return (char *)q;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+
+ private:
+  static constexpr int kIdle = 8;
+  Block remove(int i) {
+    const Block b = idle_[i];
+    for (--n_; i < n_; ++i) idle_[i] = idle_[i + 1];
+    return b;
+  }
+  void release(const Block &b) const {
+    if (b.p) (void)(pinned_ ? hipHostFree(b.p) : hipFree(b.p));
+  }
+  const bool pinned_;
+  const size_t cap_;
+  std::mutex mu_;
+  Block idle_[kIdle];  // the longest idle first
+  int n_ = 0;
+  size_t total_ = 0;   // bytes of the kept blocks, lent out and idle
+};
+struct HostMemory {
+  BlockPool dev{false, kKeptDev}, pin{true, kKeptPin};
+  int plans = 0;  // of this GPU
+  // Device memory for one call, kept or (not counted) its own.
+  Block device_block(size_t bytes) {
+    for (int attempt = 0; attempt < 2; ++attempt) {
+      Block b = dev.take(bytes);
+      if (!b.p) b.p = dev.allocate(bytes);
+      if (b.p) return b;
+      dev.trim();  // what is idle here may be what is missing
+    }
+    return Block{};
+  }
+};
+// (never destroyed: plans may outlive the library's static objects)
+std::mutex &host_memory_mutex() {
+  static std::mutex *mu = new std::mutex;
+  return *mu;
+}
+std::map<int, HostMemory> &host_memory() {
+  static std::map<int, HostMemory> *all = new std::map<int, HostMemory>;
+  return *all;
+}
 
 struct Layout {
   size_t keys0 = 0, keys1 = 0, idx0 = 0, idx1 = 0, cnt = 0, scan = 0, bin_start = 0,
@@ -280,8 +394,7 @@ struct anufft_plan {
   int lds_max = 163840; // gfx950 LDS per workgroup
   int kernel_method = kSpreadMfma;
   hipStream_t host_stream = nullptr;
-  mutable std::mutex arena_mu;  // held by the host call that uses the arena
-  mutable HostArena arena;
+  HostMemory *host_mem = nullptr;  // its GPU's (null: no GPU)
   // Second stream for the Type-2 FFT passes, which run concurrently with the
   // binning of the points (fork/join through the two events; the mutex keeps
   // concurrent callers from interleaving their record/wait pairs).
@@ -522,8 +635,13 @@ void destroy_plan(anufft_plan *p) {
       if (p->d_bhat[a]) (void)hipFree(p->d_bhat[a]);
     }
     if (p->d_poly) (void)hipFree(p->d_poly);
-    if (p->arena.dev) (void)hipFree(p->arena.dev);
-    if (p->arena.pin) (void)hipHostFree(p->arena.pin);
+    if (p->host_mem) {
+      std::lock_guard<std::mutex> lk(host_memory_mutex());
+      if (--p->host_mem->plans == 0) {
+        p->host_mem->dev.trim();
+        p->host_mem->pin.trim();
+      }
+    }
     if (p->host_stream) (void)hipStreamDestroy(p->host_stream);
     if (p->aux_stream) (void)hipStreamDestroy(p->aux_stream);
     if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
@@ -685,6 +803,11 @@ anufft_status finish_create(anufft_plan *p, anufft_plan **out) {
       return fail(ANUFFT_UNSUPPORTED, "oversampled length %lld exceeds the in-LDS FFT limit 4096",
                   (long long)p->m[a]);
     }
+  }
+  if (p->device >= 0) {
+    std::lock_guard<std::mutex> lk(host_memory_mutex());
+    p->host_mem = &host_memory()[p->device];
+    ++p->host_mem->plans;
   }
   anufft_status st = build_tables(p);
   if (st != ANUFFT_OK) {
@@ -1212,6 +1335,16 @@ anufft_status anufft_plan3d_create(int64_t nx, int64_t ny, int64_t nz, double dx
 
 anufft_status anufft_plan_destroy(anufft_plan *plan) {
   destroy_plan(plan);
+  return ANUFFT_OK;
+}
+
+anufft_status anufft_host_memory_trim(void) {
+  std::lock_guard<std::mutex> lk(host_memory_mutex());
+  for (auto &m : host_memory()) {
+    DeviceGuard guard(m.first);
+    m.second.dev.trim();
+    m.second.pin.trim();
+  }
   return ANUFFT_OK;
 }
 
@@ -1873,33 +2006,6 @@ void from_c64(int storage, const float2 *src, int64_t n, void *dst) {
   }
 }
 
-// Device and pinned host memory of a host call, at least db and pb bytes;
-// where memory cannot be pinned the call stages in pageable memory.
-hipError_t grow_arena(HostArena &a, size_t db, size_t pb) {
-  hipError_t e = hipSuccess;
-  if (a.dev_bytes < db) {
-    if (a.dev) (void)hipFree(a.dev);
-    a.dev = nullptr;
-    a.dev_bytes = 0;
-    if ((e = hipMalloc((void **)&a.dev, db)) != hipSuccess) return e;
-    a.dev_bytes = db;
-  }
-  if (a.pin_bytes < pb) {
-    if (a.pin) (void)hipHostFree(a.pin);
-    a.pin = nullptr;
-    a.pin_bytes = 0;
-    if (hipHostMalloc((void **)&a.pin, pb, hipHostMallocDefault) == hipSuccess) a.pin_bytes = pb;
-    else (void)hipGetLastError();
-  }
-  return e;
-}
-void free_arena(HostArena &a) {
-  if (a.dev) (void)hipFree(a.dev);
-  if (a.pin) (void)hipHostFree(a.pin);
-  a.dev = a.pin = nullptr;
-  a.dev_bytes = a.pin_bytes = 0;
-}
-
 anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t profile,
                         int64_t M, const double *const coords[3], int64_t stride,
                         const void *in, void *out) {
@@ -1928,35 +2034,29 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   const size_t b_in = align_up(8 * (size_t)std::max<int64_t>(nin, 1));
   const size_t b_out = align_up(8 * (size_t)std::max<int64_t>(nout, 1));
   const size_t b_c = align_up(4 * nc);
-  // The plan's memory, or (in use by another thread's call) this call's own.
-  HostArena own;
-  std::unique_lock<std::mutex> lk(p->arena_mu, std::try_to_lock);
-  HostArena &ar = lk.owns_lock() ? p->arena : own;
   const size_t staged = b_in + b_out + b_c;
-  const bool keep = lk.owns_lock() && staged + wsb <= kArenaDev;
+  const Block db = p->host_mem->device_block(staged + wsb);
+  if (!db.p) return hip_fail(hipErrorOutOfMemory, "hipMalloc");
   // (pinning memory takes longer than a copy from pageable memory: only what
   // is kept is pinned)
-  hipError_t e = grow_arena(ar, staged + wsb, lk.owns_lock() && staged <= kArenaPin ? staged : 0);
-  if (e != hipSuccess) {
-    free_arena(ar);
-    return hip_fail(e, "hipMalloc");
-  }
-  std::vector<char> pageable;
-  char *h = ar.pin_bytes >= staged ? ar.pin : nullptr;
+  const Block pb = p->host_mem->pin.take(staged);
+  std::unique_ptr<char[]> pageable(pb.p ? nullptr : new (std::nothrow) char[staged]);
+  char *const h = pb.p ? pb.p : pageable.get();
   if (!h) {
-    pageable.resize(staged);
-    h = pageable.data();
+    p->host_mem->dev.give(db);
+    return fail(ANUFFT_INVALID_ARG, "out of host memory");
   }
   float2 *h_in = (float2 *)h, *h_out = (float2 *)(h + b_in);
   float *h_c = (float *)(h + b_in + b_out);
-  float2 *d_in = (float2 *)ar.dev, *d_out = (float2 *)(ar.dev + b_in);
-  float *d_c = (float *)(ar.dev + b_in + b_out);
-  void *d_ws = ar.dev + staged;
+  float2 *d_in = (float2 *)db.p, *d_out = (float2 *)(db.p + b_in);
+  float *d_c = (float *)(db.p + b_in + b_out);
+  void *d_ws = db.p + staged;
   // interleaved coordinates are converted and taken as they are
   const bool inter = p->dim == 3 && stride == 3 && M > 0 && coords[1] == coords[0] + 1 && coords[2] == coords[0] + 2;
   const float *dc[3] = {d_c, inter ? d_c + 1 : p->dim == 3 ? d_c + M : d_c,
                         inter ? d_c + 2 : p->dim == 3 ? d_c + 2 * M : d_c};
   const int64_t st_c = inter ? 3 : 1;
+  hipError_t e = hipSuccess;
   anufft_status st = ANUFFT_OK;
   do {
     to_c64(storage, in, nin, h_in);
@@ -1976,11 +2076,8 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   } while (0);
   if (st != ANUFFT_OK || e != hipSuccess) (void)hipStreamSynchronize(s);
   if (st == ANUFFT_OK && e == hipSuccess) from_c64(storage, h_out, nout, out);
-  if (!keep) {
-    if (ar.dev) (void)hipFree(ar.dev);
-    ar.dev = nullptr;
-    ar.dev_bytes = 0;
-  }
+  p->host_mem->dev.give(db);
+  p->host_mem->pin.give(pb);
   if (st != ANUFFT_OK) return st;
   if (e != hipSuccess) return hip_fail(e, "host execute");
   return ANUFFT_OK;
@@ -2010,6 +2107,10 @@ anufft_status host_direct(const anufft_plan *p, int type, int64_t M, const doubl
   size_t b_c = align_up(8 * hc.size());
   char *buf = nullptr;
   hipError_t e = hipMalloc(&buf, b_in + b_out + b_c);
+  if (e != hipSuccess) {  // what is kept idle may be what is missing
+    p->host_mem->dev.trim();
+    e = hipMalloc(&buf, b_in + b_out + b_c);
+  }
   if (e != hipSuccess) return hip_fail(e, "hipMalloc");
   double2 *d_in = (double2 *)buf, *d_out = (double2 *)(buf + b_in);
   double *d_c = (double *)(buf + b_in + b_out);

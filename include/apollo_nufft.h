@@ -300,6 +300,12 @@ anufft_status anufft_execute_type2_host(const anufft_plan *plan, int32_t storage
                                         const double *const coords[3], int64_t coord_stride,
                                         const void *modes, void *out);
 
+/* Free the memory kept for the host-pointer calls above.  The library keeps,
+ * per GPU and for all plans together, up to 256 MiB of device memory and 32 MiB
+ * of pinned host memory between such calls, and frees it when the GPU's last
+ * plan is destroyed; this call frees what no running call is using at once. */
+anufft_status anufft_host_memory_trim(void);
+
 /* Exact direct sums on the device (replaces the WGPU direct kernels
  * nufft_type{1,2}_{1d,3d}, apollo-nufft-wgpu infrastructure/shaders/
  * nufft.wgsl:51-140, and their drivers NufftWgpuKernel::execute_type1_1d,
