@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/apollo_nufft.h"
+#include "internal.h"
 
 namespace anufft {
 anufft_status report_error(anufft_status st, const char *msg);
@@ -308,6 +309,8 @@ extern "C" anufft_status anufft_autotune3d(int64_t nx, int64_t ny, int64_t nz, d
     for (int i = 0; i < 5; ++i)
       for (int v : cand[i]) {
         if (v == knob(cur, i)) continue;
+        // (the matrix-core kernels' lists end there: the same plan again)
+        if (i == 1 && v > anufft::kClassSub && cur.kernel_method == anufft::kSpreadMfma) continue;
         Knobs k = cur;
         knob(k, i) = v;
         const double t = bench.time(k);

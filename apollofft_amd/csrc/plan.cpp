@@ -1365,8 +1365,8 @@ anufft_status anufft_plan_get_meta(const anufft_plan *p, anufft_meta *meta) {
   meta->i0_beta = p->i0b;
   meta->grid_policy = p->opts.grid_policy;
   meta->compat_reference_type2_3d_scaling = p->opts.compat_reference_type2_3d_scaling;
-  meta->max_subproblem = p->bs.max_sub;
-  meta->interp_max_subproblem = p->bi.max_sub;
+  meta->max_subproblem = p->bs.list_sub();  // in use, whatever was asked for
+  meta->interp_max_subproblem = p->bi.list_sub();
   meta->poly_degree = kPolyCoefs - 1;
   meta->poly_max_err = p->poly_err;
   meta->kernel_method = p->kernel_method;

@@ -67,7 +67,8 @@ typedef struct anufft_opts {
   int32_t compat_reference_type2_3d_scaling; /* 1: 3D T2 returns direct/(mx my mz) like the reference */
   int32_t device_id;                         /* -1: current device */
   int32_t bin_size[3];                       /* interpolation tile in cells; 0 = automatic */
-  int32_t max_subproblem;                    /* points per subproblem; 0 = automatic */
+  int32_t max_subproblem;                    /* points per subproblem; 0 = automatic (the MFMA
+                                                kernels take 32 at least, 4096 at most) */
   int32_t kernel_method;                     /* 3D spreading and interpolation kernels:
                                                 0 automatic, 1 vector ALU (register columns,
                                                 LDS tiles), 2 FP16-split MFMA blocks */
@@ -76,8 +77,8 @@ typedef struct anufft_opts {
   int32_t sub_work;      /* fixed cost of a subproblem, in units of 16 points, when the
                             subproblem list is split among workgroups (automatic: 48) */
   int32_t blocks_per_cu; /* workgroups per CU of the 3D point kernels (automatic: per kernel) */
-  int32_t fft_lines;     /* lines per workgroup of the FFT passes (automatic: 1024 / length,
-                            at least 2 workgroups per CU) */
+  int32_t fft_lines;     /* lines per workgroup of the FFT passes (automatic: 8 of up to 256
+                            points, 2048 points of longer ones, more of shorter) */
 } anufft_opts;
 
 typedef struct anufft_meta {
@@ -92,7 +93,7 @@ typedef struct anufft_meta {
   int32_t grid_policy;
   int32_t compat_reference_type2_3d_scaling;
   int32_t bin_size[3];        /* spreading tile (cells) */
-  int32_t max_subproblem;     /* points per spreading subproblem */
+  int32_t max_subproblem;     /* points per spreading subproblem, as in use */
   int32_t interp_bin_size[3]; /* interpolation / gradient tile (cells) */
   int32_t interp_max_subproblem;
   int32_t poly_degree;  /* degree of the per-tap kernel polynomials */

@@ -110,3 +110,13 @@ def test_forced_launch_settings_keep_results(dev, oracle_mod, settings):
     sel = rng.choice(int(np.prod(n)), size=256, replace=False).astype(np.int64)
     r1 = oracle_mod.direct_type1_3d(xyz.astype(np.float64), c.astype(np.complex128), n, d, sel)
     assert rel_l2(got[0].ravel()[sel], r1) < 1e-5
+
+
+def test_autotune_leaves_out_settings_that_change_nothing(dev):
+    """Above 4096 points a subproblem the matrix-core kernels' lists are the
+    same: such candidates would be picked by noise alone."""
+    import apollofft_amd as A
+    d = (TWO_PI / 32,) * 3
+    for M in (50_000, 400_000):
+        t = A.autotune3d(32, 32, 32, *d, 2, 6, num_points=M, kernel_method="mfma")
+        assert t["max_subproblem"] <= 4096

@@ -332,3 +332,13 @@ def test_workspace_for_many_points_serves_fewer(n, w, policy):
         N.check(N.lib().anufft_batch_workspace_size(plans, 2, Ms, ctypes.byref(b)), "batch")
         batch.append(b.value)
     assert batch == sorted(batch)
+
+
+@pytest.mark.parametrize("method,asked,used", [("mfma", 16384, 4096), ("mfma", 8, 32), ("mfma", 1000, 1000),
+                                               ("mfma", None, 4096), ("valu", 16384, 16384), ("valu", 8, 8)])
+def test_metadata_reports_the_points_per_subproblem_in_use(method, asked, used):
+    """The matrix-core kernels' lists hold 32 to 4096 points of a tile at once."""
+    p = A.NufftPlan3D(64, 64, 64, _d(64), _d(64), _d(64), 2, 6, kernel_method=method, max_subproblem=asked)
+    assert p.meta["max_subproblem"] == used
+    if method == "mfma":
+        assert p.meta["interp_max_subproblem"] == used
