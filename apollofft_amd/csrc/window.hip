@@ -184,13 +184,13 @@ struct ClassWalk {
 // are loaded while a round runs.
 struct Rounds {
   ClassWalk w;
-  int off;
-  __device__ __forceinline__ Rounds(const XcdChunk &r, const PointArgs &pa) : w(r, pa), off(w.lo) {}
+  uint32_t off;  // (lists end at 2^31 - 1 points, and the rounds go on past the share's end)
+  __device__ __forceinline__ Rounds(const XcdChunk &r, const PointArgs &pa) : w(r, pa), off((uint32_t)w.lo) {}
   // List position of point p of the round (a valid one past the end too).
-  __device__ __forceinline__ int pos(int p) const { return min(off + p, w.hi - 1); }
+  __device__ __forceinline__ int pos(int p) const { return (int)min(off + (uint32_t)p, (uint32_t)w.hi - 1u); }
   __device__ __forceinline__ void advance() {
     off += kWinPts;
-    if (off >= w.hi && w.next()) off = w.lo;
+    if (off >= (uint32_t)w.hi && w.next()) off = (uint32_t)w.lo;
   }
 };
 
