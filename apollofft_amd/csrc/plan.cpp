@@ -2074,7 +2074,10 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
     if ((e = hipMemcpyAsync(h_out, d_out, 8 * (size_t)nout, hipMemcpyDeviceToHost, s)) != hipSuccess) break;
     e = hipStreamSynchronize(s);
   } while (0);
-  if (st != ANUFFT_OK || e != hipSuccess) (void)hipStreamSynchronize(s);
+  if (st != ANUFFT_OK || e != hipSuccess) {  // nothing of the call runs on when its memory goes back
+    (void)hipStreamSynchronize(s);
+    (void)hipStreamSynchronize(p->aux_stream);
+  }
   if (st == ANUFFT_OK && e == hipSuccess) from_c64(storage, h_out, nout, out);
   p->host_mem->dev.give(db);
   p->host_mem->pin.give(pb);
