@@ -5,15 +5,18 @@
 // transform/dimension_3d.rs:290-327).
 //
 // A dense grid cell sums hundreds to thousands of FP32 terms, and the
-// rounding of such a sum (3e-7 of the result at 400 terms a cell, 1e-6 at
-// 6000) depends on the order of its terms.  Results that a caller keeps in
-// FP64 are compared far below that, so this kernel keeps one order: tiles of
-// PX x cells x 32 y x 32 z along x pencils, the points of a tile in input
-// order, 16 a step; runs differ only by the order of the atomic additions
-// (2e-7).  The windows of window.hip (spreading of the other entry points)
-// sum in another order: 4e-7 away, and for a host call, which is bound by
-// the conversion and the copies of its arrays, not faster: 403 us and 390 us
-// a call at 32^3 modes, w = 6, 100,000 points.
+// rounding of such a sum depends on the order of its terms: runs of this kernel
+// differ by 2e-7 (the order of the atomic additions), and the windows of
+// window.hip, the spreading of the other entry points, are 4e-7 from it.  It is
+// kept for one reason: callers who hold results in FP64 compare them more closely
+// than FP32 ones, and with it they stay as they have been to within what two runs
+// differ by.  Neither accuracy nor speed is the reason: against 64-bit sums
+// the windows are off by less (32^3 modes, w = 6, 100,000 points 3.48e-7 here and
+// 3.08e-7; 24^3, 400,000 clustered 2.65e-7 and 2.02e-7; 16^3, w = 7, 400,000
+// 1.13e-6 and 7.2e-7), and a call with them takes 220 us instead of 247.
+//
+// The order: tiles of PX x cells x 32 y x 32 z along x pencils, the points of a
+// tile in input order, 16 a step.
 //
 // For each x cell the (y, z) plane is one output block of
 // v_mfma_f32_32x32x16_f16: A[y][k] = wx_k wy_k(y) times B[k][z] = c_k wz_k(z).

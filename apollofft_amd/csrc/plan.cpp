@@ -341,8 +341,9 @@ struct anufft_plan {
   WinPoly *d_poly = nullptr;        // device polynomials of the matrix-core kernels
   KbPoly poly{};
   double poly_err = 0;
-  // Binning geometries: spreading (register columns) and interpolation /
-  // gradient (LDS tile).  Each execute sorts with the geometry it uses.
+  // Binning geometries: spreading, interpolation, and the vector-ALU gradient
+  // (LDS tile; matrix-core plans use bi).  Each execute sorts with the geometry
+  // it uses.
   struct Binning {
     Geom g{};
     int nbins = 0;
@@ -360,7 +361,7 @@ struct anufft_plan {
       return std::min<int64_t>(nbins, M) + (M + list_sub() - 1) / list_sub();
     }
   } bs, bi, bg;
-  Binning bf;  // blocks of the FP64 host Type-1 (3D, matrix cores)
+  Binning bf;  // blocks of the FP64 host Type-1 (3D, matrix cores; block_spread.hip)
   Binning bw;  // wide spreading windows (3D, matrix cores)
   Binning bt;  // tall interpolation windows: bi with one class a tile
   // Type-1 tiles of M points.  With few points to a cell spreading is bound by
@@ -373,7 +374,14 @@ struct anufft_plan {
   // w = 4, 0.05 76 and 61, 0.3 98 and 88, 0.5 103 and 111.  On small grids, or
   // with a few thousand points, too few wide windows are left to keep the
   // chip's workgroups busy (w = 6, 32^3 cells 22 and 29, 64^3 37 and 35; w = 8,
-  // 96^3, 4000 points 68 and 75, 60,000 115 and 101).
+  // 96^3, 4000 points 68 and 75, 60,000 115 and 101).  The density is the mean
+  // over the grid.  Whole calls, narrow and wide, at 0.95 of the limits on 200^3
+  // and 254^3 cells: uniform points w = 8 1803 and 1663, 3842 and 3609, w = 6 742
+  // and 698, 2085 and 1717, w = 4 411 and 360, 1376 and 1077; 70 % in eight
+  // clusters w = 8 1804 and 1789, 3992 and 3803, w = 6 744 and 684, 2253 and 1793;
+  // lines through one point, the densest, gain less and lose up to 5 %: w = 8
+  // 1517 and 1539, 3279 and 3305, w = 6 595 and 624, 1565 and 1518, w = 4 316 and
+  // 330, 1036 and 951 (at half the limits they gain: 1068 and 1002, 440 and 398).
   const Binning &spread_bins(int64_t M) const {
     const double cells = (double)m[0] * (double)m[1] * (double)m[2];
     const bool wide = (double)M < cells * (w >= 8 ? 1.0 : w >= 6 ? 0.5 : 0.25) && M >= 8192 &&
@@ -386,7 +394,12 @@ struct anufft_plan {
   // point.  Interpolation from 128^3 cells, 16-row and tall windows (us): w = 8,
   // 4 points a class 270 and 69, 38 314 and 216, 75 403 and 374 (clustered 488
   // and 429), 150 614 and 719; w = 7, 1.5 a class 68 and 44, 15 74 and 61, 30
-  // (64^3 cells) 39 and 30, 44 86 and 92, 88 120 and 141.
+  // (64^3 cells) 39 and 30, 44 86 and 92, 88 120 and 141.  The mean decides here
+  // too.  Whole calls on 96^3, 200^3 and 254^3 cells, w = 8, 60 a class: uniform
+  // points 253 and 188, 1681 and 1483, 3400 and 3188, clusters 269 and 190, 1741
+  // and 1455, 3570 and 3178, lines through one point 245 and 188, 1362 and 1361,
+  // 2810 and 2990; 84 a class: 260 and 232, 2019 and 1998, 4170 and 4340; 289 and
+  // 241, 2022 and 1961, 4212 and 4316; 273 and 230, 1673 and 1853, 3447 and 4057.
   const Binning &interp_bins(int64_t M) const {
     const int per_class = w >= 8 ? 88 : w == 7 ? 32 : 0;
     return bt.ncls > 0 && M < (int64_t)per_class * bi.nbins * bi.ncls ? bt : bi;
@@ -673,11 +686,13 @@ void init_device(anufft_plan *p) {
     p->lds_max = v;
 }
 
-// Binning geometries.  Spreading: tiles of kSpreadBinX x (32-2w) x (32-2w)
-// cells, so that the padded (y,z) extent matches the 32 x 32 lane columns of
-// the spreading workgroup.  Interpolation: the tile shape whose padded LDS
-// copy (and the gradient kernel's) fits one workgroup's LDS and maximises
-// interior / padded volume.
+// Binning geometries.  Vector-ALU spreading: tiles of kSpreadBinX x (32-2w) x
+// (32-2w) cells, so that the padded (y,z) extent matches the 32 x 32 lane
+// columns of the spreading workgroup.  Vector-ALU interpolation and gradient:
+// the tile shape whose padded LDS copy fits one workgroup's LDS and maximises
+// interior / padded volume.  Matrix cores, all three: the interior of a window
+// along x, and at most 32-2w cells along y and z (32 z cells a window; the y
+// rows are cut into classes).
 void set_geom(anufft_plan::Binning &b, const anufft_plan *p, const int bin[3]) {
   Geom &g = b.g;
   for (int a = 0; a < 3; ++a) {
@@ -2025,7 +2040,7 @@ anufft_status host_exec(const anufft_plan *p, int type, int32_t storage, int32_t
   hipStream_t s = p->host_stream;
   const int64_t N = p->modes();
   const int64_t nin = type == 1 ? M : N, nout = type == 1 ? N : M;
-  // FP64 results keep one summation order (block_spread.hip)
+  // FP64 storage: results that stay as they were (block_spread.hip)
   const bool blocks = type == 1 && storage == ANUFFT_STORAGE_C128 && p->dim == 3 &&
                       p->kernel_method == kSpreadMfma;
   const Layout lay = layout(p, M, blocks);

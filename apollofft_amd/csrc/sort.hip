@@ -1,20 +1,27 @@
-// sort.hip -- point binning by a stable LSD counting sort on integer tile keys.
+// sort.hip -- point binning by counting sorts on integer tile keys.
 //
 // Replaces the comparison sorts sort_points_{1d,3d} / sort_positions_{1d,3d}
 // of apollo-nufft (transform/dimension_1d.rs:54-99, dimension_3d.rs:74-161):
-// the reference orders points by bucket with float tie-breaks; here the key
-// is the spreading tile of the point and ties keep the input order, so the
-// permutation is a deterministic function of the coordinates that a CPU
-// replay reproduces bit for bit.
+// the reference orders points by bucket with float tie-breaks; here the key is
+// the spreading tile of the point, from an FP64 fold of its coordinates.  Each
+// binning ends in a list of subproblems of at most max_sub points of a tile,
+// tiles in pencil order (along y, or along x).  One stream, no host
+// synchronisation.
 //
-// Pipeline (one stream, no host synchronisation):
-//   keys   : key[j] = tile of point j, per-chunk histogram of digit 0
-//   per digit pass: per-digit scan of the chunk counts -> stable scatter
-//                   (histogram of the next digit)
-//   bounds : bin_start[b] = lower_bound(sorted keys, b)
-//   subproblems (one block): scan of per-tile subproblem counts, list
-//   subs   : subproblems of at most max_sub points per tile, tiles in pencil
-//            order (along y, or along x)
+// * Tile binning, with a class list (matrix-core kernels, up to kTileMaxBins
+//   tiles): places from LDS counters, ties in any order; up to kSmallPoints
+//   points in one workgroup.
+// * One-pass binning (up to kOneMaxBins tiles): stable, on the whole key.
+// * Digit passes (any tile count): a stable LSD counting sort,
+//     keys   : key[j] = tile of point j, per-chunk histogram of digit 0
+//     per digit: per-digit scan of the chunk counts -> stable scatter
+//              (histogram of the next digit)
+//     bounds : bin_start[b] = lower_bound(sorted keys, b)
+//     subproblems (one block): scan of per-tile subproblem counts, the list
+//   (with records for the matrix-core kernels, then their class list).
+// In the stable ones ties keep the input order, so the permutation is a
+// deterministic function of the coordinates that a CPU replay reproduces bit
+// for bit.
 #include <algorithm>
 
 #include "internal.h"

@@ -489,10 +489,13 @@ __device__ __forceinline__ void spread_run(const PointArgs &pa, const ZRec &zr, 
   win_flush<W, XC>(acc, grid, g, t, wave, i16, g4, 16, e_out);
 }
 
-// Workgroups resident on a CU: as many as the registers hold without
-// spilling.  Spreading's accumulators (16 XW registers a lane) allow 3, from
-// w = 4 down 4 (2e6 points on 64^3, w = 4: 166 to 158 us; w = 6 at 4: 226 to
-// 306, the spills queue behind the atomics).
+// Workgroups resident on a CU: as many as the registers (16 XW a lane for the
+// accumulators) hold, or all but: 3, with 3 x cells 4, at which 6 registers
+// spill (batched 17; w = 7 and 8 batched 6 at 3).  Type-1 calls, 4 against 3: 2e6
+// points on 128^3 cells w = 2 202 and 205 us, w = 3 229 and 234, w = 4 243 and
+// 252; 16 problems w = 4 1433 and 1482; 800,000 points, where the flush counts
+// for more, w = 4 171 and 169.  (w = 6 at 4: spreading 226 to 306 us, the spills
+// queue behind the atomics.)
 constexpr int spread_groups_per_cu(int cells) { return cells <= 3 ? 4 : cells <= 5 ? 3 : 2; }
 
 template <int W, int XC>
