@@ -417,9 +417,9 @@ __device__ __forceinline__ void spread_products(SpreadAcc<W, XC> &acc, const cha
 }
 
 // Power-of-two exponent of a maximum kept in slots: e with max 2^-e in
-// [1/2, 1), 128 for an infinite one.  Operands are scaled by ldexpf(v, bits - e):
-// over the range of finite floats neither 2^(bits - e) nor its inverse need be
-// one (strengths of 1e-36).
+// [1/2, 1), 128 for an infinite one.  Strengths and sums are scaled by ldexpf:
+// over the range of finite floats 2^(bits - e) and its inverse need not be
+// finite (strengths of 1e-36).
 __device__ __forceinline__ int max_exp(const float *slots, int lane) {
   static_assert(kMaxSlots == 64, "a slot a lane");
   const float mx = wave_max(slots[lane * kMaxStride]);
@@ -573,6 +573,14 @@ struct ILds {
 // (z offsets start at 1: no tap of the tile lies in a skipped first cell).
 __device__ __forceinline__ int even_z0(int z0) { return z0 + (z0 & 1); }
 
+// The exponent windows are scaled with, whose 2^(kValBits - e) is finite: the
+// loads multiply by it (ldexpf there took 1 % of a Type-2 call, 2e6 points on
+// 128^3 cells 334.6 and 338.1 us).  Grids below 2^-111 are scaled by 2^126 and
+// so split to 2^-150, finer than FP32 subnormals lie.
+__device__ __forceinline__ int grid_exp(const float *gmax, int lane) {
+  return max(max_exp(gmax, lane), kValBits - 126);
+}
+
 // H windows of 16 rows on top of each other: H = 2, tall windows, hold every
 // point of a tile (bin_y + 2 W <= 32 rows) for twice the products a point; row
 // y at y mod 16 H.
@@ -582,7 +590,7 @@ struct GridWin {
   static constexpr int XW = Win<W>::XW;
   half8 rh[H][XW], rl[H][XW], ih[H][XW], il[H][XW];
 
-  // Load rows `first` .. 16 H - 1 of window t (times 2^e); the other rows
+  // Load rows `first` .. 16 H - 1 of window t (scaled by s); the other rows
   // keep their content.  buf: kWinBuf float4 of LDS, the wave's own.
   //
   // A lane needs 64 bytes of its row (z cells 8 g4 .. 8 g4 + 7), but 64 lanes
@@ -597,13 +605,13 @@ struct GridWin {
   // where registers are left for them (w = 5, 6 at 4 workgroups: 25 spilled).
   template <bool AHEAD>
   __device__ __forceinline__ void load(const float2 *grid, const Geom &g, const WTile &t, int first,
-                                       int e, int wave, int i16, int g4, float4 *buf) {
+                                       float s, int wave, int i16, int g4, float4 *buf) {
 #pragma unroll
-    for (int h = 0; h < H; ++h) load_half<AHEAD>(h, grid, g, t, first, e, wave, i16, g4, buf);
+    for (int h = 0; h < H; ++h) load_half<AHEAD>(h, grid, g, t, first, s, wave, i16, g4, buf);
   }
   template <bool AHEAD>
   __device__ __forceinline__ void load_half(int h, const float2 *grid, const Geom &g, const WTile &t,
-                                            int first, int e, int wave, int i16, int g4,
+                                            int first, float s, int wave, int i16, int g4,
                                             float4 *buf) {
     int m0 = __builtin_amdgcn_readfirstlane(g.m[0]), m1 = __builtin_amdgcn_readfirstlane(g.m[1]);
     int m2 = __builtin_amdgcn_readfirstlane(g.m[2]);
@@ -667,8 +675,8 @@ struct GridWin {
       float tr[8], ti[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        tr[j] = ldexpf(v[j].x, e);
-        ti[j] = ldexpf(v[j].y, e);
+        tr[j] = v[j].x * s;
+        ti[j] = v[j].y * s;
       }
       split8(tr, rh[h][q], rl[h][q]);
       split8(ti, ih[h][q], il[h][q]);
@@ -784,8 +792,8 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
   np = perm[ahead.pos(lane)];
 
   GridWin<W, H> win;
-  const int e = max_exp(gmax, lane);
-  const int e_in = kValBits - e, e_out = e - kProdBits;
+  const int e = grid_exp(gmax, lane), e_out = e - kProdBits;
+  const float s_in = ldexpf(1.0f, kValBits - e);
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
@@ -796,7 +804,7 @@ __global__ __launch_bounds__(Win<W>::NT, interp_groups_per_cu(win_cells(W), H)) 
                           ? 16 * H - min(16 * H, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16 * H) win.template load<interp_groups_per_cu(XW, H) < 4 || XW < 4>(grid, g, t, first, e_in, wave,
+    if (first < 16 * H) win.template load<interp_groups_per_cu(XW, H) < 4 || XW < 4>(grid, g, t, first, s_in, wave,
                                                                    i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
@@ -927,8 +935,8 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
   np = perm[ahead.pos(lane)];
 
   GridWin<W, 1> win;
-  const int e = max_exp(gmax, lane);
-  const int e_in = kValBits - e, e_out = e - kProdBits, e_outd = e - kProdBitsD;
+  const int e = grid_exp(gmax, lane), e_out = e - kProdBits, e_outd = e - kProdBitsD;
+  const float s_in = ldexpf(1.0f, kValBits - e);
   ClassWalk cw(r, pa);
   WTile t{};
   bool open = false;
@@ -938,7 +946,7 @@ __global__ __launch_bounds__(Win<W>::NT, grad_groups_per_cu<W>()) void win_grad_
     const int first = open && n.xlo == t.xlo && n.z0 == t.z0 && n.y0 >= t.y0 ? 16 - min(16, n.y0 - t.y0) : 0;
     open = true;
     t = n;
-    if (first < 16) win.template load<true>(grid, g, t, first, e_in, wave, i16, g4, WB + wave * kWinBuf);
+    if (first < 16) win.template load<true>(grid, g, t, first, s_in, wave, i16, g4, WB + wave * kWinBuf);
     const int oz = t.z0 - even_z0(t.z0);
     const int npt = cw.hi - cw.lo;
     for (int c0 = 0; c0 < npt; c0 += kWinPts) {
